@@ -38,6 +38,25 @@ OPS3D_FDA_API int ops3d_nms3d(const float *boxes_sorted, const int64_t *order, i
                               void *workspace, size_t workspace_bytes, int64_t *keep, int32_t *num_keep,
                               void *stream);
 
+/*
+ * The same result from a list of the overlapping pairs instead of the n x n mask, for
+ * 0 < n <= 2^18 and iou_threshold >= 0 (EINVAL otherwise).
+ *   boxes:     fp32, unsorted; coordinate k of box i at boxes[i * box_stride + k * coord_stride];
+ *   scores:    fp32, score i at scores[i * score_stride]; ranked here (decreasing, NaN first, equal
+ *              scores in index order) when ops3d_nms3d_pairs_ranks(n); order must then be NULL;
+ *   order:     otherwise (scores not read) [n] int64, box indices by decreasing score;
+ *   keep, num_keep: as above, but *num_keep = -1 when the boxes overlap too much for the list
+ *              (more than about 64 pairs per box above the threshold) or depend on each other in
+ *              too long chains: keep is then not written and the caller runs ops3d_nms3d.
+ * The workspace (ops3d_nms3d_pairs_workspace_bytes) must be 32-byte aligned.
+ */
+OPS3D_FDA_API size_t ops3d_nms3d_pairs_workspace_bytes(int n);
+OPS3D_FDA_API int ops3d_nms3d_pairs_ranks(int n);
+OPS3D_FDA_API int ops3d_nms3d_pairs(const float *boxes, int64_t box_stride, int64_t coord_stride,
+                                    const float *scores, int64_t score_stride, const int64_t *order, int n,
+                                    float iou_threshold, void *workspace, size_t workspace_bytes, int64_t *keep,
+                                    int32_t *num_keep, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -48,6 +48,9 @@ EXPORTED_SYMBOLS = (
     "ops3d_dcnv4_backward",
     "ops3d_nms3d_workspace_bytes",
     "ops3d_nms3d",
+    "ops3d_nms3d_pairs_workspace_bytes",
+    "ops3d_nms3d_pairs_ranks",
+    "ops3d_nms3d_pairs",
     "ops3d_roi_align3d_forward",
     "ops3d_roi_align3d_backward_workspace_bytes",
     "ops3d_roi_align3d_backward",
@@ -97,6 +100,13 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.ops3d_nms3d_workspace_bytes.argtypes = [_i]
     lib.ops3d_nms3d.restype = _i
     lib.ops3d_nms3d.argtypes = [_vp, _vp, _i, ctypes.c_float, _vp, _sz, _vp, _vp, _vp]
+    _i64 = ctypes.c_int64
+    lib.ops3d_nms3d_pairs_workspace_bytes.restype = _sz
+    lib.ops3d_nms3d_pairs_workspace_bytes.argtypes = [_i]
+    lib.ops3d_nms3d_pairs_ranks.restype = _i
+    lib.ops3d_nms3d_pairs_ranks.argtypes = [_i]
+    lib.ops3d_nms3d_pairs.restype = _i
+    lib.ops3d_nms3d_pairs.argtypes = [_vp, _i64, _i64, _vp, _i64, _vp, _i, ctypes.c_float, _vp, _sz, _vp, _vp, _vp]
     lib.ops3d_roi_align3d_forward.restype = _i
     lib.ops3d_roi_align3d_forward.argtypes = [_vp] * 3 + [_i] * 10 + [ctypes.c_float, _i, _i, _vp]
     lib.ops3d_roi_align3d_backward_workspace_bytes.restype = _sz
@@ -394,17 +404,35 @@ class _NativeFDA:
             raise ValueError("dets must be [N, 6] (x1,y1,z1,x2,y2,z2)")
         if scores.dim() != 1 or scores.shape[0] != dets.shape[0] or scores.device != dets.device:
             raise ValueError("scores must be [N] on the boxes' device")
-        order = torch.sort(scores, stable=True, descending=True)[1]
+        n, dev, thr = dets.shape[0], dets.device, float(threshold)
+        keep = torch.empty(n, dtype=torch.long, device=dev)
+        num = torch.empty(1, dtype=torch.int32, device=dev)
+        order = None
+        wsb = self._lib.ops3d_nms3d_pairs_workspace_bytes(n) if thr >= 0.0 else 0
+        ranked = self._lib.ops3d_nms3d_pairs_ranks(n)
+        if wsb and (not ranked or scores.dtype in _DTYPE_CODE):
+            # from the list of overlapping pairs; -1 when they are too many or too long a chain
+            b, s = dets.to(torch.float32), scores.to(torch.float32) if ranked else None
+            if not ranked:
+                order = torch.sort(scores, stable=True, descending=True)[1]
+            ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+            with torch.cuda.device(dev):
+                rc = self._lib.ops3d_nms3d_pairs(
+                    b.data_ptr(), b.stride(0), b.stride(1), _ptr(s), s.stride(0) if ranked else 0, _ptr(order), n, thr,
+                    _ptr(ws), wsb, _ptr(keep), _ptr(num), torch.cuda.current_stream(dev).cuda_stream)
+            if rc != OPS3D_FDA_OK:
+                raise RuntimeError("nms_3d: kernel launch failed")
+            kept = int(num.item())
+            if kept >= 0:
+                return keep[:kept]
+        if order is None:
+            order = torch.sort(scores, stable=True, descending=True)[1]
         boxes = dets.index_select(0, order).to(torch.float32).contiguous()
-        n = boxes.shape[0]
         wsb = self._lib.ops3d_nms3d_workspace_bytes(n)
-        ws = torch.empty(wsb, dtype=torch.uint8, device=dets.device)
-        keep = torch.empty(n, dtype=torch.long, device=dets.device)
-        num = torch.empty(1, dtype=torch.int32, device=dets.device)
-        stream = torch.cuda.current_stream(dets.device).cuda_stream
-        with torch.cuda.device(dets.device):
-            rc = self._lib.ops3d_nms3d(_ptr(boxes), _ptr(order), n, float(threshold), _ptr(ws), wsb, _ptr(keep),
-                                       _ptr(num), stream)
+        ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+        with torch.cuda.device(dev):
+            rc = self._lib.ops3d_nms3d(_ptr(boxes), _ptr(order), n, thr, _ptr(ws), wsb, _ptr(keep), _ptr(num),
+                                       torch.cuda.current_stream(dev).cuda_stream)
         if rc == OPS3D_FDA_EINVAL:
             raise ValueError("nms_3d: too many boxes (at most 2^19)")
         if rc != OPS3D_FDA_OK:

@@ -258,15 +258,35 @@ at::Tensor nms_3d(const at::Tensor &dets, const at::Tensor &scores, double thres
   if (scores.dim() != 1 || scores.size(0) != dets.size(0) || scores.device() != dets.device())
     throw std::invalid_argument("scores must be [N] on the boxes' device");
   const DeviceGuard guard(dets.device());
-  const at::Tensor order = std::get<1>(scores.sort(/*stable=*/true, /*dim=*/0, /*descending=*/true));
-  const at::Tensor boxes = dets.index_select(0, order).to(at::kFloat).contiguous();
-  const int n = (int)boxes.size(0);
-  const size_t wsb = ops3d_nms3d_workspace_bytes(n);
-  at::Tensor ws = at::empty({(int64_t)wsb}, dets.options().dtype(at::kByte));
+  const int64_t n64 = dets.size(0);
+  if (n64 > INT32_MAX) throw std::invalid_argument("nms_3d: too many boxes (at most 2^19)");
+  const int n = (int)n64;
+  const float thr = (float)threshold;
   at::Tensor keep = at::empty({n}, dets.options().dtype(at::kLong));
   at::Tensor num = at::empty({1}, dets.options().dtype(at::kInt));
-  const int rc = ops3d_nms3d(boxes.data_ptr<float>(), order.data_ptr<int64_t>(), n, (float)threshold, ws.data_ptr(),
-                             wsb, keep.data_ptr<int64_t>(), num.data_ptr<int32_t>(), stream_of(dets));
+  at::Tensor order;
+  const size_t pairs = thr >= 0.f ? ops3d_nms3d_pairs_workspace_bytes(n) : 0;
+  const bool ranked = ops3d_nms3d_pairs_ranks(n) != 0;
+  const auto sk = scores.scalar_type();
+  if (pairs && (!ranked || sk == at::kFloat || sk == at::kHalf || sk == at::kBFloat16)) {
+    // from the list of overlapping pairs; -1 when they are too many or too long a chain
+    const at::Tensor b = dets.to(at::kFloat), s = ranked ? scores.to(at::kFloat) : scores;
+    if (!ranked) order = std::get<1>(scores.sort(/*stable=*/true, /*dim=*/0, /*descending=*/true));
+    at::Tensor ws = at::empty({(int64_t)pairs}, dets.options().dtype(at::kByte));
+    const int rc = ops3d_nms3d_pairs(
+        b.data_ptr<float>(), b.stride(0), b.stride(1), ranked ? s.data_ptr<float>() : nullptr, ranked ? s.stride(0) : 0,
+        ranked ? nullptr : order.data_ptr<int64_t>(), n, thr, ws.data_ptr(), pairs, keep.data_ptr<int64_t>(),
+        num.data_ptr<int32_t>(), stream_of(dets));
+    if (rc != OPS3D_FDA_OK) throw std::runtime_error("nms_3d: kernel launch failed");
+    const int kept = num.item<int32_t>();
+    if (kept >= 0) return keep.narrow(0, 0, kept);
+  }
+  if (!order.defined()) order = std::get<1>(scores.sort(/*stable=*/true, /*dim=*/0, /*descending=*/true));
+  const at::Tensor boxes = dets.index_select(0, order).to(at::kFloat).contiguous();
+  const size_t wsb = ops3d_nms3d_workspace_bytes(n);
+  at::Tensor ws = at::empty({(int64_t)wsb}, dets.options().dtype(at::kByte));
+  const int rc = ops3d_nms3d(boxes.data_ptr<float>(), order.data_ptr<int64_t>(), n, thr, ws.data_ptr(), wsb,
+                             keep.data_ptr<int64_t>(), num.data_ptr<int32_t>(), stream_of(dets));
   if (rc == OPS3D_FDA_EINVAL) throw std::invalid_argument("nms_3d: too many boxes (at most 2^19)");
   if (rc != OPS3D_FDA_OK) throw std::runtime_error("nms_3d: kernel launch failed");
   return keep.narrow(0, 0, num.item<int32_t>());

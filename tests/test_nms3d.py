@@ -113,3 +113,112 @@ def test_gpu_degenerate_and_thresholds(gpu_device):
         assert got == O.nms3d(boxes, scores, thr).tolist(), thr
     with pytest.raises(RuntimeError, match="CPU"):
         _C.nms_3d(torch.from_numpy(boxes), torch.from_numpy(scores), 0.5)
+
+
+# --- the pair path (ops3d_nms3d_pairs) against the mask path (ops3d_nms3d) ---------------------
+def test_pairs_host_rules():
+    """Which calls the pair path takes, and its refusals before any device work (no GPU needed)."""
+    from ops3d_amd import _C
+
+    lib = _C._lib
+    assert lib.ops3d_nms3d_pairs_workspace_bytes(0) == 0
+    assert lib.ops3d_nms3d_pairs_workspace_bytes((1 << 18) + 1) == 0
+    assert [lib.ops3d_nms3d_pairs_ranks(n) for n in (0, 1, 8192, 8193)] == [0, 1, 1, 0]
+    for n in (1, 64, 8192, 8193, 1 << 18):
+        # boxes in score order, padded to blocks of 64 (32 bytes each), and the pair lists
+        assert lib.ops3d_nms3d_pairs_workspace_bytes(n) >= (n + 63) // 64 * 64 * 32 + n * 64 * 8
+    p = 256
+
+    def call(n, thr, order=None, scores=p, ws=p, wsb=1 << 40):
+        return lib.ops3d_nms3d_pairs(p, 6, 1, scores, 1, order, n, thr, ws, wsb, p, p, None)
+
+    bad = (call(10, -0.5), call(10, float("nan")), call((1 << 18) + 1, 0.5, order=p), call(9000, 0.5),
+           call(10, 0.5, order=p), call(10, 0.5, scores=None), call(10, 0.5, wsb=64), call(10, 0.5, ws=p + 8))
+    assert set(bad) == {1}   # EINVAL
+
+
+def test_pair_block_enumeration():
+    """The pair kernel's folded grid (row blocks p and last - p share last + 2 column blocks) visits
+    every block pair on or above the diagonal once."""
+    for nblk in (1, 2, 3, 8, 63, 64, 65, 128):
+        seen = []
+        for bid in range((nblk + 1) // 2 * (nblk + 1)):
+            p, k = divmod(bid, nblk + 1)
+            if k < nblk - p:
+                seen.append((p, p + k))
+            elif nblk - 1 - p != p:
+                rb = nblk - 1 - p
+                seen.append((rb, rb + k - (nblk - p)))
+        assert sorted(seen) == [(r, c) for r in range(nblk) for c in range(r, nblk)]
+    # and its row index of pair p among nr x nc, formed in fp32, is p // nc
+    p = np.arange(64 * 64)
+    for nc in range(1, 65):
+        inv = np.float32(1) / np.float32(nc)
+        got = ((p.astype(np.float32) + np.float32(0.5)) * inv).astype(np.int64)
+        assert np.array_equal(got, p // nc), nc
+
+
+def _mask_path(boxes, scores, thr):
+    """Kept indices by torch's stable sort and the mask kernels, through the C ABI."""
+    from ops3d_amd import _C
+
+    lib, n = _C._lib, boxes.shape[0]
+    order = torch.sort(scores, stable=True, descending=True)[1]
+    b = boxes.index_select(0, order).float().contiguous()
+    wsb = lib.ops3d_nms3d_workspace_bytes(n)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=boxes.device)
+    keep = torch.empty(n, dtype=torch.long, device=boxes.device)
+    num = torch.empty(1, dtype=torch.int32, device=boxes.device)
+    st = torch.cuda.current_stream().cuda_stream
+    assert lib.ops3d_nms3d(b.data_ptr(), order.data_ptr(), n, thr, ws.data_ptr(), wsb, keep.data_ptr(),
+                           num.data_ptr(), st) == 0
+    return keep[: int(num.item())].cpu().tolist()
+
+
+def _chain(n):
+    """Overlapping boxes in a row: each depends on the one before."""
+    lo = np.zeros((n, 3), np.float32)
+    lo[:, 0] = np.arange(n)
+    return np.concatenate([lo, lo + np.float32([2.2, 1, 1])], 1).astype(np.float32), np.ones(n, np.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,n,thr", [
+    ("random", 2, 0.3), ("random", 127, 0.0), ("random", 4096, 0.1), ("random", 8192, 0.3), ("random", 8193, 0.3),
+    ("random", 65537, 0.5), ("random", 1 << 18, 0.5), ("random", (1 << 18) + 1, 0.5), ("dense", 3000, 0.1), ("dense", 9001, 0.2), ("chain", 40, 0.2), ("chain", 3000, 0.2),
+    ("chain", 10000, 0.2), ("special", 1000, 0.25), ("special", 9000, 0.0), ("random", 700, -0.5),
+    ("strided", 500, 0.3), ("half", 500, 0.3), ("double", 500, 0.3), ("double", 9000, 0.3)])
+def test_gpu_pairs_same_as_mask(gpu_device, kind, n, thr):
+    """Every route of nms_3d gives the mask path's list: ranks by counting and by torch's sort, the
+    cell order, lists that overflow (dense) and chains beyond the rounds (both fall back), scores
+    with ties, NaN, infinities and both zeros, boxes with NaN, infinite, inverted and zero extents,
+    strided and other types."""
+    from fda_helpers import log
+
+    from ops3d_amd import _C
+
+    log(f"[case] nms3d pairs {kind} n={n} thr={thr}")
+    boxes, scores = _chain(n) if kind == "chain" else _clustered(n, 3)
+    if kind == "dense":
+        boxes[:, :3] = boxes[:, :3] * np.float32(0.01)
+        boxes[:, 3:] = boxes[:, :3] + np.float32(5.0)
+    if kind == "special":
+        boxes[::9, 0] = np.nan
+        boxes[1::31, 4] = np.inf
+        boxes[2::37, :3] = -np.inf
+        boxes[3::11, 3:] = boxes[3::11, :3]
+        boxes[4::13, 3:] = boxes[4::13, :3] - 1
+        scores[::17] = np.nan
+        scores[1::19] = np.inf
+        scores[2::23] = -np.inf
+        scores[3::5] = 0.0
+        scores[4::10] = -0.0
+    b, s = torch.from_numpy(boxes).to(gpu_device), torch.from_numpy(scores).to(gpu_device)
+    if kind == "strided":
+        b = torch.cat([b, b], 1).t().contiguous().t()[:, 6:12]
+        s = torch.stack([s, -s], 1)[:, 0]
+    if kind == "half":
+        b, s = b.half(), s.half()
+    if kind == "double":
+        b, s = b.double(), s.double()
+    assert _C.nms_3d(b, s, thr).cpu().tolist() == _mask_path(b, s, thr)

@@ -46,7 +46,7 @@ OPS3D_FDA_API int ops3d_roi_align3d_to_channels_last(const void *features, void 
                                                      int D, int H, int W, void *stream);
 
 /* Bytes of workspace ops3d_roi_align3d_backward needs for R rois and output bins PD x PH x PW,
- * 16-byte aligned: when PD, PH, PW <= 64 and PD*PH*PW <= 384 (the backward is then a gather
+ * 16-byte aligned: when PD, PH, PW <= 64, PD*PH*PW <= 384 and C <= 2^20 (the backward is then a gather
  * straight into grad_input) the per-roi axis weight tables, R*(D*PD + H*PH + W*PW + D + H + W)*4
  * bytes rounded up to 16, plus a channels-last copy of grad_output, R*PD*PH*PW*C elements (0
  * when R = 0); else N*C*D*H*W*4 (the gradient is accumulated channels-last in fp32 by atomics,

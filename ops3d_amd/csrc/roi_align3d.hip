@@ -20,7 +20,7 @@
 // output has at most 64 bins per axis and 384 in all (each voxel sums, in registers, the rois
 // that reach it, in roi order: no atomics, the same bits on every run; the workspace holds the
 // rois' axis weight tables and a channels-last copy of grad_output),
-// otherwise by fp32 atomics into a channels-last workspace (64 lanes = 64 contiguous channels
+// otherwise (or with more than 2^20 channels) by fp32 atomics into a channels-last workspace (64 lanes = 64 contiguous channels
 // per atomic instruction) transposed into grad_input afterwards.  A roi whose batch index is
 // outside [0, N) reads and writes nothing (its output is 0; the reference indexes out of
 // bounds).
@@ -28,6 +28,8 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "../../include/ops3d_roi_align3d.h"
 
@@ -490,299 +492,463 @@ __global__ __launch_bounds__(64 * kBwdWaves) void roi_align3d_backward_kernel(co
   }
 }
 
-// Backward as a gather (no atomics): a block owns a tile of 4 x 8 x 8 voxels of one batch item
-// (a thread per voxel) and 16 channels, and sums into registers the contributions of every roi
-// whose footprint reaches the tile, rois in index order, so the result is the same on every run.
-// The weights are separable: voxel (z, y, x) gets, from roi r, the sum over bins (pd, ph, pw) of
-// WZ[z][pd] * WY[y][ph] * WX[x][pw] * top[r, c, pd, ph, pw] / count, where WZ[z][pd] is the sum of
-// bin pd's z-sample tap weights on z (and so on) -- the sum over the bin's samples of their
-// corner weights.  The block takes its rois in groups, so that one round trip to memory serves
-// several rois: for up to 8 rois it finds the bins that reach the tile on each axis (a thread
-// per (roi, tile position, bin)), keeps the longest prefix whose bin boxes and weight tables fit
-// the LDS arenas, writes their tables and stages top for their boxes and its 16 channels as
-// fp32, and each thread then walks, roi by roi, the nonzero bins of its voxel.  Needs at most 64
-// bins per axis and 384 in all (else the atomic path below is used).
-constexpr int kGTZ = 4, kGTY = 8, kGTX = 8;   // tile: 256 voxels, a thread each
-constexpr int kGPos = kGTZ + kGTY + kGTX;      // tile positions over the three axes
-constexpr int kGCC = 16;                       // channels per block (registers per thread)
+// Backward as a gather (no atomics).  From roi r voxel (z, y, x) gets the sum over bins
+// (pd, ph, pw) of WZ[pd][z] * WY[ph][y] * WX[pw][x] * top[r, c, pd, ph, pw] / count, where
+// WZ[pd][z] is the sum of bin pd's z-sample tap weights on z (and so on) -- the sum over the bin's
+// samples of their corner weights, separable because the samples form a full grid.  A wave owns a
+// tile of 4 x 4 x 4 voxels and 64 channels, a lane per channel, its 64 sums in registers, and adds
+// up the rois whose footprint reaches the tile in index order, so the result is the same on every
+// run.  With channels on the lanes everything but top is uniform over the wave: weights, bin
+// ranges and loop bounds sit in scalar registers, no lane diverges and nothing is staged in LDS,
+// and the sum is taken axis by axis -- over pw into 4 x positions, over ph into 4 x 4, over pd into
+// the 64 voxels -- about 5 multiply-adds per voxel and roi instead of one per bin combination.
+// A lane's top values of a bin row (one 128-byte line per bin from the channels-last copy) are
+// loaded one row ahead.
+// Three passes fill the workspace's inputs: roi_axis_table_kernel, grad_channels_last_kernel, and
+// this kernel reads them.  Needs at most 64 bins per axis and 384 in all (else the atomic path).
+// What it measured, and what bounds it: at backward().
+constexpr int kGT = 4;                           // tile edge
+constexpr int kGRun = 128;                       // consecutive tiles of one XCD when not ordered
 constexpr int kGMaxAxisBins = 64, kGMaxBins = 384;
-constexpr int kGGroup = 8;                     // rois examined per group
-constexpr int kGTab = 2048;                    // weight-table arena (floats)
-constexpr int kGList = 128;                    // rois per compaction batch
 
-__host__ __device__ inline bool gather_fits(int PD, int PH, int PW) {
-  return PD <= kGMaxAxisBins && PH <= kGMaxAxisBins && PW <= kGMaxAxisBins && PD * PH * PW <= kGMaxBins;
+constexpr int kGMaxChannels = 1 << 20;           // a roi's bins within 32-bit byte offsets
+
+__host__ __device__ inline bool gather_fits(int C, int PD, int PH, int PW) {
+  return C <= kGMaxChannels && PD <= kGMaxAxisBins && PH <= kGMaxAxisBins && PW <= kGMaxAxisBins && PD * PH * PW <= kGMaxBins;
 }
+__host__ __device__ inline int tiles_of(int n) { return (n + kGT - 1) / kGT; }
 
-// Whether a roi's taps on one axis can reach [t0, t0 + T): its samples lie in [start, end]
-// (coordinates), their taps in [floor(max(start, 0)), floor(max(end, 0)) + 1], none if
-// start > size.
-__device__ __forceinline__ bool axis_reaches(float start, float end, int size, int t0, int T) {
-  if (start > (float)size) return false;
-  const float lo = floorf(fmaxf(start, 0.f)), hi = floorf(fmaxf(end, 0.f)) + 1.f;
-  return !(hi < (float)t0 || lo > (float)(t0 + T - 1));
-}
+// A tile's bins on one axis: first, last (first > last: none); bit 31 of the z words: the roi's top
+// holds an infinity or NaN.
+constexpr uint32_t kNoBins = 1u;                 // first 1, last 0
+constexpr uint32_t kNonFinite = 0x80000000u;
+__device__ __forceinline__ int first_bin(uint32_t w) { return (int)(w & 0xffu); }
+__device__ __forceinline__ int last_bin(uint32_t w) { return (int)((w >> 8) & 0xffu); }
 
-// A roi's parameters in LDS (the Roi fields the gather needs).
-struct GatherRoi {
-  float s[3], bin[3], inv_count;   // z, y, x
-  int grid[3];
-};
-// Bin ranges of one roi of a group: [first, last] bin reaching the tile per axis, and per tile
-// position (z positions, then y, then x).
-struct GatherRanges {
-  int box[3][2];
-  int pos[kGPos][2];
-};
-constexpr int kGRangeInts = (int)(sizeof(GatherRanges) / sizeof(int));
-
-// Per-roi axis tables of the gather backward, made once per call instead of in every tile block
-// that the roi reaches (each of them recomputed them per 16-channel block): for roi r and axis a
-// (size S_a, P_a bins), wt[r][a][x][p] = axis_weight_at(x, .., p, ..) for every position x of
-// the axis, and ft[r][a][x] = the first and last bin with a nonzero weight at x (low and high
-// 16 bits; first > last when none).  The gather kernel reads the same values it computed before.
-// Layout per roi: floats D*PD (z), H*PH (y), W*PW (x); ints D, H, W.
+// Per-roi axis tables, made once per call: for roi r and axis a (size S, P bins) the weights
+// wt[r][a][p][x] of every bin at every position (z's divided by the sample count), and for every
+// tile of 4 positions the first and last bin with a nonzero weight in it, tr[tile][r] (tiles of z,
+// then y, then x: consecutive rois together, as the gather tests them).
 template <typename T>
-__global__ __launch_bounds__(256) void roi_axis_table_kernel(const T *rois, float *wt, uint32_t *ft, int D, int H,
-                                                             int W, int PD, int PH, int PW, float scale, int sr,
-                                                             int order) {
+__global__ __launch_bounds__(256) void roi_axis_table_kernel(const T *rois, float *wt, uint32_t *tr, int D, int H,
+                                                             int W, int PD, int PH, int PW, int R, float scale,
+                                                             int sr, int order) {
   const int r = blockIdx.x, ax = blockIdx.y;
   const Roi q = roi_setup(rois, r, scale, sr, PD, PH, PW);
   const int S = ax == 0 ? D : (ax == 1 ? H : W), P = ax == 0 ? PD : (ax == 1 ? PH : PW);
   const float st = ax == 0 ? q.sd : (ax == 1 ? q.sh : q.sw), bn = ax == 0 ? q.bd : (ax == 1 ? q.bh : q.bw);
   const int gr = ax == 0 ? q.gd : (ax == 1 ? q.gh : q.gw);
-  const size_t wofs = (size_t)r * ((size_t)D * PD + (size_t)H * PH + (size_t)W * PW) +
-                      (ax == 0 ? 0 : (ax == 1 ? (size_t)D * PD : (size_t)D * PD + (size_t)H * PH));
-  const size_t fofs = (size_t)r * ((size_t)D + H + W) + (ax == 0 ? 0 : (ax == 1 ? (size_t)D : (size_t)D + H));
-  for (int x = threadIdx.x; x < S; x += 256) {
-    uint32_t first = 0xffffu, last = 0u;
-    for (int p = 0; p < P; ++p) {
-      const float w = axis_weight_at(x, st, p, bn, gr, S, order);
-      wt[wofs + (size_t)x * P + p] = w;
-      if (w != 0.f) {
-        first = min(first, (uint32_t)p);
-        last = (uint32_t)p;
+  float *w = wt + (size_t)r * ((size_t)D * PD + (size_t)H * PH + (size_t)W * PW) +
+             (ax == 0 ? 0 : (ax == 1 ? (size_t)D * PD : (size_t)D * PD + (size_t)H * PH));
+  uint32_t *t = tr + (size_t)(ax == 0 ? 0 : (ax == 1 ? tiles_of(D) : tiles_of(D) + tiles_of(H))) * R + r;
+  const float norm = ax == 0 ? 1.f / q.count : 1.f;
+  for (int x0 = 0; x0 < S; x0 += 256) {
+    const int x = x0 + threadIdx.x;
+    int first = 0xff, last = 0;
+    if (x < S)
+      for (int p = 0; p < P; ++p) {
+        const float v = axis_weight_at(x, st, p, bn, gr, S, order);
+        w[(size_t)p * S + x] = v * norm;
+        if (v != 0.f) {
+          first = min(first, p);
+          last = p;
+        }
       }
+    // over the tile's 4 positions (4 consecutive lanes)
+#pragma unroll
+    for (int d = 1; d < kGT; d <<= 1) {
+      first = min(first, __shfl_xor(first, d));
+      last = max(last, __shfl_xor(last, d));
     }
-    ft[fofs + x] = first | (last << 16);
+    if (x < S && x % kGT == 0) t[(size_t)(x / kGT) * R] = first == 0xff ? kNoBins : (uint32_t)(first | (last << 8));
   }
 }
 
+// top [R, C, bins] -> [R, bins, C].  A block copies kCopyChannels channels of one roi, which are one
+// contiguous run: read in 16-byte pieces into LDS as they lie (at the run's alignment), written a
+// bin at a time, a lane per channel.  Also marks rois that hold an infinity or NaN.
+template <typename T> constexpr int kCopyChannels = sizeof(T) == 4 ? 32 : 64;   // at most 48 KB of LDS
 template <typename T>
-__global__ __launch_bounds__(256) void roi_align3d_backward_gather_kernel(const T *top_cl, const T *rois, T *grad,
-                                                                          const float *wt, const uint32_t *ft, bool vec4,
-                                                                          int N,
-                                                                          int C, int D, int H, int W, int R, int PD,
-                                                                          int PH, int PW, float scale, int sr,
-                                                                          int order) {
-#pragma clang fp contract(off)
-  __shared__ float4 g_l[kGCC / 4][kGMaxBins];   // [channel quad][bin of the group's boxes]
-  __shared__ float tab_l[kGTab];                // the group's weight tables
-  __shared__ GatherRoi roi_l[kGList];
-  __shared__ int rid_l[kGList];
-  __shared__ GatherRanges rng_l[kGGroup];
-  __shared__ int goff_l[kGGroup + 1][2];         // per group roi: first bin, first table entry
-  __shared__ int cnt_l[4], gsize_l;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int ntx = (W + kGTX - 1) / kGTX, nty = (H + kGTY - 1) / kGTY, ntz = (D + kGTZ - 1) / kGTZ;
-  const int ncc = (C + kGCC - 1) / kGCC;
-  int64_t bid = blockIdx.x;
-  const int txi = (int)(bid % ntx);
-  bid /= ntx;
-  const int tyi = (int)(bid % nty);
-  bid /= nty;
-  const int tzi = (int)(bid % ntz);
-  bid /= ntz;
-  const int cc = (int)(bid % ncc), n = (int)(bid / ncc);
-  const int t0[3] = {tzi * kGTZ, tyi * kGTY, txi * kGTX};
-  const int c0 = cc * kGCC;
-  const int zl = tid / (kGTY * kGTX), yl = (tid / kGTX) % kGTY, xl = tid % kGTX;
-  const int S[3] = {D, H, W}, TT[3] = {kGTZ, kGTY, kGTX};
-  const int pos0[3] = {0, kGTZ, kGTZ + kGTY};     // first position of each axis in the ranges
-  const int64_t pvol = (int64_t)PD * PH * PW;
-  const size_t wroi = (size_t)D * PD + (size_t)H * PH + (size_t)W * PW, froi = (size_t)D + H + W;
-  const size_t wax[3] = {0, (size_t)D * PD, (size_t)D * PD + (size_t)H * PH}, fax[3] = {0, (size_t)D, (size_t)D + H};
-  const int PA[3] = {PD, PH, PW};
+__global__ __launch_bounds__(256) void grad_channels_last_kernel(const T *top, T *top_cl, uint32_t *tr, int C, int bins,
+                                                                 int ntz, int R) {
+  extern __shared__ __align__(16) unsigned char copy_lds[];
+  constexpr int E = 16 / (int)sizeof(T), CB = kCopyChannels<T>;
+  T *l = reinterpret_cast<T *>(copy_lds);
+  const int t = threadIdx.x, r = blockIdx.x, c0 = blockIdx.y * CB, nc = min(CB, C - c0);
+  const T *src = top + ((int64_t)r * C + c0) * bins;
+  const int n = nc * bins, shift = (int)((reinterpret_cast<uintptr_t>(src) & 15u) / sizeof(T));
+  const int lead = min(n, (E - shift) % E);   // elements before the first 16-byte boundary
+  bool bad = false;
+  const auto check = [&](T v) { bad |= !(fabsf(to_f(v)) < INFINITY); };
+  if (t < lead) {
+    l[shift + t] = src[t];
+    check(src[t]);
+  }
+  const int pieces = (n - lead) / E;
+  for (int p = t; p < pieces; p += 256) {
+    const uint4 u = *reinterpret_cast<const uint4 *>(src + lead + p * E);
+    *reinterpret_cast<uint4 *>(l + shift + lead + p * E) = u;
+    const T *e = reinterpret_cast<const T *>(&u);
+#pragma unroll
+    for (int k = 0; k < E; ++k) check(e[k]);
+  }
+  for (int e = lead + pieces * E + t; e < n; e += 256) {
+    l[shift + e] = src[e];
+    check(src[e]);
+  }
+  const bool any = __syncthreads_or(bad) != 0;
+  if (any)
+    for (int z = t; z < ntz; z += 256) atomicOr(&tr[(size_t)z * R + r], kNonFinite);
+  const int ch = t % CB;
+  T *dst = top_cl + (int64_t)r * bins * C + c0 + ch;
+  if (ch < nc)
+    for (int b = t / CB; b < bins; b += 256 / CB) dst[(int64_t)b * C] = l[shift + ch * bins + b];
+}
 
-  float acc[kGCC];
+// How many rois reach each tile (at most 255 counted): a wave per tile of one batch item.
+template <typename T>
+__global__ __launch_bounds__(256) void roi_tile_count_kernel(const T *__restrict__ rois, const uint32_t *__restrict__ tr,
+                                                             uint8_t *__restrict__ counts, int ntz, int nty, int ntx,
+                                                             int R, int tiles) {
+  const int lane = threadIdx.x & 63, tile = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (tile >= tiles) return;
+  const int tx = tile % ntx, ty = tile / ntx % nty, tz = tile / (ntx * nty) % ntz, n = tile / (ntx * nty * ntz);
+  int c = 0;
+#pragma unroll 4
+  for (int r = lane; r < R; r += 64) {
+    const uint32_t z = tr[(size_t)tz * R + r], y = tr[(size_t)(ntz + ty) * R + r], x = tr[(size_t)(ntz + nty + tx) * R + r];
+    const int item = (int)to_f(rois[(int64_t)r * 7]);
+    c += item == n && first_bin(z) <= last_bin(z) && first_bin(y) <= last_bin(y) && first_bin(x) <= last_bin(x) ? 1 : 0;
+  }
 #pragma unroll
-  for (int k = 0; k < kGCC; ++k) acc[k] = 0.f;
-  for (int rb = 0; rb < R; rb += kGList) {
-    // the rois of batch item n whose taps can reach the tile, in index order, with their
-    // parameters in LDS
-    const int r = rb + tid;
-    bool hit = false;
-    Roi q;
-    if (tid < kGList && r < R) {
-      q = roi_setup(rois, r, scale, sr, PD, PH, PW);
-      hit = q.b == n && axis_reaches(q.sd, q.sd + q.bd * (float)PD, D, t0[0], kGTZ) &&
-            axis_reaches(q.sh, q.sh + q.bh * (float)PH, H, t0[1], kGTY) &&
-            axis_reaches(q.sw, q.sw + q.bw * (float)PW, W, t0[2], kGTX);
-    }
-    const uint64_t m = __ballot(hit);
-    if (lane == 0) cnt_l[wv] = __popcll(m);
-    __syncthreads();
-    int off = 0, tot = 0;
-    for (int w = 0; w < 4; ++w) {
-      off += w < wv ? cnt_l[w] : 0;
-      tot += cnt_l[w];
-    }
-    if (hit) {
-      const int i = off + __popcll(m & ((1ull << lane) - 1ull));
-      rid_l[i] = r;
-      GatherRoi g;
-      g.s[0] = q.sd, g.s[1] = q.sh, g.s[2] = q.sw;
-      g.bin[0] = q.bd, g.bin[1] = q.bh, g.bin[2] = q.bw;
-      g.grid[0] = q.gd, g.grid[1] = q.gh, g.grid[2] = q.gw;
-      g.inv_count = 1.f / q.count;
-      roi_l[i] = g;
-    }
-    for (int li = 0; li < tot;) {
-      const int gmax = min(kGGroup, tot - li);
-      for (int i = tid; i < kGGroup * kGRangeInts; i += 256)
-        reinterpret_cast<int *>(rng_l)[i] = (i & 1) ? -1 : (1 << 30);
-      __syncthreads();   // (also: the previous group's sums are done with the LDS state)
-      // 1. bin ranges of the next gmax rois, from the axis tables: a thread per (roi, position)
-      for (int e = tid; e < gmax * kGPos; e += 256) {
-        const int w = e / kGPos, k = e - w * kGPos;
-        const int ax = k < kGTZ ? 0 : (k < kGTZ + kGTY ? 1 : 2), pos = k - pos0[ax];
-        const int at = t0[ax] + pos;
-        if (at < S[ax]) {
-          const uint32_t fl = ft[(size_t)rid_l[li + w] * froi + fax[ax] + at];
-          const int first = (int)(fl & 0xffffu), last = (int)(fl >> 16);
-          if (first <= last) {
-            atomicMin(&rng_l[w].box[ax][0], first);
-            atomicMax(&rng_l[w].box[ax][1], last);
-            rng_l[w].pos[k][0] = first;
-            rng_l[w].pos[k][1] = last;
-          }
-        }
-      }
-      __syncthreads();
-      // 2. the group: the longest prefix whose boxes and tables fit (at least one roi)
-      if (tid == 0) {
-        int nbin = 0, ntab = 0, gs = 0;
-        for (; gs < gmax; ++gs) {
-          const GatherRanges &rg = rng_l[gs];
-          int b = 1, t = 0;
-          for (int ax = 0; ax < 3; ++ax) {
-            const int nb = rg.box[ax][1] < 0 ? 0 : rg.box[ax][1] - rg.box[ax][0] + 1;
-            b *= nb;
-            t += TT[ax] * nb;
-          }
-          if (b == 0) t = 0;   // reaches nothing: no table, no bins
-          if (gs > 0 && (nbin + b > kGMaxBins || ntab + t > kGTab)) break;
-          goff_l[gs][0] = nbin;
-          goff_l[gs][1] = ntab;
-          nbin += b;
-          ntab += t;
-        }
-        goff_l[gs][0] = nbin;
-        goff_l[gs][1] = ntab;
-        gsize_l = gs;
-      }
-      __syncthreads();
-      const int gs = gsize_l;
-      // 3. the group's tables (weights of the box bins at the tile positions) ...
-      const int ntab = goff_l[gs][1], nbin = goff_l[gs][0];
-      for (int e = tid; e < ntab; e += 256) {
-        int w = 0;
-        while (goff_l[w + 1][1] <= e) ++w;
-        const GatherRanges &rg = rng_l[w];
-        int f = e - goff_l[w][1], ax = 0;
-        for (; ax < 2; ++ax) {
-          const int sz = TT[ax] * (rg.box[ax][1] - rg.box[ax][0] + 1);
-          if (f < sz) break;
-          f -= sz;
-        }
-        const int nb = rg.box[ax][1] - rg.box[ax][0] + 1;
-        const int pos = f / nb, p = rg.box[ax][0] + (f - pos * nb);
-        const int at = t0[ax] + pos;
-        tab_l[e] = at < S[ax] ? wt[(size_t)rid_l[li + w] * wroi + wax[ax] + (size_t)at * PA[ax] + p] : 0.f;
-      }
-      // ... and top for their boxes of bins and the block's channels, as fp32, from the
-      // channels-last copy [R, bins, C] (consecutive threads on consecutive channel quads of one
-      // bin: the block's 16 channels of a bin are one contiguous run)
-      for (int e = tid; e < nbin * (kGCC / 4); e += 256) {
-        const int gb = e / (kGCC / 4), k4 = e - gb * (kGCC / 4);
-        int w = 0;
-        while (goff_l[w + 1][0] <= gb) ++w;
-        const GatherRanges &rg = rng_l[w];
-        const int lb = gb - goff_l[w][0];
-        const int nby = rg.box[1][1] - rg.box[1][0] + 1, nbx = rg.box[2][1] - rg.box[2][0] + 1;
-        const int bx = lb % nbx, bzy = lb / nbx, by = bzy % nby, bz = bzy / nby;
-        const int c = c0 + 4 * k4;
-        const T *src = top_cl + ((int64_t)rid_l[li + w] * pvol +
-                                 ((int64_t)(rg.box[0][0] + bz) * PH + rg.box[1][0] + by) * PW + rg.box[2][0] + bx) *
-                                    C + c;
-        float4 v;
-        if (vec4 && c < C) {   // 4 channels, one 8- or 16-byte load
-          float f[4];
-          if constexpr (sizeof(T) == 4) {
-            const float4 u = *reinterpret_cast<const float4 *>(src);
-            f[0] = u.x; f[1] = u.y; f[2] = u.z; f[3] = u.w;
-          } else {
-            const uint2 u = *reinterpret_cast<const uint2 *>(src);
-            const uint32_t wd[2] = {u.x, u.y};
+  for (int d = 32; d > 0; d >>= 1) c += __shfl_xor(c, d);
+  if (lane == 0) counts[tile] = (uint8_t)min(c, 255);
+}
+
+// Tiles by decreasing count (a counting sort in one block): order[rank] = tile.
+__global__ __launch_bounds__(1024) void roi_tile_order_kernel(const uint8_t *counts, unsigned short *order, int tiles) {
+  __shared__ uint32_t at_l[256];
+  const int t = threadIdx.x;
+  if (t < 256) at_l[t] = 0;
+  __syncthreads();
+  for (int i = t; i < tiles; i += 1024) atomicAdd(&at_l[255 - counts[i]], 1u);
+  __syncthreads();
+  if (t < 64) {   // exclusive scan, 4 levels a lane
+    uint32_t v[4], sum = 0;
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-              f[k] = to_f(__builtin_bit_cast(T, (unsigned short)((k & 1) ? (wd[k >> 1] >> 16) : (wd[k >> 1] & 0xffffu))));
-          }
-          v = make_float4(f[0], f[1], f[2], f[3]);
-        } else {
-          v.x = c + 0 < C ? to_f(src[0]) : 0.f;
-          v.y = c + 1 < C ? to_f(src[1]) : 0.f;
-          v.z = c + 2 < C ? to_f(src[2]) : 0.f;
-          v.w = c + 3 < C ? to_f(src[3]) : 0.f;
-        }
-        g_l[k4][gb] = v;
-      }
-      __syncthreads();
-      // 4. this voxel's sums, roi by roi: its bins are a contiguous range per axis
-      for (int w = 0; w < gs; ++w) {
-        const GatherRanges &rg = rng_l[w];
-        if (rg.box[0][1] < 0 || rg.box[1][1] < 0 || rg.box[2][1] < 0) continue;
-        const int pz0 = rg.box[0][0], py0 = rg.box[1][0], px0 = rg.box[2][0];
-        const int nbz = rg.box[0][1] - pz0 + 1, nby = rg.box[1][1] - py0 + 1, nbx = rg.box[2][1] - px0 + 1;
-        const float *tz = tab_l + goff_l[w][1] + zl * nbz - pz0;
-        const float *ty = tab_l + goff_l[w][1] + kGTZ * nbz + yl * nby - py0;
-        const float *tx = tab_l + goff_l[w][1] + kGTZ * nbz + kGTY * nby + xl * nbx - px0;
-        const int gb0 = goff_l[w][0];
-        const float inv_count = roi_l[li + w].inv_count;
-        const int qz0 = rg.pos[zl][0], qz1 = rg.pos[zl][1];
-        const int qy0 = rg.pos[kGTZ + yl][0], qy1 = rg.pos[kGTZ + yl][1];
-        const int qx0 = rg.pos[kGTZ + kGTY + xl][0], qx1 = rg.pos[kGTZ + kGTY + xl][1];
-        for (int pz = qz0; pz <= qz1; ++pz) {
-          const float wz = tz[pz] * inv_count;
-          for (int py = qy0; py <= qy1; ++py) {
-            const float wzy = wz * ty[py];
-            const int lrow = gb0 + ((pz - pz0) * nby + (py - py0)) * nbx - px0;
-            for (int px = qx0; px <= qx1; ++px) {
-              const float wgt = wzy * tx[px];
+    for (int k = 0; k < 4; ++k) {
+      v[k] = at_l[4 * t + k];
+      sum += v[k];
+    }
+    uint32_t inc = sum;
 #pragma unroll
-              for (int k4 = 0; k4 < kGCC / 4; ++k4) {
-                const float4 gv = g_l[k4][lrow + px];
-                acc[4 * k4 + 0] += wgt * gv.x;
-                acc[4 * k4 + 1] += wgt * gv.y;
-                acc[4 * k4 + 2] += wgt * gv.z;
-                acc[4 * k4 + 3] += wgt * gv.w;
-              }
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t u = __shfl_up(inc, d);
+      if (t >= d) inc += u;
+    }
+    uint32_t at = inc - sum;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      at_l[4 * t + k] = at;
+      at += v[k];
+    }
+  }
+  __syncthreads();
+  for (int i = t; i < tiles; i += 1024) order[atomicAdd(&at_l[255 - counts[i]], 1u)] = (unsigned short)i;
+}
+constexpr int kGOrdered = 65535;                 // tiles that are ordered (16-bit numbers)
+constexpr int kGList = 192;                      // rois listed at a time
+
+// One element by a raw buffer load at voffset + soffset.
+template <typename T> using RawOf = std::conditional_t<sizeof(T) == 4, uint32_t, unsigned short>;
+template <typename T>
+__device__ __forceinline__ RawOf<T> load_raw(__amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
+  if constexpr (sizeof(T) == 4)
+    return __builtin_amdgcn_raw_buffer_load_b32(rs, (int)voff, (int)soff, 0);
+  else
+    return __builtin_amdgcn_raw_buffer_load_b16(rs, (int)voff, (int)soff, 0);
+}
+
+template <typename T>
+__global__ __launch_bounds__(64, 4) void roi_align3d_backward_gather_kernel(
+    const T *__restrict__ top_cl, const T *__restrict__ rois, T *__restrict__ grad, const float *__restrict__ wt,
+    const uint32_t *__restrict__ tr, const unsigned short *__restrict__ order, bool vec, int N, int C, int D, int H,
+    int W, int R, int PD, int PH, int PW, int blocks) {
+  __shared__ uint4 list_l[kGList];
+  const int lane = threadIdx.x;
+  const int ntz = tiles_of(D), nty = tiles_of(H), ntx = tiles_of(W);
+  const int ncg = (C + 63) / 64;
+  // Tiles differ several times over in the rois that they meet, so a block is one wave (a larger one
+  // would hold its slots until its last wave is done), and with `order` the crowded tiles come first.
+  // Without it block i runs on XCD i % 8: an XCD takes runs of kGRun neighbouring tiles, which read
+  // the same rois' bins, and which run of a round of eight it takes moves on, so that no XCD gets
+  // only the crowded middle of the volume.
+  int bid = blockIdx.x, cg;
+  if (order) {
+    if (bid >= blocks) return;
+    cg = bid % ncg;
+    bid = order[bid / ncg];
+  } else {
+    const int seq = bid >> 3, round = seq / kGRun, xcd = (bid + round + round / 4 + round / 16) & 7;
+    bid = (round * 8 + xcd) * kGRun + seq % kGRun;
+    if (bid >= blocks) return;
+    const int tiles = ntx * nty * ntz, ng = bid / tiles;
+    cg = ng % ncg;
+    bid = ng / ncg * tiles + bid % tiles;
+  }
+  const int tx = bid % ntx;
+  bid /= ntx;
+  const int ty = bid % nty;
+  bid /= nty;
+  const int tz = bid % ntz, n = bid / ntz;
+  const int c = cg * 64 + lane;
+  const uint32_t cl_bytes = (uint32_t)min(c, C - 1) * (uint32_t)sizeof(T);
+  const int z0 = tz * kGT, y0 = ty * kGT, x0 = tx * kGT;
+  const size_t wroi = (size_t)D * PD + (size_t)H * PH + (size_t)W * PW;
+
+  // the weight of a roi that a lane fetches: axis (z, y, x; 16 lanes each), bin, position
+  const int wax = min(lane >> 4, 2), wbin = (lane >> 2) & 3, wsize = wax == 0 ? D : (wax == 1 ? H : W);
+  const uint32_t wfirst = (uint32_t)((wax == 0 ? z0 : (wax == 1 ? D * PD + y0 : D * PD + H * PH + x0)) + (lane & 3));
+  const auto lane_of = [](float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+  };
+  const auto nonzero = [](float w) { return (__float_as_int(w) << 1) != 0; };
+
+  float acc[kGT][kGT * kGT];
+#pragma unroll
+  for (int z = 0; z < kGT; ++z)
+#pragma unroll
+    for (int i = 0; i < kGT * kGT; ++i) acc[z][i] = 0.f;
+
+  // top of one plane of bins, a row of 4 per register quad: a row is reloaded with the next plane's
+  // as soon as it is used, so four rows are in flight
+  using Raw = RawOf<T>;
+  Raw v[4][4];
+  const uint32_t row_bytes = (uint32_t)(PW * C) * (uint32_t)sizeof(T), plane_bytes = (uint32_t)PH * row_bytes;
+  const auto load_row = [&](Raw(&row)[4], const char *plane, int h, const uint32_t(&off)[4]) {
+    // (buffer loads: the row's offset is a scalar operand; bounded by the roi's bins)
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(plane), (short)0, (int)((uint32_t)PD * plane_bytes), 0x00020000);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) row[k] = load_raw<T>(rs, off[k], (uint32_t)h * row_bytes);
+  };
+  // x sums of a row of up to 4 bins
+  const auto x_sum = [&](float(&t)[kGT], const float(&wx)[4][kGT], const float(&g)[4], int nx) {
+#pragma unroll
+    for (int x = 0; x < kGT; ++x) t[x] = wx[0][x] * g[0];
+#pragma unroll
+    for (int k = 1; k < 4; ++k)
+      if (k < nx)
+#pragma unroll
+        for (int x = 0; x < kGT; ++x) t[x] += wx[k][x] * g[k];
+  };
+
+  int roi = 0;
+  uint32_t b_zy = 0, b_x = 0;   // bins of the roi to come: z | y << 16, x | flag << 16
+  const auto take = [&](int i) {
+    const uint4 e = list_l[i];
+    roi = __builtin_amdgcn_readfirstlane((int)e.x);
+    b_zy = (uint32_t)__builtin_amdgcn_readfirstlane((int)e.y);
+    b_x = (uint32_t)__builtin_amdgcn_readfirstlane((int)e.z);
+  };
+  const auto count = [](uint32_t w) { return last_bin(w) - first_bin(w) + 1; };
+  const auto weights = [&]() {
+    const uint32_t zy = wax == 0 ? b_zy : b_zy >> 16, word = wax == 2 ? b_x : zy;
+    const int p = first_bin(word) + wbin, last = last_bin(word);
+    // positions past the volume's end read the next row: their sums are not stored
+    const float w = (wt + (size_t)roi * wroi)[wfirst + (uint32_t)(min(p, last) * wsize)];
+    return p <= last ? w : 0.f;
+  };
+  const uint32_t bin_bytes = (uint32_t)C * (uint32_t)sizeof(T), roi_bytes = (uint32_t)(PD * PH * PW) * bin_bytes;
+  const auto first_plane = [&]() {
+    const uint32_t bin = (uint32_t)((first_bin(b_zy) * PH + first_bin(b_zy >> 16)) * PW + first_bin(b_x));
+    return reinterpret_cast<const char *>(top_cl) + ((uint64_t)(uint32_t)roi * roi_bytes + bin * bin_bytes);
+  };
+  const auto offsets = [&](uint32_t(&off)[4], int nx) {   // bytes: a bin's channel, at most 384 bins away
+#pragma unroll
+    for (int k = 0; k < 4; ++k) off[k] = (uint32_t)min(k, nx - 1) * bin_bytes + cl_bytes;
+  };
+
+  for (int r0 = 0; r0 < R;) {
+    // the next rois of batch item n that reach the tile, in index order: from the front those with
+    // at most 4 bins on every axis of it and only finite values (nearly all), from the back the
+    // others
+    int narrow = 0, wide = 0;
+    for (; r0 < R && narrow + wide <= kGList - 64; r0 += 64) {
+      const int r = r0 + lane, q = min(r, R - 1);
+      const uint32_t z = tr[(size_t)tz * R + q], y = tr[(size_t)(ntz + ty) * R + q], x = tr[(size_t)(ntz + nty + tx) * R + q];
+      const int item = (int)to_f(rois[(int64_t)q * 7]);
+      const int cz = last_bin(z) - first_bin(z), cy = last_bin(y) - first_bin(y), cx = last_bin(x) - first_bin(x);
+      const bool hit = r < R && item == n && min(cz, min(cy, cx)) >= 0, big = max(cz, max(cy, cx)) > 3 || (z & kNonFinite) != 0;
+      const uint64_t mn = __ballot(hit && !big), mw = __ballot(hit && big), below = (1ull << lane) - 1ull;
+      const uint4 e = make_uint4((uint32_t)r, (z & 0xffffu) | (y << 16), (x & 0xffffu) | ((z & kNonFinite) >> 15), 0u);
+      if (hit) list_l[big ? kGList - 1 - (wide + __popcll(mw & below)) : narrow + __popcll(mn & below)] = e;
+      narrow += __popcll(mn);
+      wide += __popcll(mw);
+    }
+    __builtin_amdgcn_wave_barrier();
+
+    if (narrow > 0) {
+      take(0);
+      uint32_t off[4];
+      const char *plane = first_plane();
+      float w_ahead = weights();
+      int ahead_ny = count(b_zy >> 16), ahead_nx = count(b_x);
+      offsets(off, ahead_nx);
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        load_row(v[h], plane, min(h, ahead_ny - 1), off);
+        __builtin_amdgcn_sched_barrier(0);   // in the order of their use
+      }
+      for (int i = 1; i <= narrow; ++i) {
+        const float w = w_ahead;
+        uint64_t set = __ballot(w != 0.f);   // which weights are not 0, by lane
+        int nx = ahead_nx, ny = ahead_ny;
+        const int nz = count(b_zy);
+        if (i < narrow) {
+          take(i);
+          w_ahead = weights();
+        }
+        float wx[4][kGT];
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int x = 0; x < kGT; ++x) wx[b][x] = lane_of(w, 32 + b * 4 + x);
+        for (int d = 0; d < nz; ++d) {
+          // the plane to load: this roi's next, then the next roi's first (at the end: this one again)
+          if (d + 1 < nz) {
+            plane += plane_bytes;
+          } else if (i < narrow) {
+            plane = first_plane();
+            ahead_ny = count(b_zy >> 16);
+            ahead_nx = count(b_x);
+            offsets(off, ahead_nx);
+          }
+          // (opaque: the compiler would keep every test below in scalar registers over the loop)
+          asm volatile("" : "+s"(set), "+s"(nx), "+s"(ny));
+          float u[kGT * kGT];
+#pragma unroll
+          for (int j = 0; j < kGT * kGT; ++j) u[j] = 0.f;
+#pragma unroll
+          for (int h = 0; h < 4; ++h) {
+            float g[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              g[k] = to_f(__builtin_bit_cast(T, v[h][k]));
+              asm volatile("" : "+v"(g[k]));   // here: v[h][k] is free for the load
+            }
+            __builtin_amdgcn_sched_barrier(0);   // or the loads move up and need registers of their own
+            load_row(v[h], plane, min(h, ahead_ny - 1), off);
+            __builtin_amdgcn_sched_barrier(0);
+            if (h < ny) {
+              float t[kGT];
+              x_sum(t, wx, g, nx);
+#pragma unroll
+              for (int y = 0; y < kGT; ++y)
+                if ((set >> (16 + h * 4 + y)) & 1) {
+                  const float wy = lane_of(w, 16 + h * 4 + y);
+#pragma unroll
+                  for (int x = 0; x < kGT; ++x) u[y * kGT + x] += wy * t[x];
+                }
             }
           }
+#pragma unroll
+          for (int z = 0; z < kGT; ++z)
+            if ((set >> (d * 4 + z)) & 1) {
+              const float wz = lane_of(w, d * 4 + z);
+#pragma unroll
+              for (int j = 0; j < kGT * kGT; ++j) acc[z][j] += wz * u[j];
+            }
         }
       }
-      li += gs;
-      __syncthreads();   // the sums are done with the group's LDS state
     }
-    __syncthreads();   // the batch's counts are read before the next batch writes them
-  }
-  const int z = t0[0] + zl, y = t0[1] + yl, x = t0[2] + xl;
-  if (z < D && y < H && x < W) {
-    const int64_t vol = (int64_t)D * H * W, v = ((int64_t)z * H + y) * W + x;
+
+    // bins smaller than the voxels, or values that are not finite: the bins along x four at a time,
+    // row by row
+    for (int i = 0; i < wide; ++i) {
+      take(kGList - 1 - i);
+      const bool clean = (b_x >> 16) == 0;
+      const float *wz = wt + (size_t)roi * wroi + z0, *wy = wt + (size_t)roi * wroi + (size_t)D * PD + y0,
+                  *wx = wt + (size_t)roi * wroi + (size_t)D * PD + (size_t)H * PH + x0;
+      for (int px = first_bin(b_x); px <= last_bin(b_x & 0xffffu); px += 4) {
+        const int nx = min(4, last_bin(b_x) - px + 1);
+        float wxr[4][kGT];
+        uint32_t off[4];
 #pragma unroll
-    for (int k = 0; k < kGCC; ++k)
-      if (c0 + k < C) grad[((int64_t)n * C + c0 + k) * vol + v] = from_f<T>(acc[k]);
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int x = 0; x < kGT; ++x) wxr[k][x] = k < nx ? wx[(px + k) * W + x] : 0.f;
+        offsets(off, nx);
+        for (int pd = first_bin(b_zy); pd <= last_bin(b_zy); ++pd) {
+          float u[kGT * kGT];
+#pragma unroll
+          for (int j = 0; j < kGT * kGT; ++j) u[j] = 0.f;
+          const char *plane = reinterpret_cast<const char *>(top_cl) +
+                              ((uint64_t)(uint32_t)roi * roi_bytes + ((uint32_t)pd * plane_bytes + (uint32_t)px * bin_bytes));
+          for (int ph = first_bin(b_zy >> 16); ph <= last_bin(b_zy >> 16); ++ph) {
+            load_row(v[0], plane, ph, off);
+            float g[4], t[kGT];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) g[k] = to_f(__builtin_bit_cast(T, v[0][k]));
+            if (clean) {
+              x_sum(t, wxr, g, nx);
+            } else {   // 0 * infinity must not reach a voxel outside the bin
+#pragma unroll
+              for (int x = 0; x < kGT; ++x) t[x] = 0.f;
+#pragma unroll
+              for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int x = 0; x < kGT; ++x)
+                  if (nonzero(wxr[k][x])) t[x] += wxr[k][x] * g[k];
+            }
+#pragma unroll
+            for (int y = 0; y < kGT; ++y) {
+              const float w = wy[ph * H + y];
+              if (nonzero(w))
+#pragma unroll
+                for (int x = 0; x < kGT; ++x) u[y * kGT + x] += w * t[x];
+            }
+          }
+#pragma unroll
+          for (int z = 0; z < kGT; ++z) {
+            const float w = wz[pd * D + z];
+            if (nonzero(w))
+#pragma unroll
+              for (int j = 0; j < kGT * kGT; ++j) acc[z][j] += w * u[j];
+          }
+        }
+      }
+    }
+    __builtin_amdgcn_wave_barrier();   // the list is read before the next rois are written to it
   }
+  if (c >= C) return;
+  T *o = grad + ((int64_t)n * C + c) * D * H * W;
+#pragma unroll
+  for (int z = 0; z < kGT; ++z)
+#pragma unroll
+    for (int y = 0; y < kGT; ++y) {
+      if (z0 + z >= D || y0 + y >= H) continue;
+      T *row = o + ((int64_t)(z0 + z) * H + (y0 + y)) * W + x0;
+      T e[kGT];
+#pragma unroll
+      for (int x = 0; x < kGT; ++x) e[x] = from_f<T>(acc[z][y * kGT + x]);
+      if (vec) {   // W % 4 == 0 and grad aligned: one 8- or 16-byte store
+        if constexpr (sizeof(T) == 4) {
+          *reinterpret_cast<float4 *>(row) = make_float4(e[0], e[1], e[2], e[3]);
+        } else {
+          uint32_t h[2];
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+            h[k] = (uint32_t)__builtin_bit_cast(unsigned short, e[2 * k]) |
+                   ((uint32_t)__builtin_bit_cast(unsigned short, e[2 * k + 1]) << 16);
+          *reinterpret_cast<uint2 *>(row) = make_uint2(h[0], h[1]);
+        }
+      } else {
+#pragma unroll
+        for (int x = 0; x < kGT; ++x)
+          if (x0 + x < W) row[x] = e[x];
+      }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1053,33 +1219,52 @@ inline size_t gather_tables_bytes(int R, int D, int H, int W, int PD, int PH, in
   return (b + 15) & ~(size_t)15;
 }
 
+// Backward.  Measured on bf16 [2, 256, 32, 64, 64], 512 rois of 4-32 voxels, 7^3 bins, one MI355X:
+// tables 7, copy 47, tile counts and order 14, gather 445 us (0.96 ms forward and backward); before,
+// with a block per 4 x 8 x 8 voxels and 16 channels that staged its rois' bins in LDS, a thread per
+// voxel: tables 6, copy 75, gather 1572 us (2.10 ms).  The gather issues 132 M vector instructions
+// (40 % of the issue slots at four waves per SIMD) and waits for its loads for most of the rest:
+// 340 K visits of a roi to a tile and channel group, each 2 to 4 planes of 4 rows.  Steps: the first
+// form (blocks of four waves, dynamic loops, weights by scalar loads) 943 us; rows loaded a plane
+// ahead and weights fetched by the lanes 680; one wave per block 537; crowded tiles first 500 (-45);
+// no spilled registers 445.  Without `order` an XCD's runs of 8 / 32 / 128 / 512 tiles measured
+// 554 / 535 / 522 / 540 us.  Joining the tiles of a block of two or four waves in LDS, to store
+// longer runs, 502 / 520 us against 492; three waves per SIMD 542.
 template <typename T>
 int backward(const void *grad_output, const void *rois, void *grad_input, float *acc, int N, int C, int D, int H,
              int W, int R, int PD, int PH, int PW, float scale, int sr, int order, hipStream_t st) {
-  if (gather_fits(PD, PH, PW)) {
-    const int64_t blocks = (int64_t)N * ((C + kGCC - 1) / kGCC) * ((D + kGTZ - 1) / kGTZ) * ((H + kGTY - 1) / kGTY) *
-                           ((W + kGTX - 1) / kGTX);
+  if (gather_fits(C, PD, PH, PW)) {
+    const int ntz = tiles_of(D), nty = tiles_of(H), ntx = tiles_of(W);
+    const int64_t tiles = (int64_t)N * ntz * nty * ntx, blocks = tiles * ((C + 63) / 64);
+    const int64_t grid = (blocks + 8 * kGRun - 1) / (8 * kGRun) * (8 * kGRun);   // whole rounds of runs
+    if (grid >= ((int64_t)1 << 31)) return OPS3D_FDA_EINVAL;
     // workspace: the per-roi axis tables, then grad_output channels-last [R, bins, C]
     float *wt = acc;
-    uint32_t *ft = reinterpret_cast<uint32_t *>(acc + (size_t)R * ((size_t)D * PD + (size_t)H * PH + (size_t)W * PW));
+    uint32_t *tr = reinterpret_cast<uint32_t *>(acc + (size_t)R * ((size_t)D * PD + (size_t)H * PH + (size_t)W * PW));
     T *top_cl = reinterpret_cast<T *>(reinterpret_cast<char *>(acc) + gather_tables_bytes(R, D, H, W, PD, PH, PW));
-    const int64_t pvol = (int64_t)PD * PH * PW;
+    const int bins = PD * PH * PW;
     if (R > 0) {
       hipLaunchKernelGGL((roi_axis_table_kernel<T>), dim3((unsigned)R, 3), dim3(256), 0, st,
-                         static_cast<const T *>(rois), wt, ft, D, H, W, PD, PH, PW, scale, sr, order);
-      for (int r0 = 0; r0 < R; r0 += 65535) {   // grid z: at most 65535 rois per launch
-        const int nr = min(65535, R - r0);
-        const T *src = static_cast<const T *>(grad_output) + (int64_t)r0 * C * pvol;
-        T *dst = top_cl + (int64_t)r0 * C * pvol;
-        hipLaunchKernelGGL((ncdhw_to_channels_last_kernel<T>), dim3((unsigned)((pvol + 63) / 64), (unsigned)((C + 63) / 64), nr),
-                           dim3(256), 0, st, src, dst, C, pvol,
-                           C % (16 / (int)sizeof(T)) == 0 && pvol % (16 / (int)sizeof(T)) == 0 &&
-                               ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15u) == 0);
-      }
+                         static_cast<const T *>(rois), wt, tr, D, H, W, PD, PH, PW, R, scale, sr, order);
+      constexpr int CB = kCopyChannels<T>;
+      const size_t lds = ((size_t)CB * bins + 16 / sizeof(T)) * sizeof(T);
+      hipLaunchKernelGGL((grad_channels_last_kernel<T>), dim3((unsigned)R, (unsigned)((C + CB - 1) / CB)), dim3(256), lds,
+                         st, static_cast<const T *>(grad_output), top_cl, tr, C, bins, tiles_of(D), R);
     }
-    hipLaunchKernelGGL((roi_align3d_backward_gather_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st, top_cl,
-                       static_cast<const T *>(rois), static_cast<T *>(grad_input), wt, ft, C % 4 == 0, N, C, D, H, W, R,
-                       PD, PH, PW, scale, sr, order);
+    // the tiles' order, in the tables' second part beyond the words that tr takes, where it fits
+    const int64_t used = (int64_t)R * (ntz + nty + ntx) * 4, spare = (int64_t)R * (D + H + W) * 4 - used;
+    unsigned short *order = nullptr;
+    if (tiles <= kGOrdered && tiles * 3 <= spare) {
+      order = reinterpret_cast<unsigned short *>(reinterpret_cast<char *>(tr) + used);
+      uint8_t *counts = reinterpret_cast<uint8_t *>(order + tiles);
+      hipLaunchKernelGGL((roi_tile_count_kernel<T>), dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, st,
+                         static_cast<const T *>(rois), tr, counts, ntz, nty, ntx, R, (int)tiles);
+      hipLaunchKernelGGL(roi_tile_order_kernel, dim3(1), dim3(1024), 0, st, counts, order, (int)tiles);
+    }
+    const bool vec = W % kGT == 0 && (reinterpret_cast<uintptr_t>(grad_input) & (kGT * sizeof(T) - 1)) == 0;
+    hipLaunchKernelGGL((roi_align3d_backward_gather_kernel<T>), dim3((unsigned)grid), dim3(64), 0, st, top_cl,
+                       static_cast<const T *>(rois), static_cast<T *>(grad_input), wt, tr, order, vec, N, C, D, H, W, R, PD,
+                       PH, PW, (int)blocks);
     return hipGetLastError() == hipSuccess ? OPS3D_FDA_OK : OPS3D_FDA_ERUNTIME;
   }
   const int64_t nin = (int64_t)N * C * D * H * W;
@@ -1175,7 +1360,7 @@ size_t ops3d_roi_align3d_backward_workspace_bytes(int dtype, int N, int C, int D
                                                  int PH, int PW) {
   (void)dtype;
   if (N <= 0 || C <= 0 || D <= 0 || H <= 0 || W <= 0 || R < 0 || PD <= 0 || PH <= 0 || PW <= 0) return 0;
-  if (gather_fits(PD, PH, PW))   // the per-roi axis tables and grad_output channels-last
+  if (gather_fits(C, PD, PH, PW))   // the per-roi axis tables and grad_output channels-last
     return R == 0 ? 0
                   : gather_tables_bytes(R, D, H, W, PD, PH, PW) +
                         (size_t)R * C * PD * PH * PW * (dtype == OPS3D_FDA_F32 ? 4 : 2);

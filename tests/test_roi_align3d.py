@@ -368,3 +368,68 @@ def test_gpu_backward_more_rois_than_one_grid_dimension(gpu_device):
     rhs = float((x.double() * full.double()).sum())
     assert abs(lhs - rhs) <= 1e-4 * float((out.double().abs() * g.double().abs()).sum())
     assert torch.allclose(full, halves, rtol=1e-5, atol=1e-4)
+
+
+# --- the gather backward's tiles ------------------------------------------------------------------
+TILE_CASES = [
+    # N, C, (D, H, W), R, pooled, sampling_ratio, dtype
+    (1, 63, (3, 5, 9), 10, (2, 2, 2), 2, torch.float32),          # partial tiles, 63 channels
+    (2, 65, (4, 8, 4), 12, (3, 2, 4), 2, torch.bfloat16),         # whole tiles, a second channel group of 1
+    (1, 7, (1, 1, 1), 4, (2, 2, 2), 1, torch.float32),            # one voxel
+    (1, 8, (6, 7, 8), 420, (2, 2, 2), 1, torch.float32),          # more rois in a tile than are listed at a time
+    (1, 8, (8, 9, 10), 200, (6, 5, 6), 1, torch.bfloat16),        # rois of both kinds (bins below a voxel) in a tile
+    (1, 250, (8, 6, 12), 9, (3, 3, 3), 0, torch.float16),         # runs of grad_output at odd alignments
+    (1, 33, (5, 6, 8), 7, (4, 4, 4), 2, torch.float32),           # 64 bins: one row per lane in the copy
+    (1, 3, (6, 7, 9), 5, (6, 8, 8), 2, torch.bfloat16),           # 384 bins
+    (1, 8, (16, 40, 48), 3, (3, 3, 3), 2, torch.float32),         # few rois, many tiles: the natural tile order
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", range(len(TILE_CASES)))
+def test_gpu_backward_tiles(gpu_device, case):
+    """grad_input of the gather backward at the edges of its tiles, channel groups, roi lists and
+    copies, against the oracle (bars as above: fp32 sums of up to 8 * count terms per voxel)."""
+    from fda_helpers import TOL, assert_close, log
+
+    from ops3d_amd import _C
+
+    N, C, size, R, pooled, sr, dt = TILE_CASES[case]
+    log(f"[case] roi_align3d backward tiles #{case}: N={N} C={C} size={size} R={R} pooled={pooled} sr={sr} {dt}")
+    r = np.random.default_rng(300 + case)
+    rois = torch.from_numpy(_rois(R, N, size, seed=400 + case, lo=-1.0)).to(dt)
+    g = torch.from_numpy(r.normal(size=(R, C) + pooled).astype(np.float32)).to(dt)
+    grad = torch.full((N, C) + size, 7.0, dtype=dt, device=gpu_device)
+    _C.roi_align_3d_backward(g.to(gpu_device), rois.to(gpu_device), grad, *pooled, 1.0, sr, 1)
+    torch.cuda.synchronize()
+    want = O.backward(g.double().numpy(), rois.double().numpy(), (N, C) + size, 1.0, sr, 1)
+    rtol, atol = TOL[dt]
+    assert_close("roi_align grad", grad, want, rtol, atol * (10 if dt == torch.float32 else 1))
+
+
+@pytest.mark.gpu
+def test_gpu_backward_infinities_stay_in_their_bins(gpu_device):
+    """An infinite or NaN gradient reaches the voxels that its bin samples and no others of the tile."""
+    from fda_helpers import assert_close, log
+
+    from ops3d_amd import _C
+
+    log("[case] roi_align3d backward with infinities and NaN")
+    N, C, size, R, pooled = 1, 5, (8, 12, 16), 6, (3, 3, 3)
+    r = np.random.default_rng(5)
+    lo = r.uniform(0.1, 2.0, size=(R, 3))
+    rois = np.concatenate([np.zeros((R, 1)), lo, lo + r.uniform(5.0, 7.5, size=(R, 3))], 1).astype(np.float32)
+    g = r.normal(size=(R, C) + pooled).astype(np.float32)
+    g[1, 2, 0, 1, 1] = np.inf
+    g[3, 0, 2, 2, 0] = np.nan
+    grad = torch.empty((N, C) + size, device=gpu_device)
+    _C.roi_align_3d_backward(torch.from_numpy(g).to(gpu_device), torch.from_numpy(rois).to(gpu_device), grad, *pooled,
+                             1.0, 2, 1)
+    torch.cuda.synchronize()
+    with np.errstate(invalid="ignore"):
+        want = O.backward(g.astype(np.float64), rois.astype(np.float64), (N, C) + size, 1.0, 2, 1)
+    got = grad.cpu().double().numpy()
+    assert 0 < np.sum(~np.isfinite(want)) < 500
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    ok = np.isfinite(want)
+    assert_close("finite part", torch.from_numpy(np.where(ok, got, 0.0)), np.where(ok, want, 0.0), 1e-5, 1e-5)

@@ -60,7 +60,7 @@ OPS3D_FDA_API size_t ops3d_roi_align3d_backward_workspace_bytes(int dtype, int N
  * (the reference's kernel adds into a buffer its caller zeroed; a caller accumulating gradients
  * adds the result itself).  With the bin limits above it is a gather (after passes that write
  * each roi's per-axis bin weights and grad_output channels-last to the workspace): each voxel sums the rois that reach it in
- * roi order, the same bits on every run; else
+ * an order that the rois alone decide, the same bits on every run; else
  * the samples' corner contributions are added by fp32 atomics into the cleared workspace, whose
  * order -- and so the last bit -- can differ between runs, as with the reference's atomics.
  */

@@ -206,10 +206,11 @@ hipError_t launch(int dtype, int which, const Geometry &g, hipStream_t st) {
 //   bucketing matrix: B*G x 64 blocks x tcap uint32, tcap = S/16 + 64 tiles per head (volumes
 //                    cut into more tiles are bucketed with global atomics instead)
 //   tile queues    : 8 uint32 (the tile kernel's per-XCD work counters, cleared by the bucketing)
-//                    and the tile kernel's split factor
+//                    and the tile kernel's parts per tile of each level
 //   split scratch  : when fewer than kSplitTiles tiles can exist (at least ceil(S / tile voxels)
-//                    per head), kSplitSlots fp32 partial tiles [tile voxels][D] for the tile
-//                    kernel's split tiles; else nothing
+//                    per head) or a coarse level's tiles are likely to need it
+//                    (coarse_level_heavy), kSplitSlots fp32 partial tiles [tile voxels][D] for
+//                    the tile kernel's split tiles; else nothing
 //   head-major copies of value (G > 1; head slices of at most head_copy_rows_max(S) rows,
 //   large levels paired) and of grad_output (grad_out_copied)
 constexpr uint64_t kSplitTiles = 2048, kSplitSlots = 2048;
@@ -231,6 +232,21 @@ bool head_major_pays(int S, int G, int D, int e, int Q, int L, int K) {
 // query kernel more than it saves the tile kernel).
 bool grad_out_copied(int B, int Q, int G, int D, int e) {
   return G > 1 && (size_t)B * Q * G * D * e > kDirectGradOutBytes;
+}
+
+// Whether a pyramid of more than kSplitTiles tiles is likely to have a coarse level that the tile
+// kernel should split: every level takes the same number of samples, so a tile of a level of c
+// tiles per head holds 1 / (B G L c) of the entries, to be compared with a block's share.  The
+// levels' shapes are on the device; the coarsest level is taken to hold 1 / 8^(L-1) of the finest
+// (each level half the size of the one before): the wrong guess costs the split's gain, or an empty
+// combine launch.  Only for calls of at least kSplitSamples samples, whose workspace is above the
+// allocation-free entry point's limit without it, so that that entry point refuses nothing more.
+constexpr uint64_t kSplitSamples = 5ull << 18;
+bool coarse_level_heavy(int B, int S, int G, int L, int Q, int K, uint64_t tile_voxels, int threads) {
+  if (L < 2 || (uint64_t)B * Q * G * L * K < kSplitSamples) return false;
+  const uint64_t c = ((uint64_t)S * 7 / 8 >> (3 * (L - 1))) / tile_voxels;
+  const uint64_t blocks = threads >= 1024 ? 256 : (threads >= 512 ? 512 : 768);   // resident (tile_chunk)
+  return (uint64_t)B * G * L * (c > 0 ? c : 1) < blocks;
 }
 
 struct BwdLayout {
@@ -263,9 +279,11 @@ int bwd_layout(int B, int S, int G, int D, int e, int lpu, int L, int Q, int K, 
   ly.off_cursor = o; o += t4;
   ly.off_queue = o; o += 256;
   {
-    const uint64_t tvox = (uint64_t)(2 * tile_threads(lpu, big_tiles(S, lpu)) / lpu);   // voxels of a nominal tile
+    const int nt = tile_threads(lpu, big_tiles(S, lpu));
+    const uint64_t tvox = (uint64_t)(2 * nt / lpu);   // voxels of a nominal tile
     const uint64_t lb = (uint64_t)B * G * ((uint64_t)S + tvox - 1) / tvox;
-    ly.split_slots = (S > 0 && lb < kSplitTiles) ? (uint32_t)kSplitSlots : 0u;
+    ly.split_slots = S > 0 && (lb < kSplitTiles || coarse_level_heavy(B, S, G, L, Q, K, tvox, nt))
+                         ? (uint32_t)kSplitSlots : 0u;
     ly.off_split = o; o += align256((size_t)ly.split_slots * tvox * D * 4);
   }
   ly.tcap = (uint32_t)(S / 16 + 64);

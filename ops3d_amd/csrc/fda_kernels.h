@@ -27,9 +27,12 @@ constexpr int kFwdWavesPerEU = 8;     // minimum waves per SIMD the x-pair forwa
 // Backward query pair kernel: left to itself the compiler takes 107 VGPRs (4 waves per SIMD);
 // 5 waves fit without spills.
 constexpr int kQueryWavesPerEU = 5;
-// Tile splitting (tile kernel): parts per tile aim at kSplitTarget jobs per block, at most
-// kSplitMax parts per tile.
-constexpr uint32_t kSplitTarget = 2u, kSplitMax = 8u;
+// Tile splitting (tile kernel): a part aims at 1/kSplitTarget of a block's share of the entries, at
+// most kSplitMax parts per tile.  Tile kernel with target 2 / 3 / 4: levels 40x48x96 to 5x6x12
+// 1719 / 1484 / 1340 us (bf16, 8 heads; unsplit 7137), 44x56x134 to 11x14x34 2010 / 1902 / 1916
+// (2030), fp32 6 heads x 48 channels 11x27x45 to 3x7x12 285 / 256 / 251 (665), fp16 batch 2
+// 18x40x80 to 5x10x20 707 / 735 / 737 (934).
+constexpr uint32_t kSplitTarget = 4u, kSplitMax = 16u;
 
 // NW raw words from a plain global pointer (aligned to 16 bytes when NW % 4 == 0).
 template <int NW>
@@ -688,7 +691,7 @@ __global__ __launch_bounds__(kBlock) void fda_bwd_query_kernel(const Args a) {
 //      the three contiguous bins of base x0-1, x0, x0+1 -- reading only LDS.
 // The next chunk's entries and stash are loaded during the current chunk.  Every grad_value row
 // of the tile is written once, in T (or added to an fp32 buffer): no zero-fill, no global
-// atomics; split tiles (small volumes) write fp32 partials that a combine kernel adds.  Tiles
+// atomics; split tiles (small volumes, coarse levels) write fp32 partials that a combine kernel adds.  Tiles
 // are scheduled coarse levels first (their tiles hold the most entries), and with G % 8 == 0
 // the tiles of head g run on XCD g % 8, whose L2 then holds that head's grad_output rows.
 
@@ -755,22 +758,53 @@ void fda_bwd_tile_kernel(const Args a) {
     hpx = G / 8;
   }
   const uint32_t nbg = (uint32_t)a.B * (uint32_t)hpx;
-  const uint32_t total = nbg * T_h;
-  // Split tiles: when the group has fewer tiles than twice its blocks, each tile is cut into F
-  // parts (jobs) over its entry range; a part sums into fp32 and writes its partial to a scratch
-  // slot, and the tile's last part to finish adds the others' partials and writes grad_value.
+  // Split tiles: a level whose tiles hold more than a part's share of the entries (few tiles for the
+  // blocks, or a coarse level, whose few tiles take as many samples as a fine level's many) has
+  // each of them cut into F parts (jobs) over its entry range; a part sums into fp32 and writes its
+  // partial to a scratch slot, and fda_bwd_split_combine_kernel adds a tile's parts.  The shares
+  // come from the first head's entries: the same in every block.  Without the split the largest
+  // tile's serial chain of chunks was the kernel's time (figures at kSplitTarget).
+  __shared__ uint32_t parts_l[5], job0_l[6], slot0_l[5];   // per level (coarse first): parts, first job, first slot
   const uint32_t ngroups = a.tile_affinity ? 8u : 1u;
-  uint32_t F = 1;
-  if (a.split_slots > 0 && total > 0 && total < 2u * (uint32_t)nbx) {
-    F = min((kSplitTarget * (uint32_t)nbx + total - 1u) / total, kSplitMax);
-    F = min(F, a.split_slots / ngroups / total);
-    if (F < 1) F = 1;
-  }
-  const uint32_t njobs = total * F;
-  if (blockIdx.x == 0 && tid == 0) a.tile_queue[8] = F;   // for the combine kernel
   const uint32_t gslot = (uint32_t)xcd * (a.split_slots / ngroups);   // the group's first slot
+  if (tid == 0) {
+    uint32_t ent[5];
+    uint64_t all = 0;
+    for (int u = 0; u < L; ++u) {
+      const uint32_t c = lvt[u].count, f = lvbase[u];
+      ent[u] = c ? a.tile_start[f + c - 1] + a.tile_counts[f + c - 1] - a.tile_start[f] : 0u;
+      all += ent[u];
+    }
+    uint32_t target = (uint32_t)(all * nbg / (kSplitTarget * (uint32_t)nbx));
+    target = max(target, (uint32_t)a.chunk / 2u);
+    uint32_t slots = 0;
+    for (bool fits = false; !fits; target *= 2u) {   // doubled until the parts fit the slots (at most 32 times)
+      slots = 0;
+      fits = true;
+      uint32_t job = 0;
+      for (int u = L - 1; u >= 0; --u) {
+        const uint32_t c = lvt[u].count;
+        uint32_t F = 1;
+        if (a.split_slots > 0 && c > 0 && target < 0x40000000u) {
+          F = (ent[u] / c + target / 2u) / target;
+          F = F < 1u ? 1u : min(F, kSplitMax);
+        }
+        slot0_l[u] = slots;
+        if (F > 1) slots += nbg * c * F;
+        parts_l[u] = F;
+        job0_l[u] = job;
+        job += nbg * c * F;
+      }
+      job0_l[5] = job;
+      fits = slots <= a.split_slots / ngroups;
+    }
+    if (blockIdx.x == 0)
+      for (int u = 0; u < L; ++u) a.tile_queue[8 + u] = parts_l[u];   // for the combine kernel
+  }
+  __syncthreads();
+  const uint32_t njobs = job0_l[5];
   // part `part` of F of a tile with entries [s0, s0 + c)
-  const auto part_range = [&](uint32_t s0, uint32_t c, uint32_t part, uint32_t &hs, uint32_t &hc) {
+  const auto part_range = [&](uint32_t s0, uint32_t c, uint32_t part, uint32_t F, uint32_t &hs, uint32_t &hc) {
     const uint32_t lo = (uint32_t)((uint64_t)c * part / F), hi = (uint32_t)((uint64_t)c * (part + 1u) / F);
     hs = s0 + lo;
     hc = hi - lo;
@@ -781,27 +815,25 @@ void fda_bwd_tile_kernel(const Args a) {
   const T *go = static_cast<const T *>(a.gout_hm ? a.gout_hm : a.grad_out);
   const bool go_direct = a.gout_hm == nullptr;
 
-  // k -> (level, head, tile), coarse (last) levels first
-  const auto decode = [&](uint32_t k, int &l, uint32_t &bgi, uint32_t &t) {
-    uint32_t rem = k;
-    l = L - 1;
-    for (; l > 0; --l) {
-      const uint32_t nl = nbg * lvt[l].count;
-      if (rem < nl) break;
-      rem -= nl;
-    }
-    bgi = rem / lvt[l].count;
-    t = rem - bgi * lvt[l].count;
+  // job k -> (level, head, tile, part), coarse (last) levels first
+  const auto decode = [&](uint32_t k, int &l, uint32_t &bgi, uint32_t &t, uint32_t &part) {
+    l = 0;
+    while (l + 1 < L && k < job0_l[l]) ++l;
+    const uint32_t rem = k - job0_l[l], F = parts_l[l], q = rem / F;
+    part = rem - q * F;
+    bgi = q / lvt[l].count;
+    t = q - bgi * lvt[l].count;
   };
   const auto head_of = [&](uint32_t bgi, int &b, int &g) {
     b = (int)(bgi / (uint32_t)hpx);
     g = a.tile_affinity ? xcd + 8 * (int)(bgi % (uint32_t)hpx) : (int)(bgi % (uint32_t)hpx);
   };
-  const auto tile_gid = [&](uint32_t k) {
+  const auto job_tile = [&](uint32_t k, uint32_t &part, uint32_t &F) {   // the job's tile id, its part
     int l, b, g;
     uint32_t bgi, t;
-    decode(k, l, bgi, t);
+    decode(k, l, bgi, t, part);
     head_of(bgi, b, g);
+    F = parts_l[l];
     return (uint32_t)(b * G + g) * T_h + lvbase[l] + t;
   };
   // Tiles: the block's first four are bi + j nbx (j < 4); after them each block takes the next
@@ -823,23 +855,23 @@ void fda_bwd_tile_kernel(const Args a) {
     k2 = 2u * (uint32_t)nbx + (uint32_t)bi;
   }
   // header of k2 (thread 0: the tile's first entry and count, and k2's part), not yet in the ring
-  uint32_t hs_pend = 0, hc_pend = 0, hp_pend = 0;
+  uint32_t hs_pend = 0, hc_pend = 0, hp_pend = 0, hf_pend = 1;
   if (tid == 0) {
     const uint32_t kk[2] = {(uint32_t)bi, k1};
     for (int i = 0; i < 2; ++i) {
       uint32_t hs = 0u, hc = 0u;
       if (kk[i] < njobs) {
-        const uint32_t gid = tile_gid(kk[i] / F);
-        part_range(a.tile_start[gid], a.tile_counts[gid], kk[i] % F, hs, hc);
+        uint32_t part, F;
+        const uint32_t gid = job_tile(kk[i], part, F);
+        part_range(a.tile_start[gid], a.tile_counts[gid], part, F, hs, hc);
       }
       hdr_l[i][0] = hs;
       hdr_l[i][1] = hc;
     }
     if (k2 < njobs) {
-      const uint32_t gid = tile_gid(k2 / F);
+      const uint32_t gid = job_tile(k2, hp_pend, hf_pend);
       hs_pend = a.tile_start[gid];
       hc_pend = a.tile_counts[gid];
-      hp_pend = k2 % F;
     }
   }
   for (int i = tid; i < NBX; i += NT) cur_l[i] = 0u;   // bin counters of the first chunk
@@ -862,11 +894,11 @@ void fda_bwd_tile_kernel(const Args a) {
     // wave waits for the atomic), and the block reads it at the end of the next job
     const bool claimed = use_queue && k2 < njobs;
     if (claimed && tid == 0) taken = atomicAdd(a.tile_queue + xcd, 1u);
-    const uint32_t ktile = k / F, part = k - ktile * F;
     int l, b, g;
-    uint32_t bgi, t;
-    decode(ktile, l, bgi, t);
+    uint32_t bgi, t, part;
+    decode(k, l, bgi, t, part);
     head_of(bgi, b, g);
+    const uint32_t F = parts_l[l];
     const uint32_t row0 = ((uint32_t)b * (uint32_t)G + (uint32_t)g) * (uint32_t)a.Q;   // the head's first sample row
     const LevelTiles lt = lvt[l];
     const int itx = (int)(t % (uint32_t)lt.nt[2]);
@@ -1036,7 +1068,7 @@ void fda_bwd_tile_kernel(const Args a) {
       if (tid == 0) {
         grab_l[pos & 3u] = claimed ? taken : ~0u;
         uint32_t hs, hc;
-        part_range(hs_pend, hc_pend, hp_pend, hs, hc);
+        part_range(hs_pend, hc_pend, hp_pend, hf_pend, hs, hc);
         hdr_l[(pos + 2u) & 3u][0] = hs;
         hdr_l[(pos + 2u) & 3u][1] = hc;
       }
@@ -1046,7 +1078,7 @@ void fda_bwd_tile_kernel(const Args a) {
       // this part's sums go to its scratch slot (voxels of the nominal tile: pair p, x-half h);
       // fda_bwd_split_combine_kernel adds a tile's parts and writes its rows
       constexpr int kTileVox = 2 * (NT / LPU);
-      float *sl = a.split_scratch + ((size_t)(gslot + ktile * F + part) * kTileVox + (size_t)p * 2u) * (uint32_t)D +
+      float *sl = a.split_scratch + ((size_t)(gslot + slot0_l[l] + (k - job0_l[l])) * kTileVox + (size_t)p * 2u) * (uint32_t)D +
                   (uint32_t)(j * CPL);
       if (live) {
         store_elems<float, CPL>(sl, acc0);
@@ -1077,7 +1109,7 @@ void fda_bwd_tile_kernel(const Args a) {
       if (tid == 0) {
         grab_l[pos & 3u] = claimed ? taken : ~0u;
         uint32_t hs, hc;
-        part_range(hs_pend, hc_pend, hp_pend, hs, hc);
+        part_range(hs_pend, hc_pend, hp_pend, hf_pend, hs, hc);
         hdr_l[(pos + 2u) & 3u][0] = hs;
         hdr_l[(pos + 2u) & 3u][1] = hc;
       }
@@ -1098,43 +1130,43 @@ void fda_bwd_tile_kernel(const Args a) {
       if (k3 >= njobs) k3 = njobs;
     }
     if (tid == 0 && k3 < njobs) {
-      const uint32_t gid = tile_gid(k3 / F);
+      const uint32_t gid = job_tile(k3, hp_pend, hf_pend);
       hs_pend = a.tile_start[gid];
       hc_pend = a.tile_counts[gid];
-      hp_pend = k3 % F;
     }
     k = k1; k1 = k2; k2 = k3;
     ++pos;
   }
 }
 
-// Split tiles (see the tile kernel): one block per tile of every group adds the F parts'
+// Split tiles (see the tile kernel): one block per split tile of every group adds the F parts'
 // partial sums of each of its voxels and writes the rows (in T, or added to the caller's fp32
-// buffer).  Runs after the tile kernel, so plain loads see the parts; exits when F == 1.
+// buffer).  Runs after the tile kernel, so plain loads see the parts; exits when nothing is split.
 template <typename T, int CPL, int LPU, bool BIG>
 __global__ __launch_bounds__(tile_threads(LPU, BIG)) void fda_bwd_split_combine_kernel(const Args a) {
   constexpr int NT = tile_threads(LPU, BIG);
   constexpr int kTileVox = 2 * (NT / LPU);
-  const uint32_t F = a.tile_queue[8];
-  if (F <= 1) return;
   const int tid = threadIdx.x, D = a.D, G = a.G, L = a.L;
   const int p = tid / LPU, j = tid & (LPU - 1);
   const int hxn = a.TX / 2;
   const int px = p % hxn, py = (p / hxn) % a.TY, pz = p / (hxn * a.TY);
-  const uint32_t T_h = tiles_per_head(a.shapes, L, a.TX, a.TY, a.TZ);
   const uint32_t ngroups = a.tile_affinity ? 8u : 1u;
   const int hpx = a.tile_affinity ? G / 8 : G;
-  const uint32_t nbg = (uint32_t)a.B * (uint32_t)hpx, total = nbg * T_h;
-  const uint32_t xcd = blockIdx.x % ngroups, k = blockIdx.x / ngroups;   // tile k of group xcd
-  if (k >= total) return;
-  // k -> (level, head, tile) as in the tile kernel: coarse (last) levels first
-  uint32_t rem = k;
+  const uint32_t nbg = (uint32_t)a.B * (uint32_t)hpx;
+  const uint32_t xcd = blockIdx.x % ngroups, k = blockIdx.x / ngroups;   // split tile k of group xcd
+  // k -> (level, head, tile) and its first slot, as in the tile kernel: coarse (last) levels first
+  uint32_t rem = k, F = 1, slot = 0;
   int l = L - 1;
-  for (; l > 0; --l) {
+  for (; l >= 0; --l) {
+    F = a.tile_queue[8 + l];
+    if (F <= 1) continue;
     const uint32_t nl = nbg * level_tiles(a.shapes, l, a.TX, a.TY, a.TZ).count;
     if (rem < nl) break;
     rem -= nl;
+    slot += nl * F;
   }
+  if (l < 0) return;
+  slot += rem * F;
   const LevelTiles lt = level_tiles(a.shapes, l, a.TX, a.TY, a.TZ);
   const uint32_t bgi = rem / lt.count, t = rem - bgi * lt.count;
   const int b = (int)(bgi / (uint32_t)hpx);
@@ -1147,11 +1179,12 @@ __global__ __launch_bounds__(tile_threads(LPU, BIG)) void fda_bwd_split_combine_
   if (!live) return;
   const bool two = 2 * px + 1 < lt.t[2] && x0 + 1 < lt.n[2];
   const uint32_t gslot = xcd * (a.split_slots / ngroups);
-  const float *sl = a.split_scratch + ((size_t)(gslot + k * F) * kTileVox + (size_t)p * 2u) * (uint32_t)D +
+  const float *sl = a.split_scratch + ((size_t)(gslot + slot) * kTileVox + (size_t)p * 2u) * (uint32_t)D +
                     (uint32_t)(j * CPL);
   float acc0[CPL], acc1[CPL];
 #pragma unroll
   for (int c = 0; c < CPL; ++c) acc0[c] = acc1[c] = 0.f;
+#pragma unroll 4
   for (uint32_t q = 0; q < F; ++q) {
     float o0[CPL], o1[CPL];
     const float *sq = sl + (size_t)q * kTileVox * D;

@@ -18,7 +18,7 @@
 // the per-axis weight sums times the value, fewer loads than 8 corners per sample; larger sample
 // grids take the reference's per-sample loop.  Backward: the adjoint, as a gather when the
 // output has at most 64 bins per axis and 384 in all (each voxel sums, in registers, the rois
-// that reach it, in roi order: no atomics, the same bits on every run; the workspace holds the
+// that reach it, in an order that they alone decide: no atomics, the same bits on every run; the workspace holds the
 // rois' axis weight tables and a channels-last copy of grad_output),
 // otherwise (or with more than 2^20 channels) by fp32 atomics into a channels-last workspace (64 lanes = 64 contiguous channels
 // per atomic instruction) transposed into grad_input afterwards.  A roi whose batch index is
@@ -497,8 +497,8 @@ __global__ __launch_bounds__(64 * kBwdWaves) void roi_align3d_backward_kernel(co
 // WZ[pd][z] is the sum of bin pd's z-sample tap weights on z (and so on) -- the sum over the bin's
 // samples of their corner weights, separable because the samples form a full grid.  A wave owns a
 // tile of 4 x 4 x 4 voxels and 64 channels, a lane per channel, its 64 sums in registers, and adds
-// up the rois whose footprint reaches the tile in index order, so the result is the same on every
-// run.  With channels on the lanes everything but top is uniform over the wave: weights, bin
+// up the rois whose footprint reaches the tile in a fixed order (index order, except that of every
+// 192 the few with small bins come last), so the result is the same on every run.  With channels on the lanes everything but top is uniform over the wave: weights, bin
 // ranges and loop bounds sit in scalar registers, no lane diverges and nothing is staged in LDS,
 // and the sum is taken axis by axis -- over pw into 4 x positions, over ph into 4 x 4, over pd into
 // the 64 voxels -- about 5 multiply-adds per voxel and roi instead of one per bin combination.

@@ -113,6 +113,29 @@ def test_workspace_bytes(lib):
     assert lib.ops3d_fda_backward_workspace_bytes(2, *c2) == want(*c2, 2048, value_copy=False)
 
 
+def test_split_scratch_rule(lib):
+    """Split scratch beyond 2048 tiles: only from 5 * 2^18 samples on (above the allocation-free
+    entry point's 64 MiB without it), with several levels, when the coarsest is likely small."""
+    f = lib.ops3d_fda_backward_workspace_bytes
+
+    def slots(S, L, Q, dtype=2, B=1, G=8, D=32, K=4):
+        one = f(dtype, B, S, G, D, L, Q, K)
+        esize = 4 if dtype == 0 else 2
+        n = B * Q * G * L * K
+        al = lambda x: (x + 255) // 256 * 256   # noqa: E731
+        fixed = (al(4 * n) + al(16 * n) + al(32 * n) + 3 * al(4 * (B * G * S + 1)) + 256
+                 + al(4 * B * G * 64 * (S // 16 + 64)) + al(B * G * (2 * S + 10) * D * esize)
+                 + (al(B * Q * G * D * esize) if B * Q * G * D * esize > 64 << 20 else 0))
+        return (one - fixed) // (128 * D * 4)
+
+    deep = 40 * 48 * 96 * 585 // 512   # four levels, each half the size of the one before
+    assert slots(deep, 4, deep) == 2048
+    assert slots(deep, 4, 10240) == 2048 and slots(deep, 4, 10239) == 0   # 5 * 2^18 samples
+    assert slots(deep, 1, deep) == 0
+    assert slots(73728, 2, 73728) == 0 and slots(65536, 2, 65536, G=16) == 0
+    assert f(2, 1, deep, 8, 32, 4, 10240, 4) > 64 << 20
+
+
 def _fwd(lib, ptr=None, ws=None, ws_bytes=0, **kw):
     a = dict(dtype=2, B=1, S=576, G=8, D=32, L=2, Q=576, K=4, step=64)
     a.update(kw)

@@ -242,6 +242,19 @@ def test_random_configs(gpu_device, seed):
            im2col_step=B)
 
 
+# --- coarse levels whose tiles are split ------------------------------------------------------
+@pytest.mark.parametrize("shapes,B,Q,G,D,K,dt", [
+    ([(12, 14, 30), (2, 2, 4)], 1, 600, 8, 32, 4, torch.float32),               # one heavy tile per head
+    ([(11, 27, 45), (6, 14, 23), (3, 7, 12)], 2, 700, 6, 48, 4, torch.float32),  # no XCD groups, 12 heads
+    ([(7, 9, 20), (4, 5, 10), (2, 3, 5), (1, 2, 3), (1, 1, 1)], 1, 3000, 8, 16, 2, torch.bfloat16),   # all levels
+    ([(1, 1, 1), (16, 16, 24)], 1, 2500, 3, 64, 8, torch.float16),               # the first level is the small one
+    ([(24, 32, 48), (12, 16, 24), (2, 3, 4)], 1, 14000, 8, 32, 4, torch.bfloat16),   # over 2048 tiles (scratch rule)
+])
+def test_split_coarse_levels(gpu_device, shapes, B, Q, G, D, K, dt):
+    inp = random_inputs(shapes, B, Q, G, D, K, dt, seed=Q, lo=-0.05, hi=1.05)
+    _check(f"split {shapes} B={B} Q={Q} G={G} D={D}", inp, gpu_device, dt)
+
+
 # --- head widths, head counts (XCD mappings), dtypes ---------------------------------------
 @pytest.mark.parametrize("D", [8, 16, 24, 32, 48, 64, 96, 128])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])

@@ -556,7 +556,9 @@ class _NativeFDA:
         B, Din, Hin, Win, _ = value.shape
         geo = [int(v) for v in (kd, kh, kw, sd, sh, sw, pd, ph, pw, dd, dh, dw)]
         grad_value = torch.empty_like(value)
-        grad_offset = torch.zeros_like(p_offset)
+        # every unit's record is written; only a row padding has to be cleared
+        used = group * 4 * (kd * kh * kw - (1 if remove_center else 0))
+        grad_offset = torch.empty_like(p_offset) if p_offset.shape[4] == used else torch.zeros_like(p_offset)
         wsb = self._lib.ops3d_dcnv4_workspace_bytes(code, B, Din, Hin, Win, group, group_channels, *geo,
                                                    int(remove_center), 1)
         ws = torch.empty(max(wsb, 256), dtype=torch.uint8, device=value.device)

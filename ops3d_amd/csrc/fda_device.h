@@ -375,12 +375,12 @@ __device__ __forceinline__ void add_ref_grad(const Args &a, int64_t bq, int j, c
 // and DCNv4-3D (Args::dcn).
 constexpr int kModePlain = 0, kModeOffsets = 1, kModeDcn = 2;
 
-// Element offset of unit (b*Q + q)*G + g's record in loc_attn / grad_loc_attn: P per unit, or
-// (DCNv4-3D) rows of rec_stride per (b, q).
+// Element offset of the record of head g of query bq = b*Q + q in loc_attn / grad_loc_attn: P per
+// unit bq*G + g, or (DCNv4-3D) rows of rec_stride per query.
 template <int MODE>
-__device__ __forceinline__ int64_t record_offset(const Args &a, int64_t unit) {
-  if constexpr (MODE == kModeDcn) return (unit / a.G) * a.rec_stride + (unit % a.G) * a.P;
-  return unit * a.P;
+__device__ __forceinline__ int64_t record_offset(const Args &a, int64_t bq, int g) {
+  if constexpr (MODE == kModeDcn) return bq * a.rec_stride + g * a.P;
+  return (bq * a.G + g) * a.P;
 }
 
 // DCNv4-3D mode: turn the staged offsets of unit (b, q) into pixel coordinates of the input
@@ -393,16 +393,22 @@ template <int LPU>
 __device__ __forceinline__ void dcn_to_pixels(const Args &a, int q, int j, float *rec) {
 #pragma clang fp contract(off)
   const int K = a.K;
-  const int xo = q % a.Wout, yo = (q / a.Wout) % a.Hout, zo = q / (a.Wout * a.Hout);
+  const uint32_t zy = (uint32_t)q / (uint32_t)a.Wout, zu = zy / (uint32_t)a.Hout;
+  const int xo = (int)((uint32_t)q - zy * (uint32_t)a.Wout), yo = (int)(zy - zu * (uint32_t)a.Hout), zo = (int)zu;
   const int hw = (a.dlw * (a.kw - 1)) >> 1, hh = (a.dlh * (a.kh - 1)) >> 1, hd = (a.dld * (a.kd - 1)) >> 1;
   const float s = a.offset_scale;
   const float p0w = (float)(hw - a.pw + xo * a.sw) - (float)hw * s;
   const float p0h = (float)(hh - a.ph + yo * a.sh) - (float)hh * s;
   const float p0d = (float)(hd - a.pd + zo * a.sd) - (float)hd * s;
   const int centre = ((a.kw / 2) * a.kh + a.kh / 2) * a.kd + a.kd / 2;
+  // tap / n by the reciprocal, exact for the at most 129 taps: tap + 1/2 lies at least 1 / (2 n)
+  // from a multiple of n (an integer division by a run-time n is about 20 instructions)
+  const int hd_taps = a.kh * a.kd;
+  const float r_hd = 1.f / (float)hd_taps, r_d = 1.f / (float)a.kd;
   for (int t = j; t < K; t += LPU) {
     const int tap = (a.dcn_remove_center && t >= centre) ? t + 1 : t;
-    const int i = tap / (a.kh * a.kd), jj = (tap / a.kd) % a.kh, k = tap % a.kd;
+    const int i = (int)(((float)tap + 0.5f) * r_hd), rest = tap - i * hd_taps;
+    const int jj = (int)(((float)rest + 0.5f) * r_d), k = rest - jj * a.kd;
     rec[3 * t] = p0w + ((float)(i * a.dlw) + rec[3 * t]) * s;
     rec[3 * t + 1] = p0h + ((float)(jj * a.dlh) + rec[3 * t + 1]) * s;
     rec[3 * t + 2] = p0d + ((float)(k * a.dld) + rec[3 * t + 2]) * s;
@@ -561,13 +567,6 @@ __device__ inline int64_t copy_head_rows(const int64_t *shapes, const int64_t *l
   return S + extra;
 }
 
-// Element offset, in a paired level, of the row a pair lane loads: `o` is the corner's element
-// offset in the plain layout (row * RST, or OOB_ELEM), dxl the lane's x-row of the pair.  Row r
-// is read through line r - dxl: copy row 2(r - dxl + 1) + dxl.
-__device__ __forceinline__ uint32_t paired_offset(uint32_t o, int dxl, int RST) {
-  return o == OOB_ELEM ? OOB_ELEM : 2u * o + (uint32_t)((2 - dxl) * RST);
-}
-
 // Compile-time loop: f(IntConst<0>{}), ..., f(IntConst<N-1>{}).
 template <int V> struct IntConst { static constexpr int value = V; };
 template <int N, typename F>
@@ -637,6 +636,71 @@ __device__ __forceinline__ bool sample_setup(float lx, float ly, float lz, int W
   const bool in = sample_base(lx, ly, lz, Wl, Hl, Dl, sb, pix);
   sample_expand(sb, Wl, Hl, Dl, GD, sm);
   return in;
+}
+
+// A sample as one x-row of the pair kernels needs it: the lane's four corners c4 = (dz, dy) of row
+// x0 + dxl.  Byte offsets of the rows inside the level (OOB_BYTE for a corner outside the volume),
+// the row's x weight and both y and z weights, with sample_base's rules and roundings; about half
+// the instructions of the eight corners of sample_setup, of which the kernels used four.
+constexpr uint32_t OOB_BYTE = 0x80000000u;   // beyond every buffer, also after a lane's part is added
+struct PairSample {
+  uint32_t off[4];
+  float wxd, wy[2], wz[2], fx;   // fx: x weight of row x0 + 1 (the fraction)
+  int x0, y0, z0;                // base corner (unspecified when outside)
+};
+// Level geometry of the pair kernels in bytes: step of x, y and z, and of the pair's second row.
+// In a paired level row r is read through line r - dxl: copy row 2 (r - dxl + 1) + dxl.
+struct PairLevel {
+  uint32_t sx, sy, sz, first;    // `first`: byte offset of voxel 0's row for this lane's dxl
+};
+__device__ __forceinline__ PairLevel pair_level(int Wl, int Hl, uint32_t row_bytes, bool paired, int dxl) {
+  PairLevel p;
+  p.sx = paired ? 2u * row_bytes : row_bytes;
+  p.sy = (uint32_t)Wl * p.sx;
+  p.sz = (uint32_t)Hl * p.sy;
+  p.first = (paired ? 2u + (uint32_t)dxl : (uint32_t)dxl) * row_bytes;
+  return p;
+}
+__device__ __forceinline__ bool pair_setup(float lx, float ly, float lz, int Wl, int Hl, int Dl, const PairLevel &pl,
+                                           int dxl, bool live, PairSample &ps, bool pix) {
+  const float x = pix ? lx : pixel_coord(lx, (float)Wl);
+  const float y = pix ? ly : pixel_coord(ly, (float)Hl);
+  const float z = pix ? lz : pixel_coord(lz, (float)Dl);
+  const bool in = (pix ? (x > -1.f && y > -1.f && z > -1.f) : (x >= -1.f && y >= -1.f && z >= -1.f)) &&
+                  x < (float)Wl && y < (float)Hl && z < (float)Dl && live;
+  const float xf = floorf(x), yf = floorf(y), zf = floorf(z);
+  ps.x0 = (int)xf;
+  ps.y0 = (int)yf;
+  ps.z0 = (int)zf;
+  ps.fx = in ? x - xf : 0.f;
+  const float gx = in ? (xf + 1.f) - x : 0.f;
+  ps.wxd = dxl ? ps.fx : gx;
+  ps.wy[1] = in ? y - yf : 0.f;
+  ps.wy[0] = in ? (yf + 1.f) - y : 0.f;
+  ps.wz[1] = in ? z - zf : 0.f;
+  ps.wz[0] = in ? (zf + 1.f) - z : 0.f;
+  const uint32_t o = (uint32_t)ps.z0 * pl.sz + (uint32_t)ps.y0 * pl.sy + (uint32_t)ps.x0 * pl.sx + pl.first;
+  const int xr = ps.x0 + dxl;
+  const bool vx = in && xr >= 0 && xr < Wl;
+  const bool vy0 = ps.y0 >= 0, vy1 = ps.y0 + 1 < Hl, vz0 = vx && ps.z0 >= 0, vz1 = vx && ps.z0 + 1 < Dl;
+  ps.off[0] = vz0 && vy0 ? o : OOB_BYTE;
+  ps.off[1] = vz0 && vy1 ? o + pl.sy : OOB_BYTE;
+  ps.off[2] = vz1 && vy0 ? o + pl.sz : OOB_BYTE;
+  ps.off[3] = vz1 && vy1 ? o + pl.sz + pl.sy : OOB_BYTE;
+  return in;
+}
+
+// Lane k of every quad gets the quad's sum of v[k] (a transposing reduction: 6 selects and 3 adds).
+__device__ __forceinline__ float quad_sum_own(const float v[4], int lane) {
+  const bool k1 = lane & 1, k2 = lane & 2;
+  const float a = (k1 ? v[1] : v[0]) + xor_lane<1>(k1 ? v[0] : v[1]);
+  const float b = (k1 ? v[3] : v[2]) + xor_lane<1>(k1 ? v[2] : v[3]);
+  return (k2 ? b : a) + xor_lane<2>(k2 ? a : b);
+}
+
+// v plus the value four lanes up (for lanes 0..3 of every 8).
+__device__ __forceinline__ float add_upper_quad(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x104, 0xF, 0xF, true));   // row_shl:4
 }
 
 // Value of lane u of this lane's unit (units are LPU consecutive lanes; u < min(LPU, 4)).

@@ -24,9 +24,11 @@
 namespace ops3d_fda {
 
 constexpr int kFwdWavesPerEU = 8;     // minimum waves per SIMD the x-pair forward is compiled for
-// Backward query pair kernel: left to itself the compiler takes 107 VGPRs (4 waves per SIMD);
-// 5 waves fit without spills.
-constexpr int kQueryWavesPerEU = 5;
+// Waves per SIMD the backward query pair kernel is compiled for.  4 or 5, bf16, 8 heads of 32
+// channels: two levels of 73728 voxels 188 / 177 us; paired levels, whose misses more waves only
+// add to, three levels of 598016 voxels 3028 / 3109; DCNv4-3D, whose LDS records leave room for
+// three waves, [2,32,64,64] 3^3 taps 1880 / 1996 (3 as 4).
+constexpr int query_waves(bool pairs, int mode) { return pairs || mode == kModeDcn ? 4 : 5; }
 // Tile splitting (tile kernel): a part aims at 1/kSplitTarget of a block's share of the entries, at
 // most kSplitMax parts per tile.  Tile kernel with target 2 / 3 / 4: levels 40x48x96 to 5x6x12
 // 1719 / 1484 / 1340 us (bf16, 8 heads; unsplit 7137), 44x56x134 to 11x14x34 2010 / 1902 / 1916
@@ -96,12 +98,12 @@ __global__ __launch_bounds__(kBlock) void fda_forward_kernel(const Args a) {
   const bool live = q < a.Q;
   const int L = a.L, K = a.K, LK = L * K, P = a.P;
   float *rec = lds + ub * (P + 1);
-  const int64_t unit = ((int64_t)b * a.Q + (live ? q : 0)) * a.G + g;
+  const int64_t bq = (int64_t)b * a.Q + (live ? q : 0), unit = bq * a.G + g;
 
-  stage_record<T, LPU>(static_cast<const T *>(a.loc_attn) + record_offset<MODE>(a, unit), P, j, live, rec);
+  stage_record<T, LPU>(static_cast<const T *>(a.loc_attn) + record_offset<MODE>(a, bq, g), P, j, live, rec);
   wave_lds_sync();
   if constexpr (MODE == kModeOffsets) {
-    offsets_to_locations<T, LPU>(a, unit / a.G, j, live, rec);
+    offsets_to_locations<T, LPU>(a, bq, j, live, rec);
     wave_lds_sync();
   }
   if constexpr (MODE == kModeDcn) {
@@ -200,12 +202,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWave
   const bool live = q < a.Q;
   const int L = a.L, K = a.K, LK = L * K, P = a.P;
   float *rec = lds + ub * (P + 1);
-  const int64_t unit = ((int64_t)b * a.Q + (live ? q : 0)) * a.G + g;
+  const int64_t bq = (int64_t)b * a.Q + (live ? q : 0), unit = bq * a.G + g;
 
-  stage_record<T, UL>(static_cast<const T *>(a.loc_attn) + record_offset<MODE>(a, unit), P, ju, live, rec);
+  stage_record<T, UL>(static_cast<const T *>(a.loc_attn) + record_offset<MODE>(a, bq, g), P, ju, live, rec);
   wave_lds_sync();
   if constexpr (MODE == kModeOffsets) {
-    offsets_to_locations<T, UL>(a, unit / a.G, ju, live, rec);
+    offsets_to_locations<T, UL>(a, bq, ju, live, rec);
     wave_lds_sync();
   }
   if constexpr (MODE == kModeDcn) {
@@ -220,7 +222,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWave
   for (int c = 0; c < CPL; ++c) acc[c] = 0.f;
 
   const int RST = a.vhm ? a.D : a.G * a.D;
-  const uint32_t lane_elem = (uint32_t)((a.vhm ? 0 : g * a.D) + j * CPL);
+  const uint32_t lane_byte = (uint32_t)((a.vhm ? 0 : g * a.D) + j * CPL) * (uint32_t)sizeof(T);
   constexpr int kRowBytes = CPL * 4 * (int)sizeof(T);   // 64
   const T *vb = static_cast<const T *>(a.value) +
                 (a.vhm ? ((int64_t)b * a.G + g) * (kPairs ? copy_head_rows(a.shapes, a.lsi, L, a.S, kRowBytes) : a.S) * a.D
@@ -232,24 +234,20 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWave
     const int64_t rows = cl.paired ? 2 * (int64_t)Dl * Hl * Wl + 2 : (int64_t)Dl * Hl * Wl;
     const uint32_t nbytes = (uint32_t)(rows * RST * (int64_t)sizeof(T));
     const __amdgpu_buffer_rsrc_t rv = make_rsrc(vb + cl.start * RST, nbytes);
+    const PairLevel pl = pair_level(Wl, Hl, (uint32_t)(RST * (int)sizeof(T)), cl.paired, dxl);
     // 4 samples per step: lane (ju & 3) of each quad sets up sample k0 + (ju & 3) for its own
     // x-row (4 corner offsets and weights); its quad receives them by DPP broadcast
     for (int k0 = 0; k0 < K; k0 += 4) {
       const int kj = k0 + (ju & 3);
       const int sj = l * K + (kj < K ? kj : K - 1);
-      Sample ms;
-      sample_setup(rec[3 * sj], rec[3 * sj + 1], rec[3 * sj + 2], Wl, Hl, Dl, RST, ms, MODE == kModeDcn);
-      uint32_t off4[4];
+      PairSample ms;
+      pair_setup(rec[3 * sj], rec[3 * sj + 1], rec[3 * sj + 2], Wl, Hl, Dl, pl, dxl, live, ms, MODE == kModeDcn);
       float w4[4];
       // corner weights times the sample's attention weight (made once per set-up, not per channel)
       const float at_s = rec[3 * LK + sj];
-      const float wxd = dxl ? ms.wx[1] : ms.wx[0];
 #pragma unroll
-      for (int c4 = 0; c4 < 4; ++c4) {   // c4 = (dz, dy); this lane's corner c = 2*c4 + dxl
-        off4[c4] = live ? (dxl ? ms.off[2 * c4 + 1] : ms.off[2 * c4]) : OOB_ELEM;
-        if (cl.paired) off4[c4] = paired_offset(off4[c4], dxl, RST);
-        w4[c4] = ((wxd * ms.wy[c4 & 1]) * ms.wz[c4 >> 1]) * at_s;
-      }
+      for (int c4 = 0; c4 < 4; ++c4)   // c4 = (dz, dy)
+        w4[c4] = ((ms.wxd * ms.wy[c4 & 1]) * ms.wz[c4 >> 1]) * at_s;
       static_for<4>([&](auto uc) {
         constexpr int u = decltype(uc)::value;
         if (k0 + u < K) {
@@ -257,13 +255,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWave
           float w[4];
 #pragma unroll
           for (int c4 = 0; c4 < 4; ++c4) {
-            off[c4] = unit_bcast<4, u>(off4[c4]);
+            off[c4] = unit_bcast<4, u>(ms.off[c4]) + lane_byte;
             w[c4] = __uint_as_float(unit_bcast<4, u>(__float_as_uint(w4[c4])));
           }
           uint32_t v[4][NW];
 #pragma unroll
           for (int c4 = 0; c4 < 4; ++c4)
-            bload<NW * 4>(rv, (off[c4] + lane_elem) * (uint32_t)sizeof(T), v[c4]);
+            bload<NW * 4>(rv, off[c4], v[c4]);
 #pragma unroll
           for (int i = 0; i < NW; ++i) {
 #pragma unroll
@@ -290,7 +288,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWave
 // the lane that made a set-up also records that sample's stash and base corner.  The partials
 // of grad_loc / grad_attn of a lane's x-row are summed over the unit's 8 lanes.
 template <typename T, int CPL, bool kPairs, int MODE>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQueryWavesPerEU))) void fda_bwd_query_pair_kernel(const Args a) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(query_waves(kPairs, MODE)))) void fda_bwd_query_pair_kernel(const Args a) {
   extern __shared__ float lds[];
   constexpr int UL = 8;
   constexpr int UPW = kWave / UL, UPB = kWavesPerBlock * UPW;
@@ -311,7 +309,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQueryWa
   float4 *st_s = reinterpret_cast<float4 *>(lds + ub * RS + ((P + LK + 3) & ~3));
   uint32_t *cx_s = reinterpret_cast<uint32_t *>(st_s + LK);
   uint32_t *cy_s = cx_s + LK, *cz_s = cy_s + LK;
-  const int64_t unit = ((int64_t)b * a.Q + (live ? q : 0)) * a.G + g;
+  const int64_t bq = (int64_t)b * a.Q + (live ? q : 0), unit = bq * a.G + g;
   __shared__ LevelTiles lvt[5];
   __shared__ uint32_t lvbase[5];
   __shared__ CopyLevel lvcopy[5];   // each level's place in the value rows read (copy_level)
@@ -327,10 +325,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQueryWa
   }
   __syncthreads();
 
-  stage_record<T, UL>(static_cast<const T *>(a.loc_attn) + record_offset<MODE>(a, unit), P, ju, live, rec);
+  stage_record<T, UL>(static_cast<const T *>(a.loc_attn) + record_offset<MODE>(a, bq, g), P, ju, live, rec);
   wave_lds_sync();
   if constexpr (MODE == kModeOffsets) {
-    offsets_to_locations<T, UL>(a, unit / a.G, ju, live, rec);
+    offsets_to_locations<T, UL>(a, bq, ju, live, rec);
     wave_lds_sync();
   }
   if constexpr (MODE == kModeDcn) {
@@ -356,7 +354,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQueryWa
   }
 
   const int RST = a.vhm ? a.D : a.G * a.D;
-  const uint32_t lane_elem = (uint32_t)((a.vhm ? 0 : g * a.D) + j * CPL);
+  const uint32_t lane_byte = (uint32_t)((a.vhm ? 0 : g * a.D) + j * CPL) * (uint32_t)sizeof(T);
   const T *vb = static_cast<const T *>(a.value) +
                 (a.vhm ? ((int64_t)b * a.G + g) * (kPairs ? uniform_i64(head_rows) : (int64_t)a.S) * a.D
                        : (int64_t)b * a.S * a.G * a.D);
@@ -367,74 +365,59 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQueryWa
                                 : CopyLevel{a.lsi[l], false};
     const int64_t rows = cl.paired ? 2 * (int64_t)Dl * Hl * Wl + 2 : (int64_t)Dl * Hl * Wl;
     const __amdgpu_buffer_rsrc_t rv = make_rsrc(vb + cl.start * RST, (uint32_t)(rows * RST * (int64_t)sizeof(T)));
+    const PairLevel pl = pair_level(Wl, Hl, (uint32_t)(RST * (int)sizeof(T)), cl.paired, dxl);
     for (int k0 = 0; k0 < K; k0 += 4) {
       // lane k of each quad sets up sample k0 + k (both quads: each needs its own x-row)
       const int kq = k0 + (ju & 3);
       const bool have = kq < K;
       const int sj = l * K + (have ? kq : K - 1);
-      Sample ms;
-      const bool in_s = sample_setup(rec[3 * sj], rec[3 * sj + 1], rec[3 * sj + 2], Wl, Hl, Dl, RST, ms, MODE == kModeDcn) && live;
+      PairSample ms;
+      const bool in_s =
+          pair_setup(rec[3 * sj], rec[3 * sj + 1], rec[3 * sj + 2], Wl, Hl, Dl, pl, dxl, live, ms, MODE == kModeDcn);
+      const float at = rec[3 * LK + sj];
       if (dxl == 0 && have) {
         cx_s[sj] = in_s ? (uint32_t)(ms.x0 + 1) : kKeyInvalid;
         cy_s[sj] = (uint32_t)(ms.y0 + 1);
         cz_s[sj] = (uint32_t)(ms.z0 + 1);
-        st_s[sj] = make_float4(ms.wx[1], ms.wy[1], ms.wz[1], rec[3 * LK + sj]);
+        st_s[sj] = make_float4(ms.fx, ms.wy[1], ms.wz[1], at);
       }
-      uint32_t off4[4];
-#pragma unroll
-      for (int c4 = 0; c4 < 4; ++c4) {   // c4 = (dz, dy); a select, not an index, keeps ms in registers
-        off4[c4] = live ? (dxl ? ms.off[2 * c4 + 1] : ms.off[2 * c4]) : OOB_ELEM;
-        if (cl.paired) off4[c4] = paired_offset(off4[c4], dxl, RST);
-      }
-      const float wv[6] = {ms.wx[0], ms.wx[1], ms.wy[0], ms.wy[1], ms.wz[0], ms.wz[1]};
-      // all four set-ups are computed (past K they repeat sample K-1), so U and W stay in
-      // registers; only the write-back below skips them
+      // U[u][c4] = grad_output . row c4 of sample k0 + u, this lane's channels (all four set-ups are
+      // used: past K they repeat sample K - 1, so U stays in registers)
       float U[4][4];
       static_for<4>([&](auto uc) {
         constexpr int u = decltype(uc)::value;
 #pragma unroll
-        for (int c4 = 0; c4 < 4; ++c4) {
-          const uint32_t o = unit_bcast<4, u>(off4[c4]);
-          U[u][c4] = dot_elems<T, CPL>(rv, (o + lane_elem) * (uint32_t)sizeof(T), tgw);
-        }
+        for (int c4 = 0; c4 < 4; ++c4)
+          U[u][c4] = dot_elems<T, CPL>(rv, unit_bcast<4, u>(ms.off[c4]) + lane_byte, tgw);
       });
-      static_for<4>([&](auto uc) {
-        constexpr int u = decltype(uc)::value;
-        if (k0 + u < K) {
-          float W[6];   // (wx0, wx1, wy0, wy1, wz0, wz1) of sample k0 + u
+      // summed over the row's channels: lane k of a quad gets its own sample's four sums, so the
+      // chain rule below runs once per sample, on the lane that holds its weights
+      float R[4];
 #pragma unroll
-          for (int i = 0; i < 6; ++i) W[i] = __uint_as_float(unit_bcast<4, u>(__float_as_uint(wv[i])));
-          const float wxd = dxl ? W[1] : W[0];
-          const float sx = dxl ? 1.f : -1.f;
-          float gx = 0.f, gy = 0.f, gz = 0.f, ga = 0.f;
+      for (int c4 = 0; c4 < 4; ++c4) {
+        const float v[4] = {U[0][c4], U[1][c4], U[2][c4], U[3][c4]};
+        R[c4] = quad_sum_own(v, ju);
+      }
+      // d w / dx = (dxl ? +1 : -1) * wy * wz, d w / dy = (dy ? +1 : -1) * wx * wz, and so on
+      float s = 0.f;
 #pragma unroll
-          for (int c4 = 0; c4 < 4; ++c4) {
-            const int dz = c4 >> 1, dy = c4 & 1;
-            const float yz = W[2 + dy] * W[4 + dz];
-            ga = fmaf(wxd * yz, U[u][c4], ga);
-            gx = fmaf(sx * yz, U[u][c4], gx);
-          }
-          // d w / dy = (dy ? +1 : -1) * wx * wz, d w / dz = (dz ? +1 : -1) * wx * wy
-#pragma unroll
-          for (int dz = 0; dz < 2; ++dz) gy = fmaf(wxd * W[4 + dz], U[u][2 * dz + 1] - U[u][2 * dz], gy);
-#pragma unroll
-          for (int dy = 0; dy < 2; ++dy) gz = fmaf(wxd * W[2 + dy], U[u][2 + dy] - U[u][dy], gz);
-          gx = unit_sum<UL>(gx);
-          gy = unit_sum<UL>(gy);
-          gz = unit_sum<UL>(gz);
-          ga = unit_sum<UL>(ga);
-          if (ju == 0) {
-            const int su = l * K + k0 + u;
-            const float at = rec[3 * LK + su];
-            // d(pixel)/d(loc) = size (grid_sample: size/2 per unit of grid, grid = 2*loc - 1);
-            // offset mode: d(pixel)/d(offset) = 1; DCNv4-3D: d(pixel)/d(offset) = offset_scale
-            rec[3 * su] = gx * at * (MODE == kModeDcn ? a.offset_scale : (MODE == kModeOffsets ? 1.f : (float)Wl));
-            rec[3 * su + 1] = gy * at * (MODE == kModeDcn ? a.offset_scale : (MODE == kModeOffsets ? 1.f : (float)Hl));
-            rec[3 * su + 2] = gz * at * (MODE == kModeDcn ? a.offset_scale : (MODE == kModeOffsets ? 1.f : (float)Dl));
-            gat_s[su] = ga;
-          }
-        }
-      });
+      for (int c4 = 0; c4 < 4; ++c4) s = fmaf(ms.wy[c4 & 1] * ms.wz[c4 >> 1], R[c4], s);
+      float gx = dxl ? s : -s, ga = ms.wxd * s;
+      float gy = ms.wxd * fmaf(ms.wz[1], R[3] - R[2], ms.wz[0] * (R[1] - R[0]));
+      float gz = ms.wxd * fmaf(ms.wy[1], R[3] - R[1], ms.wy[0] * (R[2] - R[0]));
+      // both x-rows, on the lower quad
+      gx = add_upper_quad(gx);
+      gy = add_upper_quad(gy);
+      gz = add_upper_quad(gz);
+      ga = add_upper_quad(ga);
+      if (dxl == 0 && have) {
+        // d(pixel)/d(loc) = size (grid_sample: size/2 per unit of grid, grid = 2*loc - 1);
+        // offset mode: d(pixel)/d(offset) = 1; DCNv4-3D: d(pixel)/d(offset) = offset_scale
+        rec[3 * sj] = gx * at * (MODE == kModeDcn ? a.offset_scale : (MODE == kModeOffsets ? 1.f : (float)Wl));
+        rec[3 * sj + 1] = gy * at * (MODE == kModeDcn ? a.offset_scale : (MODE == kModeOffsets ? 1.f : (float)Hl));
+        rec[3 * sj + 2] = gz * at * (MODE == kModeDcn ? a.offset_scale : (MODE == kModeOffsets ? 1.f : (float)Dl));
+        gat_s[sj] = ga;
+      }
     }
   }
   wave_lds_sync();
@@ -479,8 +462,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kQueryWa
   }
   wave_lds_sync();
   if constexpr (MODE == kModeOffsets)
-    if (live && a.grad_ref) add_ref_grad<UL>(a, unit / a.G, ju, rec);
-  if (live) write_record<T, UL>(static_cast<T *>(a.grad_loc_attn) + record_offset<MODE>(a, unit), P, ju, rec);
+    if (live && a.grad_ref) add_ref_grad<UL>(a, bq, ju, rec);
+  if (live) write_record<T, UL>(static_cast<T *>(a.grad_loc_attn) + record_offset<MODE>(a, bq, g), P, ju, rec);
   clear_tile_counts(a);
 }
 
@@ -504,7 +487,7 @@ __global__ __launch_bounds__(kBlock) void fda_bwd_query_kernel(const Args a) {
   float4 *st_s = reinterpret_cast<float4 *>(lds + ub * RS + ((P + LK + 3) & ~3));
   uint32_t *cx_s = reinterpret_cast<uint32_t *>(st_s + LK);
   uint32_t *cy_s = cx_s + LK, *cz_s = cy_s + LK;
-  const int64_t unit = ((int64_t)b * a.Q + (live ? q : 0)) * a.G + g;
+  const int64_t bq = (int64_t)b * a.Q + (live ? q : 0), unit = bq * a.G + g;
   // per level: tile geometry and the id of the level's first tile of this (b, g)
   __shared__ LevelTiles lvt[5];
   __shared__ uint32_t lvbase[5];
@@ -518,10 +501,10 @@ __global__ __launch_bounds__(kBlock) void fda_bwd_query_kernel(const Args a) {
   }
   __syncthreads();
 
-  stage_record<T, LPU>(static_cast<const T *>(a.loc_attn) + record_offset<MODE>(a, unit), P, j, live, rec);
+  stage_record<T, LPU>(static_cast<const T *>(a.loc_attn) + record_offset<MODE>(a, bq, g), P, j, live, rec);
   wave_lds_sync();
   if constexpr (MODE == kModeOffsets) {
-    offsets_to_locations<T, LPU>(a, unit / a.G, j, live, rec);
+    offsets_to_locations<T, LPU>(a, bq, j, live, rec);
     wave_lds_sync();
   }
   if constexpr (MODE == kModeDcn) {
@@ -670,8 +653,8 @@ __global__ __launch_bounds__(kBlock) void fda_bwd_query_kernel(const Args a) {
   }
   wave_lds_sync();
   if constexpr (MODE == kModeOffsets)
-    if (live && a.grad_ref) add_ref_grad<LPU>(a, unit / a.G, j, rec);
-  if (live) write_record<T, LPU>(static_cast<T *>(a.grad_loc_attn) + record_offset<MODE>(a, unit), P, j, rec);
+    if (live && a.grad_ref) add_ref_grad<LPU>(a, bq, j, rec);
+  if (live) write_record<T, LPU>(static_cast<T *>(a.grad_loc_attn) + record_offset<MODE>(a, bq, g), P, j, rec);
   clear_tile_counts(a);
 }
 

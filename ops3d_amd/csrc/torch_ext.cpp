@@ -434,7 +434,9 @@ std::vector<at::Tensor> dcnv4_backward(const at::Tensor &value, const at::Tensor
     throw std::runtime_error("grad_output tensor has to be a contiguous CUDA tensor of the value dtype");
   const DeviceGuard guard(value.device());
   at::Tensor grad_value = at::empty_like(value);
-  at::Tensor grad_offset = at::zeros_like(p_offset);   // the row padding stays zero
+  // every unit's record is written; only a row padding has to be cleared
+  const int64_t used = group * 4 * (kd * kh * kw - (remove_center ? 1 : 0));
+  at::Tensor grad_offset = p_offset.size(4) == used ? at::empty_like(p_offset) : at::zeros_like(p_offset);
   const size_t wsb = ops3d_dcnv4_workspace_bytes(z.code, z.B, z.Din, z.Hin, z.Win, (int)group, (int)group_channels,
                                                  (int)kd, (int)kh, (int)kw, (int)sd, (int)sh, (int)sw, (int)pd,
                                                  (int)ph, (int)pw, (int)dd, (int)dh, (int)dw, (int)remove_center, 1);

@@ -250,7 +250,7 @@ bool coarse_level_heavy(int B, int S, int G, int L, int Q, int K, uint64_t tile_
 }
 
 struct BwdLayout {
-  uint64_t n, ntiles_bound;
+  uint64_t n, ntiles_bound, tiles_least;
   uint32_t tcap, split_slots;
   size_t off_keys, off_stash, off_entries, off_counts, off_start, off_cursor, off_queue, off_split,
       off_mat, off_vhm, off_ghm;
@@ -282,6 +282,7 @@ int bwd_layout(int B, int S, int G, int D, int e, int lpu, int L, int Q, int K, 
     const int nt = tile_threads(lpu, big_tiles(S, lpu));
     const uint64_t tvox = (uint64_t)(2 * nt / lpu);   // voxels of a nominal tile
     const uint64_t lb = (uint64_t)B * G * ((uint64_t)S + tvox - 1) / tvox;
+    ly.tiles_least = lb;
     ly.split_slots = S > 0 && (lb < kSplitTiles || coarse_level_heavy(B, S, G, L, Q, K, tvox, nt))
                          ? (uint32_t)kSplitSlots : 0u;
     ly.off_split = o; o += align256((size_t)ly.split_slots * tvox * D * 4);
@@ -685,6 +686,11 @@ static int backward_impl(const void *value, const void *value_head_major, const 
     g3.a.tile_affinity = num_heads % 8 == 0;
     g3.a.chunk = tile_chunk(channels, elem_size(dtype), tile_lanes(geo.lpu, geo.cpl * elem_size(dtype)),
                             a.big_tiles != 0);
+    // Few entries per tile (at least ceil(S / tile voxels) tiles per head): a tile is a chain of
+    // loads of which each waits for the one before, so smaller chunks, which leave room for more
+    // blocks per CU.  200 queries of 3 levels, 37376 voxels, batch 2 (8 samples per tile): tile
+    // kernel 38.8 us, with chunks of 256 / 192 / 128 entries 33.8 / 34.0 / 35.2.
+    if ((uint64_t)ly.n < 16 * ly.tiles_least) g3.a.chunk = g3.a.chunk < 256 ? g3.a.chunk : 256;
     g3.lds = tile_kernel_lds_bytes(g3.a.chunk, channels * elem_size(dtype),
                                    tile_lanes(geo.lpu, geo.cpl * elem_size(dtype)), a.big_tiles != 0);
     g3.grid = (unsigned)device_cus();   // times the resident blocks per CU (launch_one)

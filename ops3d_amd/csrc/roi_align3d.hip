@@ -13,10 +13,10 @@
 // the reference computes in the element type), rounded step by step (no contraction).
 //
 // Forward: a gather, one thread per (roi, CPT = 4 channels, bin), or on channels-last features
-// one lane per (bin, 8 channels) (the same bits).  With at most 2 samples per bin and axis it is
-// separable: the bin's average is the sum over its distinct z, y and x taps (at most 4 each) of
-// the per-axis weight sums times the value, fewer loads than 8 corners per sample; larger sample
-// grids take the reference's per-sample loop.  Backward: the adjoint, as a gather when the
+// one lane per (bin, 8 channels) (the same bits).  It is separable: the bin's average is the sum
+// over its distinct z, y and x taps of the per-axis weight sums times the value, taken along x, then
+// y, then z in fused multiply-adds, fewer loads than 8 corners per sample; bins of more than 8 taps
+// on an axis take the reference's per-sample loop.  Backward: the adjoint, as a gather when the
 // output has at most 64 bins per axis and 384 in all (each voxel sums, in registers, the rois
 // that reach it, in an order that they alone decide: no atomics, the same bits on every run; the workspace holds the
 // rois' axis weight tables and a channels-last copy of grad_output),
@@ -164,6 +164,12 @@ __device__ __forceinline__ AxisTaps4 bin_taps(float start, int p, float bin, int
 template <int NT>
 __device__ __forceinline__ AxisTaps<NT> bin_taps_n(float start, int p, float bin, int grid, int size, int order);
 
+// One step of a sum over taps: the first product, then fused multiply-adds.
+__device__ __forceinline__ float tap_add(int k, float w, float v, float sum) {
+#pragma clang fp contract(off)
+  return k == 0 ? w * v : fmaf(w, v, sum);
+}
+
 template <typename T, int CPT>
 __global__ __launch_bounds__(256) void roi_align3d_forward_kernel(const T *feat, const T *rois, T *out, int N, int C, int D,
                                                                   int H, int W, int R, int PD, int PH, int PW,
@@ -186,25 +192,32 @@ __global__ __launch_bounds__(256) void roi_align3d_forward_kernel(const T *feat,
   if (inb && q.gd <= 2 && q.gh <= 2 && q.gw <= 2) {
     // separable: the bin's average is sum over its distinct z, y, x taps of WZ * WY * WX * value
     // (the samples form a full grid and the corner weights are products, so the per-axis weight
-    // sums factor), at most 4 taps per axis instead of 8 corners per sample
+    // sums factor), at most 4 taps per axis instead of 8 corners per sample; summed along x, then
+    // y, then z (tap_add), as in the channels-last kernel
     const AxisTaps4 tz = bin_taps(q.sd, pd, q.bd, q.gd, D, order);
     const AxisTaps4 ty = bin_taps(q.sh, ph, q.bh, q.gh, H, order);
     const AxisTaps4 tx = bin_taps(q.sw, pw, q.bw, q.gw, W, order);
+    if (tx.n > 0 && ty.n > 0) {
 #pragma unroll
-    for (int kz = 0; kz < 4; ++kz) {
-      if (kz >= tz.n) break;
+      for (int kz = 0; kz < 4; ++kz) {
+        if (kz >= tz.n) break;
+        float u[CPT];
 #pragma unroll
-      for (int ky = 0; ky < 4; ++ky) {
-        if (ky >= ty.n) break;
-        const float wzy = tz.w[kz] * ty.w[ky];
-        const int64_t rowo = ((int64_t)tz.pos[kz] * H + ty.pos[ky]) * W;
+        for (int ky = 0; ky < 4; ++ky) {
+          if (ky >= ty.n) break;
+          const int64_t rowo = ((int64_t)tz.pos[kz] * H + ty.pos[ky]) * W;
+          float t[CPT];
 #pragma unroll
-        for (int kx = 0; kx < 4; ++kx) {
-          if (kx >= tx.n) break;
-          const float wgt = wzy * tx.w[kx];
+          for (int kx = 0; kx < 4; ++kx) {
+            if (kx >= tx.n) break;
 #pragma unroll
-          for (int c = 0; c < CPT; ++c) acc[c] = acc[c] + wgt * to_f(base[(int64_t)c * vol + rowo + tx.pos[kx]]);
+            for (int c = 0; c < CPT; ++c) t[c] = tap_add(kx, tx.w[kx], to_f(base[(int64_t)c * vol + rowo + tx.pos[kx]]), t[c]);
+          }
+#pragma unroll
+          for (int c = 0; c < CPT; ++c) u[c] = tap_add(ky, ty.w[ky], t[c], u[c]);
         }
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) acc[c] = tap_add(kz, tz.w[kz], u[c], acc[c]);
       }
     }
   }
@@ -217,20 +230,28 @@ __global__ __launch_bounds__(256) void roi_align3d_forward_kernel(const T *feat,
     const AxisTaps8 tx = bin_taps_n<kSepTaps>(q.sw, pw, q.bw, q.gw, W, order);
     if (!tz.over && !ty.over && !tx.over) {
       wide = false;
-      for (; tz.n > 0; tz.shift()) {
-        AxisTaps8 tyc = ty;
-        for (; tyc.n > 0; tyc.shift()) {
-          const float wzy = tz.w[0] * tyc.w[0];
-          const int64_t rowo = ((int64_t)tz.pos[0] * H + tyc.pos[0]) * W;
+      if (tx.n > 0 && ty.n > 0)
+        for (int kz = 0; tz.n > 0; tz.shift(), ++kz) {
+          AxisTaps8 tyc = ty;
+          float u[CPT];
 #pragma unroll
-          for (int kx = 0; kx < kSepTaps; ++kx) {
-            if (kx >= tx.n) break;
-            const float wgt = wzy * tx.w[kx];
+          for (int c = 0; c < CPT; ++c) u[c] = 0.f;
+          for (int ky = 0; tyc.n > 0; tyc.shift(), ++ky) {
+            const int64_t rowo = ((int64_t)tz.pos[0] * H + tyc.pos[0]) * W;
+            float t[CPT];
 #pragma unroll
-            for (int c = 0; c < CPT; ++c) acc[c] = acc[c] + wgt * to_f(base[(int64_t)c * vol + rowo + tx.pos[kx]]);
+            for (int kx = 0; kx < kSepTaps; ++kx) {
+              if (kx >= tx.n) break;
+#pragma unroll
+              for (int c = 0; c < CPT; ++c)
+                t[c] = tap_add(kx, tx.w[kx], to_f(base[(int64_t)c * vol + rowo + tx.pos[kx]]), t[c]);
+            }
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) u[c] = tap_add(ky, tyc.w[0], t[c], u[c]);
           }
+#pragma unroll
+          for (int c = 0; c < CPT; ++c) acc[c] = tap_add(kz, tz.w[0], u[c], acc[c]);
         }
-      }
     }
   }
   for (int iz = 0; wide && iz < q.gd; ++iz) {
@@ -960,6 +981,12 @@ __global__ __launch_bounds__(64, 4) void roi_align3d_backward_gather_kernel(
 // results are staged in LDS and written out as [R, C, PD, PH, PW] runs of bpb elements per
 // channel.  The blocks of a roi run on one XCD, whose L2 then serves the overlap of their taps.
 // The arithmetic is the NCDHW kernel's, term by term, so both give the same bits.
+// Measured (bf16 [2, 256, 32, 64, 64], 512 rois of 4-32 voxels, 7^3 bins, 2 samples per axis): 430 us
+// with every lane's own tap lists, one weight product, multiplication and addition per tap and
+// channel; 305 us with the lists made once per bin in LDS and the sum taken along x, y, z in fused
+// multiply-adds, four loads at a time (fp32 [1, 120, 21, 45, 77], 150 rois, adaptive samples: 130 ->
+// 72 us).  Bound by the lines that the rois' overlapping regions fetch past L2, about 2 GB; loading
+// only the taps that a bin has, or two rows at a time, measured the same (306, 307 us).
 constexpr int kClChannels = 8;                  // channels per lane
 
 template <typename T>
@@ -980,8 +1007,7 @@ __device__ __forceinline__ void load8(const T *p, float f[8]) {
 }
 
 // Bins per block: one per lane group (256 / (C / 8) groups), the (ph, pw) plane of a (roi, pd)
-// cut into equal parts.  One bin per thread measured fastest (more blocks in flight; bench
-// workload, rows of 7 bins: 1, 2, 7 rows per block 415, 453, 448 us).
+// cut into equal parts (one bin per thread: more blocks in flight).
 inline void cl_split(int C, int PHW, int &bpb, int &parts) {
   const int slots = 256 / (C / kClChannels);
   parts = (PHW + slots - 1) / slots;
@@ -990,16 +1016,30 @@ inline void cl_split(int C, int PHW, int &bpb, int &parts) {
 
 inline bool cl_supported(int C) { return C > 0 && C % kClChannels == 0 && C / kClChannels <= 256; }
 
-// WIDE: compiled with the separable path for grids of more than 2 samples per axis (launched
-// when sampling_ratio is adaptive or above 2; without it the kernel needs fewer registers).
+// The taps of one axis of one bin, in LDS.
+template <int NT>
+struct TapList {
+  int n, over, pos[NT];
+  float w[NT];
+};
+
+// WIDE: lists of 8 taps, for grids of more than 2 samples per axis (launched when sampling_ratio is
+// adaptive or above 2; without it the kernel needs fewer registers).  The tap lists of the block's
+// bins (one per axis and bin, z's once) are made by a thread each and read from LDS: the C / 8 lanes
+// of a bin each made all three before, 40 % of the kernel's instructions.
 template <typename T, bool WIDE>
-__global__ __launch_bounds__(256) void roi_align3d_forward_cl_kernel(const T *feat, const T *rois, T *out, int N, int C,
-                                                                     int D, int H, int W, int PD, int PH, int PW,
-                                                                     float scale, int sr, int order, int bpb, int parts,
-                                                                     int nblk) {
+__global__ __launch_bounds__(256) void roi_align3d_forward_cl_kernel(const T *__restrict__ feat, const T *__restrict__ rois,
+                                                                     T *__restrict__ out, int N, int C, int D, int H,
+                                                                     int W, int PD, int PH, int PW, float scale, int sr,
+                                                                     int order, int bpb, int parts, int nblk) {
 #pragma clang fp contract(off)
+  constexpr int NT = WIDE ? kSepTaps : 4;
+  using Taps = TapList<NT>;
   extern __shared__ __align__(16) unsigned char cl_lds[];
-  T *res = reinterpret_cast<T *>(cl_lds);   // [C][bpb]
+  Taps *list_l = reinterpret_cast<Taps *>(cl_lds);          // y of every bin, x of every bin, z
+  T *res = reinterpret_cast<T *>(list_l + 2 * bpb + 1);     // [C][bpb]
+  __shared__ float count_l;
+  __shared__ int item_l;
   // block i runs on XCD i % 8: XCD x takes the x-th eighth of the (roi, pd, part) blocks, so a
   // roi's blocks share one L2 (gridDim.x is a multiple of 8; nblk blocks are real)
   const unsigned blk = (blockIdx.x & 7u) * (gridDim.x / 8u) + (blockIdx.x >> 3);
@@ -1008,94 +1048,99 @@ __global__ __launch_bounds__(256) void roi_align3d_forward_cl_kernel(const T *fe
   const int rem = (int)(blk % (unsigned)(PD * parts));
   const int pd = rem / parts, b0 = (rem - pd * parts) * bpb;
   const int nbin = min(bpb, PH * PW - b0);
-  const int CG = C / kClChannels, slots = 256 / CG;
-  const int tid = threadIdx.x, cg = tid % CG, slot = tid / CG;
-  const Roi q = roi_setup(rois, r, scale, sr, PD, PH, PW);
-  const bool inb = q.b >= 0 && q.b < N;
+  const int CG = C / kClChannels;
+  const int tid = threadIdx.x, cg = tid % CG, bin = tid / CG;   // bpb * CG <= 256: one bin per lane group
+  for (int i = tid; i < 2 * nbin + 1; i += 256) {
+    const Roi q = roi_setup(rois, r, scale, sr, PD, PH, PW);
+    const int ax = i == 2 * nbin ? 0 : (i < nbin ? 1 : 2), b = b0 + (i < nbin ? i : i - nbin);
+    const int p = ax == 0 ? pd : (ax == 1 ? b / PW : b % PW);
+    const AxisTaps<NT> t = bin_taps_n<NT>(ax == 0 ? q.sd : (ax == 1 ? q.sh : q.sw), p, ax == 0 ? q.bd : (ax == 1 ? q.bh : q.bw),
+                                          ax == 0 ? q.gd : (ax == 1 ? q.gh : q.gw), ax == 0 ? D : (ax == 1 ? H : W), order);
+    Taps &l = list_l[i < nbin ? i : (i < 2 * nbin ? bpb + i - nbin : 2 * bpb)];
+    l.n = t.n;
+    l.over = t.over;
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+      l.pos[k] = t.pos[k];
+      l.w[k] = t.w[k];
+    }
+    if (ax == 0) {
+      count_l = q.count;
+      item_l = q.b;
+    }
+  }
+  __syncthreads();
+  const bool inb = item_l >= 0 && item_l < N;
   const int64_t vol = (int64_t)D * H * W;
-  const T *base = feat + (int64_t)(inb ? q.b : 0) * vol * C + cg * kClChannels;
-  const bool sep = q.gd <= 2 && q.gh <= 2 && q.gw <= 2;
-  AxisTaps4 tz;
-  if (inb && sep) tz = bin_taps(q.sd, pd, q.bd, q.gd, D, order);
-  AxisTaps8 tz8;   // larger grids: the z taps of plane pd, if they fit
-  tz8.over = true;
-  if (WIDE && inb && !sep) tz8 = bin_taps_n<kSepTaps>(q.sd, pd, q.bd, q.gd, D, order);
-  for (int bin = slot; slot < slots && bin < nbin; bin += slots) {
-    const int ph = (b0 + bin) / PW, pw = (b0 + bin) % PW;
+  const T *base = feat + (int64_t)(inb ? item_l : 0) * vol * C + cg * kClChannels;
+  if (bin < nbin) {
     float acc[kClChannels];
 #pragma unroll
     for (int c = 0; c < kClChannels; ++c) acc[c] = 0.f;
-    if (inb && sep) {
-      const AxisTaps4 ty = bin_taps(q.sh, ph, q.bh, q.gh, H, order);
-      const AxisTaps4 tx = bin_taps(q.sw, pw, q.bw, q.gw, W, order);
+    const Taps &ty = list_l[bin], &tz = list_l[2 * bpb];
+    const Taps tx = list_l[bpb + bin];
+    if (inb && !tz.over && !ty.over && !tx.over) {
+      // along x, then y, then z (the NCDHW kernel's sums)
+      const int nz = tx.n > 0 && ty.n > 0 ? tz.n : 0, ny = ty.n;
+      for (int kz = 0; kz < nz; ++kz) {
+        const uint32_t plane = (uint32_t)tz.pos[kz] * (uint32_t)H;
+        float u[kClChannels];
 #pragma unroll
-      for (int kz = 0; kz < 4; ++kz) {
-        if (kz >= tz.n) break;
+        for (int c = 0; c < kClChannels; ++c) u[c] = 0.f;
+        for (int ky = 0; ky < ny; ++ky) {
+          const uint32_t rowo = (plane + (uint32_t)ty.pos[ky]) * (uint32_t)W;
+          const float wy = ty.w[ky];
+          float t[kClChannels];
+          // four loads in flight; past the last tap its row again, left out of the sum
 #pragma unroll
-        for (int ky = 0; ky < 4; ++ky) {
-          if (ky >= ty.n) break;
-          const float wzy = tz.w[kz] * ty.w[ky];
-          const uint32_t rowo = ((uint32_t)tz.pos[kz] * (uint32_t)H + (uint32_t)ty.pos[ky]) * (uint32_t)W;
+          for (int x0 = 0; x0 < NT; x0 += 4) {
+            if (x0 > 0 && x0 >= tx.n) break;
+            float v[4][kClChannels];
 #pragma unroll
-          for (int kx = 0; kx < 4; ++kx) {
-            if (kx >= tx.n) break;
-            const float wgt = wzy * tx.w[kx];
-            float v[kClChannels];
-            load8(base + (rowo + (uint32_t)tx.pos[kx]) * (uint32_t)C, v);
-#pragma unroll
-            for (int c = 0; c < kClChannels; ++c) acc[c] = acc[c] + wgt * v[c];
-          }
-        }
-      }
-    }
-    bool wide = inb && !sep;
-    if (WIDE && wide && !tz8.over) {
-      // separable too when every axis has at most kSepTaps taps (the NCDHW kernel's loop)
-      AxisTaps8 ty = bin_taps_n<kSepTaps>(q.sh, ph, q.bh, q.gh, H, order);
-      const AxisTaps8 tx = bin_taps_n<kSepTaps>(q.sw, pw, q.bw, q.gw, W, order);
-      if (!ty.over && !tx.over) {
-        wide = false;
-        for (AxisTaps8 tzc = tz8; tzc.n > 0; tzc.shift()) {
-          for (AxisTaps8 tyc = ty; tyc.n > 0; tyc.shift()) {
-            const float wzy = tzc.w[0] * tyc.w[0];
-            const uint32_t rowo = ((uint32_t)tzc.pos[0] * (uint32_t)H + (uint32_t)tyc.pos[0]) * (uint32_t)W;
-#pragma unroll
-            for (int kx = 0; kx < kSepTaps; ++kx) {
-              if (kx >= tx.n) break;
-              const float wgt = wzy * tx.w[kx];
-              float v[kClChannels];
-              load8(base + (rowo + (uint32_t)tx.pos[kx]) * (uint32_t)C, v);
-#pragma unroll
-              for (int c = 0; c < kClChannels; ++c) acc[c] = acc[c] + wgt * v[c];
+            for (int k = 0; k < 4; ++k) {
+              const int pos = x0 + k < tx.n ? tx.pos[x0 + k] : tx.pos[x0];
+              load8(base + (rowo + (uint32_t)pos) * (uint32_t)C, v[k]);
             }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              if (x0 + k < tx.n)
+#pragma unroll
+                for (int c = 0; c < kClChannels; ++c) t[c] = tap_add(x0 + k, tx.w[x0 + k], v[k][c], t[c]);
+          }
+#pragma unroll
+          for (int c = 0; c < kClChannels; ++c) u[c] = tap_add(ky, wy, t[c], u[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < kClChannels; ++c) acc[c] = tap_add(kz, tz.w[kz], u[c], acc[c]);
+      }
+    } else if (WIDE && inb) {   // too many taps on some axis: sample by sample
+      const Roi q = roi_setup(rois, r, scale, sr, PD, PH, PW);
+      const int ph = (b0 + bin) / PW, pw = (b0 + bin) % PW;
+      for (int iz = 0; iz < q.gd; ++iz) {
+        const float z = sample_coord(q.sd, pd, q.bd, iz, q.gd);
+        for (int iy = 0; iy < q.gh; ++iy) {
+          const float y = sample_coord(q.sh, ph, q.bh, iy, q.gh);
+          for (int ix = 0; ix < q.gw; ++ix) {
+            const float x = sample_coord(q.sw, pw, q.bw, ix, q.gw);
+            int64_t off[8];
+            float w[8];
+            if (!corners(z, y, x, D, H, W, order, off, w)) continue;
+            float s[kClChannels];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              float v[kClChannels];
+              load8(base + (uint32_t)off[k] * (uint32_t)C, v);
+#pragma unroll
+              for (int c = 0; c < kClChannels; ++c) s[c] = k == 0 ? w[0] * v[c] : s[c] + w[k] * v[c];
+            }
+#pragma unroll
+            for (int c = 0; c < kClChannels; ++c) acc[c] = acc[c] + s[c];
           }
         }
       }
     }
-    for (int iz = 0; wide && iz < q.gd; ++iz) {
-      const float z = sample_coord(q.sd, pd, q.bd, iz, q.gd);
-      for (int iy = 0; iy < q.gh; ++iy) {
-        const float y = sample_coord(q.sh, ph, q.bh, iy, q.gh);
-        for (int ix = 0; ix < q.gw; ++ix) {
-          const float x = sample_coord(q.sw, pw, q.bw, ix, q.gw);
-          int64_t off[8];
-          float w[8];
-          if (!corners(z, y, x, D, H, W, order, off, w)) continue;
-          float s[kClChannels];
 #pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            float v[kClChannels];
-            load8(base + (uint32_t)off[k] * (uint32_t)C, v);
-#pragma unroll
-            for (int c = 0; c < kClChannels; ++c) s[c] = k == 0 ? w[0] * v[c] : s[c] + w[k] * v[c];
-          }
-#pragma unroll
-          for (int c = 0; c < kClChannels; ++c) acc[c] = acc[c] + s[c];
-        }
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < kClChannels; ++c) res[(cg * kClChannels + c) * nbin + bin] = from_f<T>(acc[c] / q.count);
+    for (int c = 0; c < kClChannels; ++c) res[(cg * kClChannels + c) * nbin + bin] = from_f<T>(acc[c] / count_l);
   }
   __syncthreads();
   // channel c's bins b0 .. b0 + nbin - 1 of plane pd are nbin consecutive output elements
@@ -1191,8 +1236,9 @@ int forward_cl(const void *features_cl, const void *rois, void *output, int N, i
   const int64_t blocks = (int64_t)R * PD * parts;
   const int64_t grid = (blocks + 7) / 8 * 8;   // a multiple of 8: the kernel maps blocks to XCDs
   if (grid >= ((int64_t)1 << 31)) return OPS3D_FDA_EINVAL;
-  const size_t lds = (size_t)C * bpb * sizeof(T);
-  if (sr > 0 && sr <= 2)   // every roi's grid is separable with 4 taps per axis
+  const bool narrow = sr > 0 && sr <= 2;
+  const size_t lds = (size_t)C * bpb * sizeof(T) + (size_t)(2 * bpb + 1) * (narrow ? sizeof(TapList<4>) : sizeof(TapList<kSepTaps>));
+  if (narrow)   // every roi's grid is separable with 4 taps per axis
     hipLaunchKernelGGL((roi_align3d_forward_cl_kernel<T, false>), dim3((unsigned)grid), dim3(256), lds, st,
                        static_cast<const T *>(features_cl), static_cast<const T *>(rois), static_cast<T *>(output), N,
                        C, D, H, W, PD, PH, PW, scale, sr, order, bpb, parts, (int)blocks);

@@ -433,3 +433,38 @@ def test_gpu_backward_infinities_stay_in_their_bins(gpu_device):
     assert np.array_equal(np.isfinite(got), np.isfinite(want))
     ok = np.isfinite(want)
     assert_close("finite part", torch.from_numpy(np.where(ok, got, 0.0)), np.where(ok, want, 0.0), 1e-5, 1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C,pooled,sr,dt", [
+    (120, (2, 3, 9), 2, torch.bfloat16),      # 15 lanes a bin: one thread of a block without a bin
+    (200, (1, 5, 41), 2, torch.float16),      # 205 bins of a plane in parts of 10
+    (8, (2, 17, 19), 1, torch.float32),       # 323 bins, up to 256 a block
+    (2048, (1, 2, 3), 4, torch.float32),      # one bin a block, lists of 8
+    (64, (3, 2, 40), 0, torch.bfloat16),      # adaptive: lists of 8, wider bins sample by sample
+])
+def test_gpu_channels_last_blocks(gpu_device, C, pooled, sr, dt):
+    """The channels-last forward's split of a plane's bins over blocks and its tap lists: the NCDHW
+    kernel's bits, and the oracle's values."""
+    import ctypes
+
+    from fda_helpers import TOL, assert_close, log
+
+    from ops3d_amd import _extension
+
+    lib = _extension.load_library()
+    log(f"[case] roi_align3d channels-last blocks: C={C} pooled={pooled} sr={sr} {dt}")
+    code = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dt]
+    N, size, R = 1, (5, 7, 33), 4
+    r = np.random.default_rng(C)
+    x = torch.from_numpy(r.normal(size=(N, C) + size).astype(np.float32)).to(dt).to(gpu_device)
+    rois = torch.from_numpy(_rois(R, N, size, seed=C + 1, lo=-1.0)).to(dt).to(gpu_device)
+    xc = x.permute(0, 2, 3, 4, 1).contiguous()
+    o1, o2 = (torch.full((R, C) + pooled, 7.0, dtype=dt, device=gpu_device) for _ in range(2))
+    args = (code, N, C, *size, R, *pooled, ctypes.c_float(1.0), sr, 1, torch.cuda.current_stream().cuda_stream)
+    assert lib.ops3d_roi_align3d_forward(x.data_ptr(), rois.data_ptr(), o1.data_ptr(), *args) == 0
+    assert lib.ops3d_roi_align3d_forward_channels_last(xc.data_ptr(), rois.data_ptr(), o2.data_ptr(), *args) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(o1, o2)
+    want = O.forward(x.cpu().double().numpy(), rois.cpu().double().numpy(), pooled, 1.0, sr, 1)
+    assert_close("channels-last blocks", o2, want, *TOL[dt])

@@ -18,7 +18,7 @@
 // counters, tile_headscan scans them per head (one block) into tile_start and the cursors,
 // and tile_scatter reserves each block's range of a tile with one global atomic on
 // the tile's cursor.  Correct for any size, slower (the atomics of all blocks contend).
-// Heads of at most kFusedHeadSamples samples take one block each, and tile_scatter<.., true>
+// Small heads (one_block_per_head) take one block each, and tile_scatter<.., true>
 // counts, scans and places them in one launch (no count or head-scan launch; its counters are
 // read past L1 in atomic mode, since other heads' blocks may have cached the same lines).
 // Each head owns the entry range [bg * 8 * per_head, ...) (a sample has at most 8 entries), so
@@ -33,7 +33,11 @@ namespace ops3d_fda {
 constexpr int kBucketThreads = 1024;
 constexpr int kWin = 8192;                            // LDS histogram window (tiles of one head)
 constexpr int kBlocksPerHead = 64;
-constexpr uint32_t kFusedHeadSamples = 4096;          // heads this small take one fused block
+// Heads of at most this many samples take one fused block: in any call, in a call of few heads,
+// and in one whose heads alone occupy half the CUs (one_block_per_head()).
+constexpr uint32_t kFusedHeadSamples = 4096, kFusedFewHeads = 5120, kFusedManyHeads = 32768;
+constexpr uint32_t kFusedHeads = 128;                 // heads of a call that count as many
+constexpr uint32_t kFusedTcap = 16 * kWin;            // 2^21 voxels: kWin tiles of 256
 
 struct BucketArgs {
   const uint32_t *keys;        // [N] tile_key of each sample or kKeyInvalid
@@ -462,6 +466,25 @@ uint32_t tile_window(uint32_t tcap) { return tcap < (uint32_t)kWin ? (tcap > 0 ?
 // to tcap tiles.
 size_t tile_matrix_words(uint32_t BG, uint32_t tcap) { return (size_t)BG * kBlocksPerHead * tcap; }
 
+// Whether one block per head counts, scans and places its samples (two launches fewer, the keys
+// read twice instead of three times and no count matrix) or kBlocksPerHead blocks do.  One block
+// is a serial chain over its head's samples, so it pays while the chain is shorter than the
+// launches it saves, or while the heads alone fill the chip.  Whole backward pass, us, one
+// block / many blocks (two levels of 4x8x16 and 2x4x8, fp32; three of 16x32x64 .. 4x8x16, bf16):
+//     8 heads   4608: 46.7 / 46.7, 57.8 / 58.6   6144: 49.8 / 46.9, 61.3 / 59.3
+//    32 heads   4608: 56.9 / 57.5, 96.6 / 99.4   6144: 61.3 / 58.0, 105 / 105
+//    64 heads   5120: 84 / 88, 165 / 177         8192: 108 / 105, 189 / 195
+//   128 heads   8192: 151 / 161, 344 / 371      32768: 478 / 500, 601 / 658
+//   256 heads   8192: 233 / 267, 672 / 739      16384: 438 / 501, 859 / 967
+// (the host saves 5 us of its 20 per call in each of them), and over the 32x64x256 .. 8x16x64
+// levels, bf16, 128 heads of 16 channels: 5120: 2654 / 2706, 32768: 2342 / 2500.  Volumes that can
+// pass the LDS window (atomic mode) keep the lower bound: not measured beyond it.
+inline bool one_block_per_head(uint32_t per_head, uint32_t heads, uint32_t tcap) {
+  if (per_head <= kFusedHeadSamples) return true;
+  if (tcap > kFusedTcap) return false;
+  return per_head <= (heads >= kFusedHeads ? kFusedManyHeads : kFusedFewHeads);
+}
+
 hipError_t launch_tile_bucketing(const uint32_t *keys, uint32_t n, uint32_t per_head,
                                  const int64_t *shapes, int L, int BG, int TX, int TY, int TZ, uint32_t *counts,
                                  uint32_t *start, uint32_t *cursor, uint32_t *mat, uint32_t tcap, uint32_t *entries, uint32_t *queue,
@@ -478,7 +501,7 @@ hipError_t launch_tile_bucketing(const uint32_t *keys, uint32_t n, uint32_t per_
   a.chunk = (a.chunk + kBucketThreads - 1) / kBucketThreads * kBucketThreads;
   if (a.chunk == 0) a.chunk = kBucketThreads;
   // small heads: one block per head that counts, scans and scatters in one launch
-  a.fused = n > 0 && per_head <= kFusedHeadSamples;
+  a.fused = n > 0 && one_block_per_head(per_head, (uint32_t)BG, tcap);
   if (a.fused) a.chunk = (per_head + kBucketThreads - 1) / kBucketThreads * kBucketThreads;
   a.blocks_per_head = (per_head + a.chunk - 1) / a.chunk;
   if (n == 0) a.blocks_per_head = 0;   // every counter is zero: the head scan writes zeros

@@ -255,6 +255,20 @@ def test_split_coarse_levels(gpu_device, shapes, B, Q, G, D, K, dt):
     _check(f"split {shapes} B={B} Q={Q} G={G} D={D}", inp, gpu_device, dt)
 
 
+# --- bucketing by one block per head or by many ------------------------------------------------
+@pytest.mark.parametrize("shapes,B,Q,G,D,K,dt", [
+    ([(4, 8, 16), (2, 4, 8)], 1, 640, 8, 32, 4, torch.float32),      # 5120 samples per head: one block
+    ([(4, 8, 16), (2, 4, 8)], 1, 641, 8, 32, 4, torch.bfloat16),     # 5128: many blocks
+    ([(5, 9, 17), (3, 5, 9)], 8, 641, 16, 8, 4, torch.float32),      # 128 heads, ragged staging rounds
+    ([(6, 9, 14)], 8, 8192, 16, 8, 4, torch.bfloat16),               # 128 heads of 32768: one block
+    ([(6, 9, 14)], 8, 8193, 16, 8, 4, torch.bfloat16),               # one query more: many blocks
+    ([(1, 1, 66000), (2, 3, 4)], 1, 600, 2, 8, 4, torch.float32),    # 8251 tiles: atomic mode
+])
+def test_bucketing_blocks(gpu_device, shapes, B, Q, G, D, K, dt):
+    inp = random_inputs(shapes, B, Q, G, D, K, dt, seed=Q, lo=-0.05, hi=1.05)
+    _check(f"bucketing {shapes} B={B} Q={Q} G={G}", inp, gpu_device, dt)
+
+
 # --- head widths, head counts (XCD mappings), dtypes ---------------------------------------
 @pytest.mark.parametrize("D", [8, 16, 24, 32, 48, 64, 96, 128])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])

@@ -18,10 +18,10 @@
 // y, then z in fused multiply-adds, fewer loads than 8 corners per sample; bins of more than 8 taps
 // on an axis take the reference's per-sample loop.  Backward: the adjoint, as a gather when the
 // output has at most 64 bins per axis and 384 in all (each voxel sums, in registers, the rois
-// that reach it, in an order that they alone decide: no atomics, the same bits on every run; the workspace holds the
-// rois' axis weight tables and a channels-last copy of grad_output),
-// otherwise (or with more than 2^20 channels) by fp32 atomics into a channels-last workspace (64 lanes = 64 contiguous channels
-// per atomic instruction) transposed into grad_input afterwards.  A roi whose batch index is
+// that reach it, in an order that they alone decide: no atomics, the same bits on every run; the
+// workspace holds the rois' axis weight tables and a channels-last copy of grad_output), otherwise
+// (or with more than 2^20 channels) by fp32 atomics into a channels-last workspace (64 lanes = 64
+// contiguous channels per atomic instruction) transposed into grad_input afterwards.  A roi whose batch index is
 // outside [0, N) reads and writes nothing (its output is 0; the reference indexes out of
 // bounds).
 #include <hip/hip_runtime.h>
@@ -519,17 +519,16 @@ __global__ __launch_bounds__(64 * kBwdWaves) void roi_align3d_backward_kernel(co
 // samples of their corner weights, separable because the samples form a full grid.  A wave owns a
 // tile of 4 x 4 x 4 voxels and 64 channels, a lane per channel, its 64 sums in registers, and adds
 // up the rois whose footprint reaches the tile in a fixed order (index order, except that of every
-// 192 the few with small bins come last), so the result is the same on every run.  With channels on the lanes everything but top is uniform over the wave: weights, bin
-// ranges and loop bounds sit in scalar registers, no lane diverges and nothing is staged in LDS,
-// and the sum is taken axis by axis -- over pw into 4 x positions, over ph into 4 x 4, over pd into
+// 192 the few with small bins come last), so the result is the same on every run.  With channels
+// on the lanes everything but top is uniform over the wave: weights, bin ranges and loop bounds sit
+// in scalar registers, no lane diverges, and the sum is taken axis by axis -- over pw into 4 x positions, over ph into 4 x 4, over pd into
 // the 64 voxels -- about 5 multiply-adds per voxel and roi instead of one per bin combination.
 // A lane's top values of a bin row (one 128-byte line per bin from the channels-last copy) are
 // loaded one row ahead.
-// Three passes fill the workspace's inputs: roi_axis_table_kernel, grad_channels_last_kernel, and
-// this kernel reads them.  Needs at most 64 bins per axis and 384 in all (else the atomic path).
+// Two passes fill the workspace first: roi_axis_table_kernel and grad_channels_last_kernel.  Needs at most 64 bins per axis and 384 in all (else the atomic path).
 // What it measured, and what bounds it: at backward().
 constexpr int kGT = 4;                           // tile edge
-constexpr int kGRun = 128;                       // consecutive tiles of one XCD when not ordered
+constexpr int kGRun = 128;                       // consecutive tiles of one XCD when not ordered, at most
 constexpr int kGMaxAxisBins = 64, kGMaxBins = 384;
 
 constexpr int kGMaxChannels = 1 << 20;           // a roi's bins within 32-bit byte offsets
@@ -677,6 +676,8 @@ __global__ __launch_bounds__(1024) void roi_tile_order_kernel(const uint8_t *cou
   __syncthreads();
   for (int i = t; i < tiles; i += 1024) order[atomicAdd(&at_l[255 - counts[i]], 1u)] = (unsigned short)i;
 }
+constexpr int kGUnordered = 8192;                // waves whose order is no matter: twice what runs at once
+constexpr int kGSplitBlocks = 1024, kGSplitRois = 8;
 constexpr int kGOrdered = 65535;                 // tiles that are ordered (16-bit numbers)
 constexpr int kGList = 192;                      // rois listed at a time
 
@@ -690,18 +691,26 @@ __device__ __forceinline__ RawOf<T> load_raw(__amdgpu_buffer_rsrc_t rs, uint32_t
     return __builtin_amdgcn_raw_buffer_load_b16(rs, (int)voff, (int)soff, 0);
 }
 
-template <typename T>
-__global__ __launch_bounds__(64, 4) void roi_align3d_backward_gather_kernel(
+// SPLIT: a block of kGSplit waves per tile and channel group, each taking every kGSplit-th roi; their
+// sums are added in LDS, wave w those of plane w (launched where the tiles alone leave most of the
+// chip idle).
+constexpr int kGSplit = 4;
+template <typename T, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, SPLIT ? 2 : 4) void roi_align3d_backward_gather_kernel(
     const T *__restrict__ top_cl, const T *__restrict__ rois, T *__restrict__ grad, const float *__restrict__ wt,
-    const uint32_t *__restrict__ tr, const unsigned short *__restrict__ order, bool vec, int N, int C, int D, int H,
-    int W, int R, int PD, int PH, int PW, int blocks) {
-  __shared__ uint4 list_l[kGList];
-  const int lane = threadIdx.x;
+    const uint32_t *__restrict__ tr, const unsigned short *__restrict__ order, int N, int C, int D, int H,
+    int W, int R, int PD, int PH, int PW, int blocks, int run) {
+  constexpr int NW = SPLIT ? kGSplit : 1;
+  static_assert(!SPLIT || kGSplit == kGT, "a wave per plane of the tile");
+  __shared__ uint4 lists_l[NW][kGList];
+  __shared__ float sums_l[SPLIT ? kGSplit : 1][SPLIT ? kGT * kGT * kGT : 1][64];
+  const int lane = threadIdx.x & 63, wave = SPLIT ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  uint4 *const list_l = lists_l[wave];
   const int ntz = tiles_of(D), nty = tiles_of(H), ntx = tiles_of(W);
   const int ncg = (C + 63) / 64;
   // Tiles differ several times over in the rois that they meet, so a block is one wave (a larger one
   // would hold its slots until its last wave is done), and with `order` the crowded tiles come first.
-  // Without it block i runs on XCD i % 8: an XCD takes runs of kGRun neighbouring tiles, which read
+  // Without it block i runs on XCD i % 8: an XCD takes runs of `run` neighbouring tiles, which read
   // the same rois' bins, and which run of a round of eight it takes moves on, so that no XCD gets
   // only the crowded middle of the volume.
   int bid = blockIdx.x, cg;
@@ -710,8 +719,8 @@ __global__ __launch_bounds__(64, 4) void roi_align3d_backward_gather_kernel(
     cg = bid % ncg;
     bid = order[bid / ncg];
   } else {
-    const int seq = bid >> 3, round = seq / kGRun, xcd = (bid + round + round / 4 + round / 16) & 7;
-    bid = (round * 8 + xcd) * kGRun + seq % kGRun;
+    const int seq = bid >> 3, round = seq / run, xcd = (bid + round + round / 4 + round / 16) & 7;
+    bid = (round * 8 + xcd) * run + seq % run;
     if (bid >= blocks) return;
     const int tiles = ntx * nty * ntz, ng = bid / tiles;
     cg = ng % ncg;
@@ -790,13 +799,13 @@ __global__ __launch_bounds__(64, 4) void roi_align3d_backward_gather_kernel(
     for (int k = 0; k < 4; ++k) off[k] = (uint32_t)min(k, nx - 1) * bin_bytes + cl_bytes;
   };
 
-  for (int r0 = 0; r0 < R;) {
+  for (int r0 = 0; r0 * NW + wave < R;) {
     // the next rois of batch item n that reach the tile, in index order: from the front those with
     // at most 4 bins on every axis of it and only finite values (nearly all), from the back the
     // others
     int narrow = 0, wide = 0;
-    for (; r0 < R && narrow + wide <= kGList - 64; r0 += 64) {
-      const int r = r0 + lane, q = min(r, R - 1);
+    for (; r0 * NW + wave < R && narrow + wide <= kGList - 64; r0 += 64) {
+      const int r = (r0 + lane) * NW + wave, q = min(r, R - 1);
       const uint32_t z = tr[(size_t)tz * R + q], y = tr[(size_t)(ntz + ty) * R + q], x = tr[(size_t)(ntz + nty + tx) * R + q];
       const int item = (int)to_f(rois[(int64_t)q * 7]);
       const int cz = last_bin(z) - first_bin(z), cy = last_bin(y) - first_bin(y), cx = last_bin(x) - first_bin(x);
@@ -942,27 +951,41 @@ __global__ __launch_bounds__(64, 4) void roi_align3d_backward_gather_kernel(
     }
     __builtin_amdgcn_wave_barrier();   // the list is read before the next rois are written to it
   }
+  if constexpr (SPLIT) {   // wave w: the sums of plane w, in acc[0]
+#pragma unroll
+    for (int z = 0; z < kGT; ++z)
+#pragma unroll
+      for (int j = 0; j < kGT * kGT; ++j) sums_l[wave][z * kGT * kGT + j][lane] = acc[z][j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kGT * kGT; ++j) {
+      acc[0][j] = sums_l[0][wave * kGT * kGT + j][lane];
+#pragma unroll
+      for (int k = 1; k < NW; ++k) acc[0][j] += sums_l[k][wave * kGT * kGT + j][lane];
+    }
+  }
   if (c >= C) return;
   T *o = grad + ((int64_t)n * C + c) * D * H * W;
 #pragma unroll
-  for (int z = 0; z < kGT; ++z)
+  for (int z = 0; z < (SPLIT ? 1 : kGT); ++z)
 #pragma unroll
     for (int y = 0; y < kGT; ++y) {
-      if (z0 + z >= D || y0 + y >= H) continue;
-      T *row = o + ((int64_t)(z0 + z) * H + (y0 + y)) * W + x0;
+      const int zz = z0 + (SPLIT ? wave : z);
+      if (zz >= D || y0 + y >= H) continue;
+      T *row = o + ((int64_t)zz * H + (y0 + y)) * W + x0;
       T e[kGT];
 #pragma unroll
       for (int x = 0; x < kGT; ++x) e[x] = from_f<T>(acc[z][y * kGT + x]);
-      if (vec) {   // W % 4 == 0 and grad aligned: one 8- or 16-byte store
+      if (x0 + kGT <= W) {   // one 8- or 16-byte store, at any alignment
         if constexpr (sizeof(T) == 4) {
-          *reinterpret_cast<float4 *>(row) = make_float4(e[0], e[1], e[2], e[3]);
+          __builtin_memcpy(row, e, sizeof(e));
         } else {
           uint32_t h[2];
 #pragma unroll
           for (int k = 0; k < 2; ++k)
             h[k] = (uint32_t)__builtin_bit_cast(unsigned short, e[2 * k]) |
                    ((uint32_t)__builtin_bit_cast(unsigned short, e[2 * k + 1]) << 16);
-          *reinterpret_cast<uint2 *>(row) = make_uint2(h[0], h[1]);
+          __builtin_memcpy(row, h, sizeof(h));
         }
       } else {
 #pragma unroll
@@ -1266,7 +1289,7 @@ inline size_t gather_tables_bytes(int R, int D, int H, int W, int PD, int PH, in
 }
 
 // Backward.  Measured on bf16 [2, 256, 32, 64, 64], 512 rois of 4-32 voxels, 7^3 bins, one MI355X:
-// tables 7, copy 47, tile counts and order 14, gather 445 us (0.96 ms forward and backward); before,
+// tables 7, copy 47, tile counts and order 14, gather 445 us (0.86 ms forward and backward); before,
 // with a block per 4 x 8 x 8 voxels and 16 channels that staged its rois' bins in LDS, a thread per
 // voxel: tables 6, copy 75, gather 1572 us (2.10 ms).  The gather issues 132 M vector instructions
 // (40 % of the issue slots at four waves per SIMD) and waits for its loads for most of the rest:
@@ -1274,7 +1297,14 @@ inline size_t gather_tables_bytes(int R, int D, int H, int W, int PD, int PH, in
 // form (blocks of four waves, dynamic loops, weights by scalar loads) 943 us; rows loaded a plane
 // ahead and weights fetched by the lanes 680; one wave per block 537; crowded tiles first 500 (-45);
 // no spilled registers 445.  Without `order` an XCD's runs of 8 / 32 / 128 / 512 tiles measured
-// 554 / 535 / 522 / 540 us.  Joining the tiles of a block of two or four waves in LDS, to store
+// 554 / 535 / 522 / 540 us.  Launches of few waves are not ordered (the two passes cost 10 us).  With few waves the rois' serial chain is the time: four
+// waves per tile, each with a quarter of the rois, up to kGSplitBlocks blocks (forward and backward,
+// split / not: 17x24x28, 404 rois, 32 channels 264 / 639 us; 26x35x31, 21 rois, 64 channels 74 / 102;
+// 10x23x65, 213 rois, 256 channels (2448 blocks) 96 / 92; 13x25x50, 160 rois, nearest 80 / 48).
+// Stores of 4 voxels at any alignment: W = 50, 35 rois 320 -> 249 us.  Slower than the voxel threads
+// before it: few rois over many channels of a large volume, where the 4-voxel stores, which take
+// about 0.2 ms per 105 MB of gradient, are the time (64 rois of 4-16 voxels 330 / 285, 35 nearest rois
+// over [2, 256, 41, 50, 50] 249 / 187).  Joining the tiles of a block of two or four waves in LDS, to store
 // longer runs, 502 / 520 us against 492; three waves per SIMD 542.
 template <typename T>
 int backward(const void *grad_output, const void *rois, void *grad_input, float *acc, int N, int C, int D, int H,
@@ -1282,7 +1312,8 @@ int backward(const void *grad_output, const void *rois, void *grad_input, float 
   if (gather_fits(C, PD, PH, PW)) {
     const int ntz = tiles_of(D), nty = tiles_of(H), ntx = tiles_of(W);
     const int64_t tiles = (int64_t)N * ntz * nty * ntx, blocks = tiles * ((C + 63) / 64);
-    const int64_t grid = (blocks + 8 * kGRun - 1) / (8 * kGRun) * (8 * kGRun);   // whole rounds of runs
+    // tiles in runs (at least about four rounds of them over the XCDs), the grid whole rounds
+    const int64_t run = blocks >= 32 * kGRun ? kGRun : (blocks + 31) / 32, grid = (blocks + 8 * run - 1) / (8 * run) * (8 * run);
     if (grid >= ((int64_t)1 << 31)) return OPS3D_FDA_EINVAL;
     // workspace: the per-roi axis tables, then grad_output channels-last [R, bins, C]
     float *wt = acc;
@@ -1300,17 +1331,20 @@ int backward(const void *grad_output, const void *rois, void *grad_input, float 
     // the tiles' order, in the tables' second part beyond the words that tr takes, where it fits
     const int64_t used = (int64_t)R * (ntz + nty + ntx) * 4, spare = (int64_t)R * (D + H + W) * 4 - used;
     unsigned short *order = nullptr;
-    if (tiles <= kGOrdered && tiles * 3 <= spare) {
+    if (blocks > kGUnordered && tiles <= kGOrdered && tiles * 3 <= spare) {
       order = reinterpret_cast<unsigned short *>(reinterpret_cast<char *>(tr) + used);
       uint8_t *counts = reinterpret_cast<uint8_t *>(order + tiles);
       hipLaunchKernelGGL((roi_tile_count_kernel<T>), dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, st,
                          static_cast<const T *>(rois), tr, counts, ntz, nty, ntx, R, (int)tiles);
       hipLaunchKernelGGL(roi_tile_order_kernel, dim3(1), dim3(1024), 0, st, counts, order, (int)tiles);
     }
-    const bool vec = W % kGT == 0 && (reinterpret_cast<uintptr_t>(grad_input) & (kGT * sizeof(T) - 1)) == 0;
-    hipLaunchKernelGGL((roi_align3d_backward_gather_kernel<T>), dim3((unsigned)grid), dim3(64), 0, st, top_cl,
-                       static_cast<const T *>(rois), static_cast<T *>(grad_input), wt, tr, order, vec, N, C, D, H, W, R, PD,
-                       PH, PW, (int)blocks);
+    const auto gather = [&](auto kern, int threads) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), 0, st, top_cl, static_cast<const T *>(rois),
+                         static_cast<T *>(grad_input), wt, tr, order, N, C, D, H, W, R, PD, PH, PW, (int)blocks,
+                         (int)run);
+    };
+    if (blocks <= kGSplitBlocks && R >= kGSplitRois) gather(roi_align3d_backward_gather_kernel<T, true>, 64 * kGSplit);
+    else gather(roi_align3d_backward_gather_kernel<T, false>, 64);
     return hipGetLastError() == hipSuccess ? OPS3D_FDA_OK : OPS3D_FDA_ERUNTIME;
   }
   const int64_t nin = (int64_t)N * C * D * H * W;

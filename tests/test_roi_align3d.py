@@ -382,6 +382,10 @@ TILE_CASES = [
     (1, 33, (5, 6, 8), 7, (4, 4, 4), 2, torch.float32),           # 64 bins: one row per lane in the copy
     (1, 3, (6, 7, 9), 5, (6, 8, 8), 2, torch.bfloat16),           # 384 bins
     (1, 8, (16, 40, 48), 3, (3, 3, 3), 2, torch.float32),         # few rois, many tiles: the natural tile order
+    (1, 70, (9, 10, 11), 8, (3, 3, 3), 2, torch.float32),         # rois over four waves, two each
+    (2, 5, (4, 6, 7), 259, (2, 2, 2), 1, torch.bfloat16),         # the same, over 64 rois to a wave
+    (2, 70, (16, 40, 46), 9, (3, 2, 3), 2, torch.bfloat16),       # 1920 blocks: one wave each, W not of 4
+    (1, 8, (1, 2, 32900), 12, (2, 2, 3), 2, torch.float32),       # 8225 blocks: crowded tiles first
 ]
 
 

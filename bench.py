@@ -235,8 +235,8 @@ def measure_offsets(w, steps, warmup, device):
 
 def measure_nms(n, steps, warmup, device, threshold=0.3, cpu=True):
     """3-D NMS over n clustered boxes (a few hundred clusters, extents 2-12, scores with ties):
-    the whole _C.nms_3d call (sort, IoU mask, greedy pass, the kept count read back), and the
-    float32 CPU oracle on the same boxes."""
+    the whole _C.nms_3d call (order, overlapping pairs, suppression rounds, the kept count read
+    back), and the float32 CPU oracle on the same boxes."""
     import numpy as np
     import torch
 
@@ -622,7 +622,7 @@ def main():
         for n in (4096, 16384, 65536):
             o = measure_nms(n, args.steps, args.warmup, dev, cpu=n <= 16384)
             cpu = f" | CPU oracle (numpy fp32, 1 core) {o['cpu_ms']:9.1f} ms" if "cpu_ms" in o else ""
-            log(f" nms3d n={n:6d} | GPU {o['gpu']['median'] * 1e3:9.1f} us per call (sort + mask + greedy + count), "
+            log(f" nms3d n={n:6d} | GPU {o['gpu']['median'] * 1e3:9.1f} us per call (order + pairs + rounds + count), "
                 f"kept {o['kept']}{cpu}")
         if args.nms:
             return

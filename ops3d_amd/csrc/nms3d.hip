@@ -444,8 +444,10 @@ __global__ __launch_bounds__(256) void nms3d_extent_kernel(const Box *placed, in
 //   they are packed in LDS and the wave's lanes take their pairs.
 //   otherwise: one pair of blocks; lane r holds row box r, each wave a quarter of the columns, which
 //   come four at a time through scalar registers.
-// Pairs are collected in LDS and appended to one of kLists lists with one add per workgroup (more
-// only when a wave's buffer fills up).
+// Pairs are collected in LDS and appended to the kLists lists with one add per workgroup.  A wave whose
+// buffer fills up writes it out, each time to its next list, and what is left at the end goes to one
+// list only if it is no more than such a piece: a few crowded blocks (or a single one) fill all lists
+// evenly, so the lists hold kPairsPerBox pairs per box together, wherever the pairs lie.
 constexpr int kPairBuf = 256;
 constexpr int kColumns = 4;   // column boxes in scalar registers at a time
 template <bool PLACED>
@@ -455,9 +457,11 @@ __global__ __launch_bounds__(256) void nms3d_pair_kernel(const Box *__restrict__
   __shared__ uint2 buf_l[4][kPairBuf];
   __shared__ int cnt_l[4], base_l;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int list = (int)(blockIdx.x + blockIdx.y) % kLists;
-  uint2 *out = lists + (int64_t)list * capacity;
-  uint32_t *counter = counters + list * kCounterStride;
+  // the block's first list, hashed (the pairs lie in blocks at regular distances: the diagonal), its
+  // waves' 4 apart, moved on by one with every piece
+  static_assert(kLists == 16, "the top four bits of the hash");
+  const uint32_t first_list = (blockIdx.x * 0x9e3779b1u + blockIdx.y * 0x85ebca77u) >> 28;
+  uint32_t piece = first_list + 4u * (uint32_t)wv;
   int rb, cb0;
   if (PLACED) {
     rb = blockIdx.y;
@@ -480,6 +484,20 @@ __global__ __launch_bounds__(256) void nms3d_pair_kernel(const Box *__restrict__
   const auto overlap = [](const float *a, const float *b) {
     return (a[0] < b[3]) & (b[0] < a[3]) & (a[1] < b[4]) & (b[1] < a[4]) & (a[2] < b[5]) & (b[2] < a[5]);
   };
+  // the wave's buffer out (LDS operations of one wave are in order)
+  const auto write_out = [&]() {
+    const uint32_t list = piece++ % kLists;
+    uint2 *out = lists + (int64_t)list * capacity;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(counters + list * kCounterStride, (uint32_t)cnt);
+    base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+    __builtin_amdgcn_wave_barrier();
+    if (base > (uint32_t)capacity) full = true;   // the call falls back to the mask
+    for (int e = lane; e < cnt; e += 64)
+      if (base + (uint32_t)e < (uint32_t)capacity) out[base + e] = buf_l[wv][e];
+    __builtin_amdgcn_wave_barrier();
+    cnt = 0;
+  };
   // adds the pairs (a, b) of the lanes in `near` whose IoU is above thresh
   const auto add_pairs = [&](const Box &a, const Box &b, bool near) {
     if (__ballot(near) == 0) return;
@@ -491,17 +509,7 @@ __global__ __launch_bounds__(256) void nms3d_pair_kernel(const Box *__restrict__
       buf_l[wv][at] = make_uint2((uint32_t)min(a.rank, b.rank), (uint32_t)max(a.rank, b.rank));
     }
     cnt += __builtin_popcountll(m);
-    if (cnt > kPairBuf - 64) {   // the wave's buffer out (LDS operations of one wave are in order)
-      uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(counter, (uint32_t)cnt);
-      base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
-      __builtin_amdgcn_wave_barrier();
-      if (base > (uint32_t)capacity) full = true;   // the call falls back to the mask
-      for (int e = lane; e < cnt; e += 64)
-        if (base + (uint32_t)e < (uint32_t)capacity) out[base + e] = buf_l[wv][e];
-      __builtin_amdgcn_wave_barrier();
-      cnt = 0;
-    }
+    if (cnt > kPairBuf - 64) write_out();
   };
   if constexpr (PLACED) {
     __shared__ Box row_l[4][64], col_l[4][64];
@@ -562,10 +570,13 @@ __global__ __launch_bounds__(256) void nms3d_pair_kernel(const Box *__restrict__
   }
   if (lane == 0) cnt_l[wv] = cnt;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const int all = cnt_l[0] + cnt_l[1] + cnt_l[2] + cnt_l[3];
-    base_l = all ? (int)atomicAdd(counter, (uint32_t)all) : 0;
+  const int all = cnt_l[0] + cnt_l[1] + cnt_l[2] + cnt_l[3];
+  if (all > kPairBuf) {
+    if (cnt > 0) write_out();
+    return;
   }
+  uint2 *out = lists + (int64_t)first_list * capacity;
+  if (threadIdx.x == 0) base_l = all ? (int)atomicAdd(counters + first_list * kCounterStride, (uint32_t)all) : 0;
   __syncthreads();
   uint32_t base = (uint32_t)base_l;
   for (int w = 0; w < wv; ++w) base += (uint32_t)cnt_l[w];
@@ -698,7 +709,7 @@ struct PairLayout {
       at = (at + b + 255) & ~(size_t)255;
       return o;
     };
-    capacity = (int)((size_t)n * kPairsPerBox / kLists + 64);
+    capacity = (int)((size_t)n * kPairsPerBox / kLists + kPairBuf);
     sorted = take(nblk * 64 * sizeof(Box));
     counters = take(kLists * kCounterStride * 4);
     lists = take((size_t)kLists * capacity * sizeof(uint2));

@@ -222,3 +222,45 @@ def test_gpu_pairs_same_as_mask(gpu_device, kind, n, thr):
     if kind == "double":
         b, s = b.double(), s.double()
     assert _C.nms_3d(b, s, thr).cpu().tolist() == _mask_path(b, s, thr)
+
+
+def _pairs_path(boxes, scores, thr):
+    """ops3d_nms3d_pairs itself: the kept indices, or None where it gave up (num_keep = -1)."""
+    from ops3d_amd import _C
+
+    lib, n = _C._lib, boxes.shape[0]
+    order = None if lib.ops3d_nms3d_pairs_ranks(n) else torch.sort(scores, stable=True, descending=True)[1]
+    wsb = lib.ops3d_nms3d_pairs_workspace_bytes(n)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=boxes.device)
+    keep = torch.full((n,), -7, dtype=torch.long, device=boxes.device)
+    num = torch.full((1,), -7, dtype=torch.int32, device=boxes.device)
+    rc = lib.ops3d_nms3d_pairs(boxes.data_ptr(), boxes.stride(0), boxes.stride(1),
+                               None if order is not None else scores.data_ptr(), scores.stride(0),
+                               None if order is None else order.data_ptr(), n, thr, ws.data_ptr(), wsb,
+                               keep.data_ptr(), num.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    kept = int(num.item())
+    assert -1 <= kept <= n
+    return keep[:kept].cpu().tolist() if kept >= 0 else None
+
+
+def _clusters(n, m):
+    """Clusters of m boxes that overlap each other, far apart."""
+    r = np.random.default_rng(n)
+    c = (np.arange(n) % -(-n // m) * 100.0)[:, None] + r.uniform(-0.3, 0.3, (n, 3))
+    return np.concatenate([c - 5, c + 5], 1).astype(np.float32), r.uniform(size=n).astype(np.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m", [(64, 25), (64, 64), (128, 25), (128, 64), (300, 25), (1000, 25), (2000, 50)])
+def test_gpu_pairs_crowded_blocks(gpu_device, n, m):
+    """The pair path itself (no fallback to the mask behind it) holds the pairs of a few crowded blocks,
+    down to a call of a single one: they are spread over all lists."""
+    from fda_helpers import log
+
+    log(f"[case] nms3d pair path, clusters of {m} among {n}")
+    boxes, scores = _clusters(n, m)
+    b, s = torch.from_numpy(boxes).to(gpu_device), torch.from_numpy(scores).to(gpu_device)
+    got = _pairs_path(b, s, 0.3)
+    assert got is not None
+    assert got == _mask_path(b, s, 0.3)

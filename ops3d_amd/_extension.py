@@ -411,7 +411,7 @@ class _NativeFDA:
         wsb = self._lib.ops3d_nms3d_pairs_workspace_bytes(n) if thr >= 0.0 else 0
         ranked = self._lib.ops3d_nms3d_pairs_ranks(n)
         if wsb and (not ranked or scores.dtype in _DTYPE_CODE):
-            # from the list of overlapping pairs; -1 when they are too many or too long a chain
+            # from the list of overlapping pairs; -1 when they are too many
             b, s = dets.to(torch.float32), scores.to(torch.float32) if ranked else None
             if not ranked:
                 order = torch.sort(scores, stable=True, descending=True)[1]

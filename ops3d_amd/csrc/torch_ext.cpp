@@ -269,7 +269,7 @@ at::Tensor nms_3d(const at::Tensor &dets, const at::Tensor &scores, double thres
   const bool ranked = ops3d_nms3d_pairs_ranks(n) != 0;
   const auto sk = scores.scalar_type();
   if (pairs && (!ranked || sk == at::kFloat || sk == at::kHalf || sk == at::kBFloat16)) {
-    // from the list of overlapping pairs; -1 when they are too many or too long a chain
+    // from the list of overlapping pairs; -1 when they are too many
     const at::Tensor b = dets.to(at::kFloat), s = ranked ? scores.to(at::kFloat) : scores;
     if (!ranked) order = std::get<1>(scores.sort(/*stable=*/true, /*dim=*/0, /*descending=*/true));
     at::Tensor ws = at::empty({(int64_t)pairs}, dets.options().dtype(at::kByte));

@@ -264,3 +264,48 @@ def test_gpu_pairs_crowded_blocks(gpu_device, n, m):
     got = _pairs_path(b, s, 0.3)
     assert got is not None
     assert got == _mask_path(b, s, 0.3)
+
+
+def _row(n, reach, thr):
+    """Boxes in a row, each above the threshold with the next `reach`, scores falling along the row."""
+    lo = np.zeros((n, 3), np.float32)
+    lo[:, 0] = np.arange(n)
+    width = (reach + 0.5) * (1 + thr) / (1 - thr)
+    return np.concatenate([lo, lo + np.float32([width, 1, 1])], 1).astype(np.float32), -np.arange(n, dtype=np.float32)
+
+
+def _raster(shape):
+    """Boxes of edge 8 on a grid of step 2, equal scores: ranked in raster order."""
+    lo = np.stack(np.meshgrid(*[np.arange(k) for k in shape], indexing="ij"), -1).reshape(-1, 3) * np.float32(2)
+    return np.concatenate([lo, lo + 8], 1).astype(np.float32), np.ones(len(lo), np.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,n,arg", [
+    ("random", 1, 0.3), ("random", 64, 0.0), ("random", 4096, 0.1), ("random", 8192, 0.3), ("random", 8193, 0.3),
+    ("random", 1 << 18, 0.5), ("chain", 40, 0.2), ("chain", 3000, 0.2), ("chain", 10000, 0.2), ("row", 65, 3),
+    ("row", 2000, 25), ("row", 9000, 28), ("row", 20011, 12), ("raster", 0, (12, 12, 12)), ("raster", 0, (4, 4, 500)),
+    ("raster", 0, (25, 25, 25))])
+def test_gpu_pairs_take_chains(gpu_device, kind, n, arg):
+    """The pair path itself (no fallback to the mask behind it) decides independent scores and chains
+    of any length -- a row, equal scores in raster order -- with the mask path's list."""
+    from fda_helpers import log
+
+    log(f"[case] nms3d pair path {kind} n={n} {arg}")
+    thr = arg if kind in ("random", "chain") else 0.3
+    boxes, scores = {"random": lambda: _clustered(n, 5), "chain": lambda: _chain(n),
+                     "row": lambda: _row(n, arg, thr), "raster": lambda: _raster(arg)}[kind]()
+    b, s = torch.from_numpy(boxes).to(gpu_device), torch.from_numpy(scores).to(gpu_device)
+    got = _pairs_path(b, s, thr)
+    assert got is not None
+    assert got == _mask_path(b, s, thr)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [3000, 9001])
+def test_gpu_pairs_report_overflow(gpu_device, n):
+    """More overlapping pairs than the lists hold: the pair path says so and writes no list."""
+    r = np.random.default_rng(1)
+    lo = r.uniform(0, 1, (n, 3)).astype(np.float32)
+    b = torch.from_numpy(np.concatenate([lo, lo + 5], 1)).to(gpu_device)
+    assert _pairs_path(b, torch.rand(n, device=gpu_device), 0.2) is None

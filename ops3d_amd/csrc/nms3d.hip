@@ -588,6 +588,17 @@ __global__ __launch_bounds__(256) void nms3d_pair_kernel(const Box *__restrict__
     if (base + (uint32_t)e < (uint32_t)capacity) out[base + e] = buf_l[wv][e];
 }
 
+// Sum over the wave, on lane 63.
+__device__ __forceinline__ int wave_total(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, true);   // row_bcast 15, 31
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, true);
+  return v;
+}
+
 // The pairs resolved, in one workgroup: three bitmaps of the boxes (kept, removed, blocked) in LDS.
 //
 // Rounds first: a wave per list, which drops decided pairs by compacting its list in place.  At least
@@ -609,6 +620,7 @@ constexpr int kResolveThreads = 64 * kLists;
 // Costs in units of a pair read by a round (about 0.5 ns): a round besides its pairs, rounds per
 // inverse share of the boxes decided, the block pass, each of its blocks, each of its pairs.
 constexpr float kRoundCost = 2048.f, kRoundsPerShare = 8.f, kPassCost = 16384.f, kBlockCost = 3072.f, kSortCost = 2.5f;
+constexpr int kMarkPairs = 1024;   // of a list: fewer are not worth a loop of their own
 __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *lists, int capacity,
                                                                         const uint32_t *counters, uint2 *by_block, int n,
                                                                         const int64_t *order, int64_t *keep,
@@ -617,7 +629,7 @@ __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *l
   __shared__ uint32_t left_l[2], open_l[2], part_l[kLists], over_l;
   __shared__ uint32_t mask_l[2][64][2];
   __shared__ uint64_t gone_l;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int words = (n + 31) / 32;
   uint32_t *kept = bits_l, *removed = bits_l + words, *blocked = bits_l + 2 * words;
   for (int w = t; w < words; w += kResolveThreads) {
@@ -641,7 +653,7 @@ __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *l
   int cnt = (int)total;
   // undecided boxes that no undecided box precedes are kept; the pairs left in all lists and the
   // boxes left undecided
-  uint32_t more, open_boxes;
+  uint32_t more = 0, open_boxes = 0;
   const auto settle = [&](int round) {
     if (cnt && lane == 0) atomicAdd(&left_l[round & 1], (uint32_t)cnt);
     __syncthreads();
@@ -653,40 +665,39 @@ __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *l
       blocked[w] = 0;
       u += __builtin_popcount(open);
     }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) u += __shfl_xor(u, d);
-    if (u && lane == 0) atomicAdd(&open_l[round & 1], (uint32_t)u);
+    if (more && __ballot(u != 0) != 0) {
+      u = wave_total(u);
+      if (lane == 63) atomicAdd(&open_l[round & 1], (uint32_t)u);
+    }
     if (t == 0) left_l[(round & 1) ^ 1] = open_l[(round & 1) ^ 1] = 0;
     __syncthreads();
     open_boxes = open_l[round & 1];
   };
-  // the first round: nothing is decided yet, so every pair only blocks its second box
-  for (int e0 = 0; e0 < cnt; e0 += 64 * 8) {
-    uint32_t b[8];
-    bool seen[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int e = e0 + u * 64 + lane;
-      b[u] = e < cnt ? list[e].y : ~0u;
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) seen[u] = b[u] == ~0u || (blocked[b[u] >> 5] >> (b[u] & 31) & 1u);
-#pragma unroll
-    for (int u = 0; u < 8; ++u)   // (adds to one word wait for each other)
-      if (!seen[u]) atomicOr(&blocked[b[u] >> 5], 1u << (b[u] & 31));
-  }
-  settle(0);
   const auto pass_cost = [&]() {
     return kPassCost + kBlockCost * fminf((float)nblk, (float)more) + kSortCost * (float)more;
   };
-  const float first_pass = pass_cost();
-  float spent = 0.f, open2 = (float)n, open1 = (float)open_boxes;   // undecided two rounds ago and one
+  float first_pass = 0.f, spent = 0.f, open2 = (float)n, open1 = (float)n;   // undecided two rounds ago and one
   bool chains = false;
-  for (int round = 1; more; ++round) {
-    spent += kRoundCost + (float)more;
+  for (int round = 0;; ++round) {
     constexpr int U = 8;   // pairs per lane in flight
     int left = 0;
-    for (int e0 = 0; e0 < cnt; e0 += 64 * U) {
+    // the first round of a long list: nothing is decided yet, every pair only blocks its second box
+    const bool mark = round == 0 && cnt > kMarkPairs;
+    for (int e0 = 0; mark && e0 < cnt; e0 += 64 * U) {
+      uint32_t b[U];
+      bool seen[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = e0 + u * 64 + lane;
+        b[u] = e < cnt ? list[e].y : ~0u;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) seen[u] = b[u] == ~0u || (blocked[b[u] >> 5] >> (b[u] & 31) & 1u);
+#pragma unroll
+      for (int u = 0; u < U; ++u)   // (adds to one word wait for each other)
+        if (!seen[u]) atomicOr(&blocked[b[u] >> 5], 1u << (b[u] & 31));
+    }
+    for (int e0 = 0; !mark && e0 < cnt; e0 += 64 * U) {
       uint2 p[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -697,6 +708,7 @@ __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *l
       uint32_t gone[U], keep_a[U], seen[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
+        if (e0 + u * 64 >= cnt) break;
         const uint32_t a = p[u].x, b = p[u].y;
         gone[u] = (removed[a >> 5] >> (a & 31) | removed[b >> 5] >> (b & 31)) & 1u;
         keep_a[u] = kept[a >> 5] >> (a & 31) & 1u;
@@ -704,6 +716,7 @@ __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *l
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
+        if (e0 + u * 64 >= cnt) break;
         const uint32_t b = p[u].y, bb = 1u << (b & 31);
         bool open = p[u].x != b && !gone[u];
         if (open) {
@@ -717,10 +730,13 @@ __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *l
         left += __builtin_popcountll(m);
       }
     }
-    cnt = left;
+    if (!mark) cnt = left;
+    spent += kRoundCost + (float)more;
     settle(round);
+    if (!more) break;
+    if (round == 0) first_pass = pass_cost();
     const float share = (open2 - (float)open_boxes) / open2;   // decided by the last two rounds
-    chains = more != 0 && (spent > first_pass ||
+    chains = round > 0 && (spent > first_pass ||
                            (share < 0.25f && kRoundCost * kRoundsPerShare + 2.f * (float)more > pass_cost() * share));
     if (chains) break;
     open2 = open1;

@@ -47,7 +47,7 @@ OPS3D_FDA_API int ops3d_nms3d(const float *boxes_sorted, const int64_t *order, i
  *   order:     otherwise (scores not read) [n] int64, box indices by decreasing score;
  *   keep, num_keep: as above, but *num_keep = -1 when the boxes overlap too much for the list
  *              (more than about 32 pairs per box above the threshold): keep is then not written and
- *              the caller runs ops3d_nms3d.
+ *              the caller runs ops3d_nms3d_after_pairs.
  * The workspace (ops3d_nms3d_pairs_workspace_bytes) must be 32-byte aligned.
  */
 OPS3D_FDA_API size_t ops3d_nms3d_pairs_workspace_bytes(int n);
@@ -56,6 +56,15 @@ OPS3D_FDA_API int ops3d_nms3d_pairs(const float *boxes, int64_t box_stride, int6
                                     const float *scores, int64_t score_stride, const int64_t *order, int n,
                                     float iou_threshold, void *workspace, size_t workspace_bytes, int64_t *keep,
                                     int32_t *num_keep, void *stream);
+
+/*
+ * ops3d_nms3d on the boxes in score order that a call of ops3d_nms3d_pairs on the same stream left in
+ * its workspace, and on their order: the one given to that call, or NULL where it ranked the scores.
+ * The workspace is the mask's (ops3d_nms3d_workspace_bytes).
+ */
+OPS3D_FDA_API int ops3d_nms3d_after_pairs(const void *pairs_workspace, size_t pairs_workspace_bytes,
+                                          const int64_t *order, int n, float iou_threshold, void *workspace,
+                                          size_t workspace_bytes, int64_t *keep, int32_t *num_keep, void *stream);
 
 #ifdef __cplusplus
 }

@@ -51,6 +51,7 @@ EXPORTED_SYMBOLS = (
     "ops3d_nms3d_pairs_workspace_bytes",
     "ops3d_nms3d_pairs_ranks",
     "ops3d_nms3d_pairs",
+    "ops3d_nms3d_after_pairs",
     "ops3d_roi_align3d_forward",
     "ops3d_roi_align3d_backward_workspace_bytes",
     "ops3d_roi_align3d_backward",
@@ -107,6 +108,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.ops3d_nms3d_pairs_ranks.argtypes = [_i]
     lib.ops3d_nms3d_pairs.restype = _i
     lib.ops3d_nms3d_pairs.argtypes = [_vp, _i64, _i64, _vp, _i64, _vp, _i, ctypes.c_float, _vp, _sz, _vp, _vp, _vp]
+    lib.ops3d_nms3d_after_pairs.restype = _i
+    lib.ops3d_nms3d_after_pairs.argtypes = [_vp, _sz, _vp, _i, ctypes.c_float, _vp, _sz, _vp, _vp, _vp]
     lib.ops3d_roi_align3d_forward.restype = _i
     lib.ops3d_roi_align3d_forward.argtypes = [_vp] * 3 + [_i] * 10 + [ctypes.c_float, _i, _i, _vp]
     lib.ops3d_roi_align3d_backward_workspace_bytes.restype = _sz
@@ -407,32 +410,35 @@ class _NativeFDA:
         n, dev, thr = dets.shape[0], dets.device, float(threshold)
         keep = torch.empty(n, dtype=torch.long, device=dev)
         num = torch.empty(1, dtype=torch.int32, device=dev)
-        order = None
-        wsb = self._lib.ops3d_nms3d_pairs_workspace_bytes(n) if thr >= 0.0 else 0
+        wsb = self._lib.ops3d_nms3d_workspace_bytes(n)
+        pairs_wsb = self._lib.ops3d_nms3d_pairs_workspace_bytes(n) if thr >= 0.0 else 0
         ranked = self._lib.ops3d_nms3d_pairs_ranks(n)
-        if wsb and (not ranked or scores.dtype in _DTYPE_CODE):
+        if pairs_wsb and (not ranked or scores.dtype in _DTYPE_CODE):
             # from the list of overlapping pairs; -1 when they are too many
             b, s = dets.to(torch.float32), scores.to(torch.float32) if ranked else None
-            if not ranked:
-                order = torch.sort(scores, stable=True, descending=True)[1]
-            ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+            order = None if ranked else torch.sort(scores, stable=True, descending=True)[1]
+            pairs_ws = torch.empty(pairs_wsb, dtype=torch.uint8, device=dev)
             with torch.cuda.device(dev):
                 rc = self._lib.ops3d_nms3d_pairs(
                     b.data_ptr(), b.stride(0), b.stride(1), _ptr(s), s.stride(0) if ranked else 0, _ptr(order), n, thr,
-                    _ptr(ws), wsb, _ptr(keep), _ptr(num), torch.cuda.current_stream(dev).cuda_stream)
+                    _ptr(pairs_ws), pairs_wsb, _ptr(keep), _ptr(num), torch.cuda.current_stream(dev).cuda_stream)
             if rc != OPS3D_FDA_OK:
                 raise RuntimeError("nms_3d: kernel launch failed")
             kept = int(num.item())
             if kept >= 0:
                 return keep[:kept]
-        if order is None:
+            ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+            with torch.cuda.device(dev):
+                rc = self._lib.ops3d_nms3d_after_pairs(
+                    _ptr(pairs_ws), pairs_wsb, _ptr(order), n, thr, _ptr(ws), wsb, _ptr(keep), _ptr(num),
+                    torch.cuda.current_stream(dev).cuda_stream)
+        else:
             order = torch.sort(scores, stable=True, descending=True)[1]
-        boxes = dets.index_select(0, order).to(torch.float32).contiguous()
-        wsb = self._lib.ops3d_nms3d_workspace_bytes(n)
-        ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
-            rc = self._lib.ops3d_nms3d(_ptr(boxes), _ptr(order), n, thr, _ptr(ws), wsb, _ptr(keep), _ptr(num),
-                                       torch.cuda.current_stream(dev).cuda_stream)
+            boxes = dets.index_select(0, order).to(torch.float32).contiguous()
+            ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+            with torch.cuda.device(dev):
+                rc = self._lib.ops3d_nms3d(_ptr(boxes), _ptr(order), n, thr, _ptr(ws), wsb, _ptr(keep), _ptr(num),
+                                           torch.cuda.current_stream(dev).cuda_stream)
         if rc == OPS3D_FDA_EINVAL:
             raise ValueError("nms_3d: too many boxes (at most 2^19)")
         if rc != OPS3D_FDA_OK:

@@ -265,28 +265,32 @@ at::Tensor nms_3d(const at::Tensor &dets, const at::Tensor &scores, double thres
   at::Tensor keep = at::empty({n}, dets.options().dtype(at::kLong));
   at::Tensor num = at::empty({1}, dets.options().dtype(at::kInt));
   at::Tensor order;
-  const size_t pairs = thr >= 0.f ? ops3d_nms3d_pairs_workspace_bytes(n) : 0;
+  const size_t wsb = ops3d_nms3d_workspace_bytes(n), pairs = thr >= 0.f ? ops3d_nms3d_pairs_workspace_bytes(n) : 0;
   const bool ranked = ops3d_nms3d_pairs_ranks(n) != 0;
   const auto sk = scores.scalar_type();
+  int rc;
   if (pairs && (!ranked || sk == at::kFloat || sk == at::kHalf || sk == at::kBFloat16)) {
     // from the list of overlapping pairs; -1 when they are too many
     const at::Tensor b = dets.to(at::kFloat), s = ranked ? scores.to(at::kFloat) : scores;
     if (!ranked) order = std::get<1>(scores.sort(/*stable=*/true, /*dim=*/0, /*descending=*/true));
-    at::Tensor ws = at::empty({(int64_t)pairs}, dets.options().dtype(at::kByte));
-    const int rc = ops3d_nms3d_pairs(
-        b.data_ptr<float>(), b.stride(0), b.stride(1), ranked ? s.data_ptr<float>() : nullptr, ranked ? s.stride(0) : 0,
-        ranked ? nullptr : order.data_ptr<int64_t>(), n, thr, ws.data_ptr(), pairs, keep.data_ptr<int64_t>(),
-        num.data_ptr<int32_t>(), stream_of(dets));
+    const int64_t *ord = ranked ? nullptr : order.data_ptr<int64_t>();
+    at::Tensor pws = at::empty({(int64_t)pairs}, dets.options().dtype(at::kByte));
+    rc = ops3d_nms3d_pairs(b.data_ptr<float>(), b.stride(0), b.stride(1), ranked ? s.data_ptr<float>() : nullptr,
+                           ranked ? s.stride(0) : 0, ord, n, thr, pws.data_ptr(), pairs, keep.data_ptr<int64_t>(),
+                           num.data_ptr<int32_t>(), stream_of(dets));
     if (rc != OPS3D_FDA_OK) throw std::runtime_error("nms_3d: kernel launch failed");
     const int kept = num.item<int32_t>();
     if (kept >= 0) return keep.narrow(0, 0, kept);
+    at::Tensor ws = at::empty({(int64_t)wsb}, dets.options().dtype(at::kByte));
+    rc = ops3d_nms3d_after_pairs(pws.data_ptr(), pairs, ord, n, thr, ws.data_ptr(), wsb, keep.data_ptr<int64_t>(),
+                                 num.data_ptr<int32_t>(), stream_of(dets));
+  } else {
+    order = std::get<1>(scores.sort(/*stable=*/true, /*dim=*/0, /*descending=*/true));
+    const at::Tensor boxes = dets.index_select(0, order).to(at::kFloat).contiguous();
+    at::Tensor ws = at::empty({(int64_t)wsb}, dets.options().dtype(at::kByte));
+    rc = ops3d_nms3d(boxes.data_ptr<float>(), order.data_ptr<int64_t>(), n, thr, ws.data_ptr(), wsb,
+                     keep.data_ptr<int64_t>(), num.data_ptr<int32_t>(), stream_of(dets));
   }
-  if (!order.defined()) order = std::get<1>(scores.sort(/*stable=*/true, /*dim=*/0, /*descending=*/true));
-  const at::Tensor boxes = dets.index_select(0, order).to(at::kFloat).contiguous();
-  const size_t wsb = ops3d_nms3d_workspace_bytes(n);
-  at::Tensor ws = at::empty({(int64_t)wsb}, dets.options().dtype(at::kByte));
-  const int rc = ops3d_nms3d(boxes.data_ptr<float>(), order.data_ptr<int64_t>(), n, thr, ws.data_ptr(), wsb,
-                             keep.data_ptr<int64_t>(), num.data_ptr<int32_t>(), stream_of(dets));
   if (rc == OPS3D_FDA_EINVAL) throw std::invalid_argument("nms_3d: too many boxes (at most 2^19)");
   if (rc != OPS3D_FDA_OK) throw std::runtime_error("nms_3d: kernel launch failed");
   return keep.narrow(0, 0, num.item<int32_t>());

@@ -302,10 +302,26 @@ def test_gpu_pairs_take_chains(gpu_device, kind, n, arg):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [3000, 9001])
-def test_gpu_pairs_report_overflow(gpu_device, n):
-    """More overlapping pairs than the lists hold: the pair path says so and writes no list."""
-    r = np.random.default_rng(1)
+@pytest.mark.parametrize("n", [300, 3000, 9001])
+def test_gpu_mask_after_pairs(gpu_device, n):
+    """More overlapping pairs than the lists hold: the pair path says so, and the mask path that goes on
+    from its workspace (boxes and order) gives the mask path's list."""
+    from ops3d_amd import _C
+
+    lib, r = _C._lib, np.random.default_rng(1)
     lo = r.uniform(0, 1, (n, 3)).astype(np.float32)
-    b = torch.from_numpy(np.concatenate([lo, lo + 5], 1)).to(gpu_device)
-    assert _pairs_path(b, torch.rand(n, device=gpu_device), 0.2) is None
+    b = torch.from_numpy(np.concatenate([lo, lo + r.uniform(3, 5, (n, 3)).astype(np.float32)], 1)).to(gpu_device)
+    s = torch.rand(n, device=gpu_device)
+    order = None if lib.ops3d_nms3d_pairs_ranks(n) else torch.sort(s, stable=True, descending=True)[1]
+    op = None if order is None else order.data_ptr()
+    sizes = lib.ops3d_nms3d_pairs_workspace_bytes(n), lib.ops3d_nms3d_workspace_bytes(n)
+    pws, ws = (torch.empty(v, dtype=torch.uint8, device=gpu_device) for v in sizes)
+    keep = torch.empty(n, dtype=torch.long, device=gpu_device)
+    num = torch.empty(1, dtype=torch.int32, device=gpu_device)
+    st = torch.cuda.current_stream().cuda_stream
+    out = (keep.data_ptr(), num.data_ptr(), st)
+    assert lib.ops3d_nms3d_pairs(b.data_ptr(), 6, 1, None if op else s.data_ptr(), 1, op, n, 0.2, pws.data_ptr(), sizes[0],
+                                 *out) == 0
+    assert int(num.item()) == -1
+    assert lib.ops3d_nms3d_after_pairs(pws.data_ptr(), sizes[0], op, n, 0.2, ws.data_ptr(), sizes[1], *out) == 0
+    assert keep[: int(num.item())].cpu().tolist() == _mask_path(b, s, 0.2)

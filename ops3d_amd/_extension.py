@@ -415,7 +415,9 @@ class _NativeFDA:
         ranked = self._lib.ops3d_nms3d_pairs_ranks(n)
         if pairs_wsb and (not ranked or scores.dtype in _DTYPE_CODE):
             # from the list of overlapping pairs; -1 when they are too many
-            b, s = dets.to(torch.float32), scores.to(torch.float32) if ranked else None
+            # (resolve_neg: the imaginary part of a conjugate is a view whose memory holds the negatives)
+            b = dets.to(torch.float32).resolve_neg()
+            s = scores.to(torch.float32).resolve_neg() if ranked else None
             order = None if ranked else torch.sort(scores, stable=True, descending=True)[1]
             pairs_ws = torch.empty(pairs_wsb, dtype=torch.uint8, device=dev)
             with torch.cuda.device(dev):

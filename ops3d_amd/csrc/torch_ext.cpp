@@ -271,7 +271,8 @@ at::Tensor nms_3d(const at::Tensor &dets, const at::Tensor &scores, double thres
   int rc;
   if (pairs && (!ranked || sk == at::kFloat || sk == at::kHalf || sk == at::kBFloat16)) {
     // from the list of overlapping pairs; -1 when they are too many
-    const at::Tensor b = dets.to(at::kFloat), s = ranked ? scores.to(at::kFloat) : scores;
+    // (resolve_neg: the imaginary part of a conjugate is a view whose memory holds the negatives)
+    const at::Tensor b = dets.to(at::kFloat).resolve_neg(), s = ranked ? scores.to(at::kFloat).resolve_neg() : scores;
     if (!ranked) order = std::get<1>(scores.sort(/*stable=*/true, /*dim=*/0, /*descending=*/true));
     const int64_t *ord = ranked ? nullptr : order.data_ptr<int64_t>();
     at::Tensor pws = at::empty({(int64_t)pairs}, dets.options().dtype(at::kByte));

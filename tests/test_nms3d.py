@@ -325,3 +325,25 @@ def test_gpu_mask_after_pairs(gpu_device, n):
     assert int(num.item()) == -1
     assert lib.ops3d_nms3d_after_pairs(pws.data_ptr(), sizes[0], op, n, 0.2, ws.data_ptr(), sizes[1], *out) == 0
     assert keep[: int(num.item())].cpu().tolist() == _mask_path(b, s, 0.2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [500, 9000])
+def test_gpu_negated_views(gpu_device, n):
+    """Boxes and scores that are negated views (the imaginary part of a conjugate), through both
+    modules: the values count, not what lies in memory."""
+    import importlib
+
+    from ops3d_amd import _C
+
+    boxes, scores = _clustered(n, 4)
+    want = O.nms3d(boxes, scores, 0.3).tolist()
+
+    def view(a):
+        t = torch.from_numpy(a).to(gpu_device)
+        v = torch.complex(t, -t).conj().imag
+        assert v.is_neg() and torch.equal(v, t)
+        return v
+
+    for module in (_C, importlib.import_module("ops3d_amd._fda_torch")):
+        assert module.nms_3d(view(boxes), view(scores), 0.3).cpu().tolist() == want

@@ -37,7 +37,6 @@ constexpr int kBlocksPerHead = 64;
 // and in one whose heads alone occupy half the CUs (one_block_per_head()).
 constexpr uint32_t kFusedHeadSamples = 4096, kFusedFewHeads = 5120, kFusedManyHeads = 32768;
 constexpr uint32_t kFusedHeads = 128;                 // heads of a call that count as many
-constexpr uint32_t kFusedTcap = 16 * kWin;            // 2^21 voxels: kWin tiles of 256
 
 struct BucketArgs {
   const uint32_t *keys;        // [N] tile_key of each sample or kKeyInvalid
@@ -477,11 +476,17 @@ size_t tile_matrix_words(uint32_t BG, uint32_t tcap) { return (size_t)BG * kBloc
 //   128 heads   8192: 151 / 161, 344 / 371      32768: 478 / 500, 601 / 658
 //   256 heads   8192: 233 / 267, 672 / 739      16384: 438 / 501, 859 / 967
 // (the host saves 5 us of its 20 per call in each of them), and over the 32x64x256 .. 8x16x64
-// levels, bf16, 128 heads of 16 channels: 5120: 2654 / 2706, 32768: 2342 / 2500.  Volumes that can
-// pass the LDS window (atomic mode) keep the lower bound: not measured beyond it.
-inline bool one_block_per_head(uint32_t per_head, uint32_t heads, uint32_t tcap) {
+// levels, bf16, 128 heads of 16 channels: 5120: 2654 / 2706, 32768: 2342 / 2500.  The line for few
+// heads lies where the GPU time alone is level, 5 whole steps of kBucketThreads samples: the host's
+// 5 us count only in a program that waits for it.  Volumes whose nominal tiles pass the LDS window
+// (atomic mode) keep the lower bound; there, as for thin levels, whose tiles are narrower than the
+// nominal ones and pass the window earlier (their shapes are on the device), the two are level:
+// 96x128x128, 64 bf16 channels, 8 heads of 4608 samples 679 / 679, 128 of 8192 11370 / 11350;
+// 1x1x66000, 32 channels, 8 of 4608 207 / 204, 128 of 8192 2564 / 2582, of 32768 3806 / 3811;
+// 1x300x300 and half, 128 of 8192 1836 / 1903.
+inline bool one_block_per_head(uint32_t per_head, uint32_t heads, uint32_t tcap, uint32_t tile_voxels) {
   if (per_head <= kFusedHeadSamples) return true;
-  if (tcap > kFusedTcap) return false;
+  if ((uint64_t)(tcap - 64) * 16 > (uint64_t)kWin * tile_voxels) return false;   // S > kWin whole tiles
   return per_head <= (heads >= kFusedHeads ? kFusedManyHeads : kFusedFewHeads);
 }
 
@@ -501,7 +506,7 @@ hipError_t launch_tile_bucketing(const uint32_t *keys, uint32_t n, uint32_t per_
   a.chunk = (a.chunk + kBucketThreads - 1) / kBucketThreads * kBucketThreads;
   if (a.chunk == 0) a.chunk = kBucketThreads;
   // small heads: one block per head that counts, scans and scatters in one launch
-  a.fused = n > 0 && one_block_per_head(per_head, (uint32_t)BG, tcap);
+  a.fused = n > 0 && one_block_per_head(per_head, (uint32_t)BG, tcap, (uint32_t)(TX * TY * TZ));
   if (a.fused) a.chunk = (per_head + kBucketThreads - 1) / kBucketThreads * kBucketThreads;
   a.blocks_per_head = (per_head + a.chunk - 1) / a.chunk;
   if (n == 0) a.blocks_per_head = 0;   // every counter is zero: the head scan writes zeros

@@ -588,11 +588,14 @@ __global__ __launch_bounds__(256) void roi_axis_table_kernel(const T *rois, floa
 // contiguous run: read in 16-byte pieces into LDS as they lie (at the run's alignment), written a
 // bin at a time, a lane per channel.  Also marks rois that hold an infinity or NaN.
 template <typename T> constexpr int kCopyChannels = sizeof(T) == 4 ? 32 : 64;   // at most 48 KB of LDS
-template <typename T>
+// Fewer channels where the call would have fewer blocks than the chip CUs: 2 to 6 us of a call of 9 to
+// 35 rois over 64 to 256 channels.
+constexpr int kCopyFewChannels = 16, kCopyFewBlocks = 256;
+template <typename T, int CB>
 __global__ __launch_bounds__(256) void grad_channels_last_kernel(const T *top, T *top_cl, uint32_t *tr, int C, int bins,
                                                                  int ntz, int R) {
   extern __shared__ __align__(16) unsigned char copy_lds[];
-  constexpr int E = 16 / (int)sizeof(T), CB = kCopyChannels<T>;
+  constexpr int E = 16 / (int)sizeof(T);
   T *l = reinterpret_cast<T *>(copy_lds);
   const int t = threadIdx.x, r = blockIdx.x, c0 = blockIdx.y * CB, nc = min(CB, C - c0);
   const T *src = top + ((int64_t)r * C + c0) * bins;
@@ -676,8 +679,12 @@ __global__ __launch_bounds__(1024) void roi_tile_order_kernel(const uint8_t *cou
   __syncthreads();
   for (int i = t; i < tiles; i += 1024) order[atomicAdd(&at_l[255 - counts[i]], 1u)] = (unsigned short)i;
 }
-constexpr int kGUnordered = 8192;                // waves whose order is no matter: twice what runs at once
-constexpr int kGSplitBlocks = 1024, kGSplitRois = 8;
+// How a gather is launched, by its blocks (a wave per tile and 64 channels), the rois R and the tiles
+// (figures: at backward()).
+constexpr int kGSplitBlocks = 4096, kGSplitRois = 16;   // up to so many blocks, from so many rois: SPLIT
+constexpr int kGClearRois = 27;                  // R * 27 <= tiles: most tiles are empty, clear_tiles()
+constexpr int kGUnordered = 8192, kGOrderRois = 12;     // more blocks, R * 12 > tiles: crowded tiles first
+constexpr int kGNotCleared = 0x7fffffff;
 constexpr int kGOrdered = 65535;                 // tiles that are ordered (16-bit numbers)
 constexpr int kGList = 192;                      // rois listed at a time
 
@@ -691,21 +698,70 @@ __device__ __forceinline__ RawOf<T> load_raw(__amdgpu_buffer_rsrc_t rs, uint32_t
     return __builtin_amdgcn_raw_buffer_load_b16(rs, (int)voff, (int)soff, 0);
 }
 
+// Zeros for the tiles that no roi reaches (the waves of those tiles then store nothing): a block per
+// row of tiles along x and kGClearChannels channels, 4 voxels per thread with the lanes along x.
+constexpr int kGClearWords = 8, kGClearChannels = 8;   // 256 tiles at a time
+template <typename T, int NT>
+__device__ __forceinline__ void clear_tiles(int blk, uint32_t *reached_l, const T *__restrict__ rois,
+                                            const uint32_t *__restrict__ tr, T *__restrict__ grad, int C, int D, int H,
+                                            int W, int R) {
+  const int t = threadIdx.x, ntz = tiles_of(D), nty = tiles_of(H), ntx = tiles_of(W);
+  const int parts = (C + kGClearChannels - 1) / kGClearChannels, c0 = blk % parts * kGClearChannels;
+  const int ty = blk / parts % nty, tz = blk / parts / nty % ntz, n = blk / parts / nty / ntz;
+  const int nc = min(kGClearChannels, C - c0);
+  for (int tx0 = 0; tx0 < ntx; tx0 += 32 * kGClearWords) {
+    const int nt = min(32 * kGClearWords, ntx - tx0);
+    if (t < kGClearWords) reached_l[t] = 0;
+    __syncthreads();
+    for (int i = t; i < R * 4; i += NT) {   // four threads per roi
+      const int r = i >> 2;
+      const uint32_t z = tr[(size_t)tz * R + r], y = tr[(size_t)(ntz + ty) * R + r];
+      if ((int)to_f(rois[(int64_t)r * 7]) != n || first_bin(z) > last_bin(z) || first_bin(y) > last_bin(y)) continue;
+      for (int k = i & 3; k < nt; k += 4) {
+        const uint32_t x = tr[(size_t)(ntz + nty + tx0 + k) * R + r];
+        if (first_bin(x) <= last_bin(x)) atomicOr(&reached_l[k >> 5], 1u << (k & 31));
+      }
+    }
+    __syncthreads();
+    for (int k0 = 0; k0 < nt; k0 += NT) {
+      // threads in rows of the next power of two above the tiles
+      const int m = min(NT, nt - k0), shift = m > 1 ? 32 - __clz(m - 1) : 0, kk = t & ((1 << shift) - 1), k = k0 + kk;
+      if (kk >= m || ((reached_l[k >> 5] >> (k & 31)) & 1u)) continue;
+      const int x0 = (tx0 + k) * kGT;
+      for (int row = t >> shift; row < nc * kGT * kGT; row += NT >> shift) {
+        const int c = c0 + row / (kGT * kGT), z = tz * kGT + row / kGT % kGT, y = ty * kGT + row % kGT;
+        if (z >= D || y >= H) continue;
+        T *o = grad + ((((int64_t)n * C + c) * D + z) * H + y) * W + x0;
+        if (x0 + kGT <= W) {   // at any alignment
+          const uint32_t zero[kGT * sizeof(T) / 4] = {};
+          __builtin_memcpy(o, zero, sizeof(zero));
+        } else {
+          for (int x = 0; x < W - x0; ++x) o[x] = from_f<T>(0.f);
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // SPLIT: a block of kGSplit waves per tile and channel group, each taking every kGSplit-th roi; their
-// sums are added in LDS, wave w those of plane w (launched where the tiles alone leave most of the
-// chip idle).
+// sums are added in LDS, two planes at a time, wave w those of plane w (launched where a tile's chain
+// of rois is the time: few tiles, which run at once or nearly).  Blocks from clear_from on are
+// clear_tiles()'s, behind the tiles' since those end with the few crowded ones.
 constexpr int kGSplit = 4;
 template <typename T, bool SPLIT>
-__global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, SPLIT ? 2 : 4) void roi_align3d_backward_gather_kernel(
+__global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, 4) void roi_align3d_backward_gather_kernel(
     const T *__restrict__ top_cl, const T *__restrict__ rois, T *__restrict__ grad, const float *__restrict__ wt,
     const uint32_t *__restrict__ tr, const unsigned short *__restrict__ order, int N, int C, int D, int H,
-    int W, int R, int PD, int PH, int PW, int blocks, int run) {
+    int W, int R, int PD, int PH, int PW, int blocks, int run, int clear_from) {
   constexpr int NW = SPLIT ? kGSplit : 1;
   static_assert(!SPLIT || kGSplit == kGT, "a wave per plane of the tile");
-  __shared__ uint4 lists_l[NW][kGList];
-  __shared__ float sums_l[SPLIT ? kGSplit : 1][SPLIT ? kGT * kGT * kGT : 1][64];
+  // the rois' lists; with SPLIT then the waves' sums of two planes (32 KB: four blocks per CU)
+  constexpr int kSums = 2 * kGT * kGT;
+  __shared__ uint4 lds_l[SPLIT ? NW * kSums * 64 / 4 : kGList];
+  static_assert(!SPLIT || NW * kGList <= NW * kSums * 64 / 4, "the lists fit");
   const int lane = threadIdx.x & 63, wave = SPLIT ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
-  uint4 *const list_l = lists_l[wave];
+  uint4 *const list_l = lds_l + wave * kGList;
   const int ntz = tiles_of(D), nty = tiles_of(H), ntx = tiles_of(W);
   const int ncg = (C + 63) / 64;
   // Tiles differ several times over in the rois that they meet, so a block is one wave (a larger one
@@ -714,6 +770,10 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, SPLIT ? 2 : 4) void roi_
   // the same rois' bins, and which run of a round of eight it takes moves on, so that no XCD gets
   // only the crowded middle of the volume.
   int bid = blockIdx.x, cg;
+  if (bid >= clear_from) {
+    clear_tiles<T, 64 * NW>(bid - clear_from, reinterpret_cast<uint32_t *>(lds_l), rois, tr, grad, C, D, H, W, R);
+    return;
+  }
   if (order) {
     if (bid >= blocks) return;
     cg = bid % ncg;
@@ -799,6 +859,7 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, SPLIT ? 2 : 4) void roi_
     for (int k = 0; k < 4; ++k) off[k] = (uint32_t)min(k, nx - 1) * bin_bytes + cl_bytes;
   };
 
+  bool reached = false;
   for (int r0 = 0; r0 * NW + wave < R;) {
     // the next rois of batch item n that reach the tile, in index order: from the front those with
     // at most 4 bins on every axis of it and only finite values (nearly all), from the back the
@@ -817,6 +878,7 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, SPLIT ? 2 : 4) void roi_
       wide += __popcll(mw);
     }
     __builtin_amdgcn_wave_barrier();
+    reached = reached || narrow + wide > 0;
 
     if (narrow > 0) {
       take(0);
@@ -915,28 +977,35 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, SPLIT ? 2 : 4) void roi_
           for (int j = 0; j < kGT * kGT; ++j) u[j] = 0.f;
           const char *plane = reinterpret_cast<const char *>(top_cl) +
                               ((uint64_t)(uint32_t)roi * roi_bytes + ((uint32_t)pd * plane_bytes + (uint32_t)px * bin_bytes));
-          for (int ph = first_bin(b_zy >> 16); ph <= last_bin(b_zy >> 16); ++ph) {
-            load_row(v[0], plane, ph, off);
-            float g[4], t[kGT];
+          const int last_ph = last_bin(b_zy >> 16);
+          for (int ph0 = first_bin(b_zy >> 16); ph0 <= last_ph; ph0 += 4) {   // four rows in flight
 #pragma unroll
-            for (int k = 0; k < 4; ++k) g[k] = to_f(__builtin_bit_cast(T, v[0][k]));
-            if (clean) {
-              x_sum(t, wxr, g, nx);
-            } else {   // 0 * infinity must not reach a voxel outside the bin
+            for (int h = 0; h < 4; ++h) load_row(v[h], plane, min(ph0 + h, last_ph), off);
 #pragma unroll
-              for (int x = 0; x < kGT; ++x) t[x] = 0.f;
+            for (int h = 0; h < 4; ++h) {
+              const int ph = ph0 + h;
+              if (ph > last_ph) break;
+              float g[4], t[kGT];
 #pragma unroll
-              for (int k = 0; k < 4; ++k)
+              for (int k = 0; k < 4; ++k) g[k] = to_f(__builtin_bit_cast(T, v[h][k]));
+              if (clean) {
+                x_sum(t, wxr, g, nx);
+              } else {   // 0 * infinity must not reach a voxel outside the bin
 #pragma unroll
-                for (int x = 0; x < kGT; ++x)
-                  if (nonzero(wxr[k][x])) t[x] += wxr[k][x] * g[k];
-            }
+                for (int x = 0; x < kGT; ++x) t[x] = 0.f;
 #pragma unroll
-            for (int y = 0; y < kGT; ++y) {
-              const float w = wy[ph * H + y];
-              if (nonzero(w))
+                for (int k = 0; k < 4; ++k)
 #pragma unroll
-                for (int x = 0; x < kGT; ++x) u[y * kGT + x] += w * t[x];
+                  for (int x = 0; x < kGT; ++x)
+                    if (nonzero(wxr[k][x])) t[x] += wxr[k][x] * g[k];
+              }
+#pragma unroll
+              for (int y = 0; y < kGT; ++y) {
+                const float w = wy[ph * H + y];
+                if (nonzero(w))
+#pragma unroll
+                  for (int x = 0; x < kGT; ++x) u[y * kGT + x] += w * t[x];
+              }
             }
           }
 #pragma unroll
@@ -951,20 +1020,31 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, SPLIT ? 2 : 4) void roi_
     }
     __builtin_amdgcn_wave_barrier();   // the list is read before the next rois are written to it
   }
+  // nothing to store where the zeros come from clear_tiles(), no sums to add where there are none
+  const bool any = (SPLIT ? __syncthreads_or(reached) != 0 : reached) || clear_from == kGNotCleared;
   if constexpr (SPLIT) {   // wave w: the sums of plane w, in acc[0]
+    if (any) {
+      float(*sums_l)[kSums][64] = reinterpret_cast<float(*)[kSums][64]>(lds_l);
+      float sum[kGT * kGT];
 #pragma unroll
-    for (int z = 0; z < kGT; ++z)
+      for (int half = 0; half < 2; ++half) {
+        __syncthreads();
 #pragma unroll
-      for (int j = 0; j < kGT * kGT; ++j) sums_l[wave][z * kGT * kGT + j][lane] = acc[z][j];
-    __syncthreads();
+        for (int j = 0; j < kSums; ++j) sums_l[wave][j][lane] = acc[2 * half + j / (kGT * kGT)][j % (kGT * kGT)];
+        __syncthreads();
+        if (wave >> 1 == half)
 #pragma unroll
-    for (int j = 0; j < kGT * kGT; ++j) {
-      acc[0][j] = sums_l[0][wave * kGT * kGT + j][lane];
+          for (int j = 0; j < kGT * kGT; ++j) {
+            sum[j] = sums_l[0][(wave & 1) * kGT * kGT + j][lane];
 #pragma unroll
-      for (int k = 1; k < NW; ++k) acc[0][j] += sums_l[k][wave * kGT * kGT + j][lane];
+            for (int k = 1; k < NW; ++k) sum[j] += sums_l[k][(wave & 1) * kGT * kGT + j][lane];
+          }
+      }
+#pragma unroll
+      for (int j = 0; j < kGT * kGT; ++j) acc[0][j] = sum[j];
     }
   }
-  if (c >= C) return;
+  if (c >= C || !any) return;
   T *o = grad + ((int64_t)n * C + c) * D * H * W;
 #pragma unroll
   for (int z = 0; z < (SPLIT ? 1 : kGT); ++z)
@@ -1296,16 +1376,25 @@ inline size_t gather_tables_bytes(int R, int D, int H, int W, int PD, int PH, in
 // 340 K visits of a roi to a tile and channel group, each 2 to 4 planes of 4 rows.  Steps: the first
 // form (blocks of four waves, dynamic loops, weights by scalar loads) 943 us; rows loaded a plane
 // ahead and weights fetched by the lanes 680; one wave per block 537; crowded tiles first 500 (-45);
-// no spilled registers 445.  Without `order` an XCD's runs of 8 / 32 / 128 / 512 tiles measured
-// 554 / 535 / 522 / 540 us.  Launches of few waves are not ordered (the two passes cost 10 us).  With few waves the rois' serial chain is the time: four
-// waves per tile, each with a quarter of the rois, up to kGSplitBlocks blocks (forward and backward,
-// split / not: 17x24x28, 404 rois, 32 channels 264 / 639 us; 26x35x31, 21 rois, 64 channels 74 / 102;
-// 10x23x65, 213 rois, 256 channels (2448 blocks) 96 / 92; 13x25x50, 160 rois, nearest 80 / 48).
-// Stores of 4 voxels at any alignment: W = 50, 35 rois 320 -> 249 us.  Slower than the voxel threads
-// before it: few rois over many channels of a large volume, where the 4-voxel stores, which take
-// about 0.2 ms per 105 MB of gradient, are the time (64 rois of 4-16 voxels 330 / 285, 35 nearest rois
-// over [2, 256, 41, 50, 50] 249 / 187).  Joining the tiles of a block of two or four waves in LDS, to store
-// longer runs, 502 / 520 us against 492; three waves per SIMD 542.
+// no spilled registers 445, four rows at a time where bins are smaller than voxels 435.  Without
+// `order` an XCD's runs of 8 / 32 / 128 / 512 tiles measured 554 / 535 / 522 / 540 us.  Joining the
+// tiles of a block of two or four waves in LDS, to store longer runs, 502 / 520 us against 492; three
+// waves per SIMD 542.
+// The rules of a launch, by the GPU time of all passes of a call (us; 7^3 bins, 2 samples, rois of
+// 4-32 voxels where not said; f: fp32, others 16 bits; "N x" batch items):
+//   SPLIT / one wave per tile: 17x24x28, 32 channels, 404 rois of 4-16 (252 blocks) 357 / 1119;
+//     26x35x31, 64, 21 of 4-16 (504) 49 / 59; 12x40x40, 200, 90 of 4-24, 3^3 bins (1200) 39 / 60;
+//     10x23x65, 256, 213 of 4-16 (1224) 199 / 411; 30x60x60 f, 32, 60 (1800) 58 / 68; 24x48x48, 256,
+//     300 of 4-24 (3456) 260 / 322, 30 rois 82 / 77; 32x64x64, 192, 200 rois, 5^3 (6144) 132 / 130.
+//     Four blocks per CU: with 64 KB of sums, two, 213 rois took 267 and 21 rois 53.
+//   clear_tiles() / every wave stores: 2 x 32x64x64, 256, 64 rois of 4-16 (4096 tiles) 135 / 180; 110 of
+//     4-16 158 / 193; 150 of 4-32 212 / 215; f, 16 rois 127 / 211; 2 x 41x50x50, 256, 35 of 4-16, one
+//     sample, nearest (3718) 83 / 123, of 4-32 113 / 131; 24x48x48, 256, 9 rois (864) 50 / 51.  The
+//     stores of 4 voxels take 0.1 to 0.2 ms per 100 MB of gradient, a clear about 30 us, most of it
+//     beside the crowded tiles' chains.  As a pass of its own before the gather 64 rois took 141.
+//   Crowded tiles first / in place: 2 x 32x64x64, 256, 512 rois 430 / 459, 400 rois 372 / 371, 300
+//     rois 321 / 288, 220 rois 292 / 248; 2 x 40x80x80, 512 rois (8000 tiles) 648 / 610, 300 rois
+//     521 / 425: the neighbours' stores then meet in no L2.
 template <typename T>
 int backward(const void *grad_output, const void *rois, void *grad_input, float *acc, int N, int C, int D, int H,
              int W, int R, int PD, int PH, int PW, float scale, int sr, int order, hipStream_t st) {
@@ -1323,15 +1412,22 @@ int backward(const void *grad_output, const void *rois, void *grad_input, float 
     if (R > 0) {
       hipLaunchKernelGGL((roi_axis_table_kernel<T>), dim3((unsigned)R, 3), dim3(256), 0, st,
                          static_cast<const T *>(rois), wt, tr, D, H, W, PD, PH, PW, R, scale, sr, order);
+      const auto copy = [&](auto kern, int cb) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)R, (unsigned)((C + cb - 1) / cb)), dim3(256),
+                           ((size_t)cb * bins + 16 / sizeof(T)) * sizeof(T), st, static_cast<const T *>(grad_output),
+                           top_cl, tr, C, bins, ntz, R);
+      };
       constexpr int CB = kCopyChannels<T>;
-      const size_t lds = ((size_t)CB * bins + 16 / sizeof(T)) * sizeof(T);
-      hipLaunchKernelGGL((grad_channels_last_kernel<T>), dim3((unsigned)R, (unsigned)((C + CB - 1) / CB)), dim3(256), lds,
-                         st, static_cast<const T *>(grad_output), top_cl, tr, C, bins, tiles_of(D), R);
+      if ((int64_t)R * ((C + CB - 1) / CB) < kCopyFewBlocks) copy(grad_channels_last_kernel<T, kCopyFewChannels>, kCopyFewChannels);
+      else copy(grad_channels_last_kernel<T, CB>, CB);
     }
     // the tiles' order, in the tables' second part beyond the words that tr takes, where it fits
     const int64_t used = (int64_t)R * (ntz + nty + ntx) * 4, spare = (int64_t)R * (D + H + W) * 4 - used;
     unsigned short *order = nullptr;
-    if (blocks > kGUnordered && tiles <= kGOrdered && tiles * 3 <= spare) {
+    const bool split = blocks <= kGSplitBlocks && R >= kGSplitRois;
+    const int64_t clears = (int64_t)N * ntz * nty * ((C + kGClearChannels - 1) / kGClearChannels);
+    const bool cleared = (int64_t)R * kGClearRois <= tiles && grid + clears < (1 << 24);
+    if (blocks > kGUnordered && (int64_t)R * kGOrderRois > tiles && tiles <= kGOrdered && tiles * 3 <= spare) {
       order = reinterpret_cast<unsigned short *>(reinterpret_cast<char *>(tr) + used);
       uint8_t *counts = reinterpret_cast<uint8_t *>(order + tiles);
       hipLaunchKernelGGL((roi_tile_count_kernel<T>), dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, st,
@@ -1339,11 +1435,11 @@ int backward(const void *grad_output, const void *rois, void *grad_input, float 
       hipLaunchKernelGGL(roi_tile_order_kernel, dim3(1), dim3(1024), 0, st, counts, order, (int)tiles);
     }
     const auto gather = [&](auto kern, int threads) {
-      hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), 0, st, top_cl, static_cast<const T *>(rois),
-                         static_cast<T *>(grad_input), wt, tr, order, N, C, D, H, W, R, PD, PH, PW, (int)blocks,
-                         (int)run);
+      hipLaunchKernelGGL(kern, dim3((unsigned)(grid + (cleared ? clears : 0))), dim3(threads), 0, st, top_cl,
+                         static_cast<const T *>(rois), static_cast<T *>(grad_input), wt, tr, order, N, C, D, H, W, R, PD,
+                         PH, PW, (int)blocks, (int)run, cleared ? (int)grid : kGNotCleared);
     };
-    if (blocks <= kGSplitBlocks && R >= kGSplitRois) gather(roi_align3d_backward_gather_kernel<T, true>, 64 * kGSplit);
+    if (split) gather(roi_align3d_backward_gather_kernel<T, true>, 64 * kGSplit);
     else gather(roi_align3d_backward_gather_kernel<T, false>, 64);
     return hipGetLastError() == hipSuccess ? OPS3D_FDA_OK : OPS3D_FDA_ERUNTIME;
   }

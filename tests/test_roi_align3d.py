@@ -339,9 +339,9 @@ def test_gpu_channels_last_through_the_op(gpu_device):
 
 @pytest.mark.gpu
 def test_gpu_backward_more_rois_than_one_grid_dimension(gpu_device):
-    """More than 65535 rois: the gather backward's channels-last copy of grad_output is made in
-    launches of at most 65535 rois.  Checked two ways: the adjoint identity <F(x), g> = <x, F^T g>
-    (float64 sums of the GPU's fp32 results) and against the sum of the two halves' gradients."""
+    """More than 65535 rois, a block per roi in the passes over rois.  Checked two ways: the adjoint
+    identity <F(x), g> = <x, F^T g> (float64 sums of the GPU's fp32 results) and against the sum of the
+    two halves' gradients."""
     from fda_helpers import log
 
     from ops3d_amd.roi_align import roi_align_3d
@@ -382,10 +382,12 @@ TILE_CASES = [
     (1, 33, (5, 6, 8), 7, (4, 4, 4), 2, torch.float32),           # 64 bins: one row per lane in the copy
     (1, 3, (6, 7, 9), 5, (6, 8, 8), 2, torch.bfloat16),           # 384 bins
     (1, 8, (16, 40, 48), 3, (3, 3, 3), 2, torch.float32),         # few rois, many tiles: the natural tile order
-    (1, 70, (9, 10, 11), 8, (3, 3, 3), 2, torch.float32),         # rois over four waves, two each
-    (2, 5, (4, 6, 7), 259, (2, 2, 2), 1, torch.bfloat16),         # the same, over 64 rois to a wave
-    (2, 70, (16, 40, 46), 9, (3, 2, 3), 2, torch.bfloat16),       # 1920 blocks: one wave each, W not of 4
-    (1, 8, (1, 2, 32900), 12, (2, 2, 3), 2, torch.float32),       # 8225 blocks: crowded tiles first
+    (1, 70, (9, 10, 11), 8, (3, 3, 3), 2, torch.float32),         # partial tiles on every axis
+    (2, 5, (4, 6, 7), 259, (2, 2, 2), 1, torch.bfloat16),         # over four waves, over 64 rois to a wave
+    (2, 70, (16, 40, 46), 9, (3, 2, 3), 2, torch.bfloat16),       # 1920 blocks of one wave, W not of 4
+    (1, 8, (1, 2, 32900), 12, (2, 2, 3), 2, torch.float32),       # 8225 blocks, 32 strips of 256 tiles
+    (1, 70, (9, 10, 11), 17, (3, 3, 3), 2, torch.float32),        # rois over four waves, four or five each
+    (1, 8, (10, 11, 12), 9, (7, 7, 7), 1, torch.float32),         # one wave each, bins below a voxel
 ]
 
 
@@ -409,6 +411,61 @@ def test_gpu_backward_tiles(gpu_device, case):
     want = O.backward(g.double().numpy(), rois.double().numpy(), (N, C) + size, 1.0, sr, 1)
     rtol, atol = TOL[dt]
     assert_close("roi_align grad", grad, want, rtol, atol * (10 if dt == torch.float32 else 1))
+
+
+CLEAR_CASES = [
+    # N, C, (D, H, W), R, pooled, dtype; at least 27 tiles per roi
+    (2, 10, (9, 11, 50), 3, (3, 2, 4), torch.float32),            # blocks of one wave, W not of 4
+    (1, 12, (3, 4, 1030), 2, (2, 2, 2), torch.float16),           # more than 256 tiles in x, one wave
+    (2, 9, (5, 6, 1101), 20, (2, 2, 2), torch.bfloat16),          # more than 256 tiles in x, four waves
+    (1, 66, (24, 40, 41), 16, (2, 2, 2), torch.bfloat16),         # a second channel group of 2, four waves
+    (2, 5, (6, 7, 9), 0, (2, 2, 2), torch.float32),               # no rois
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", range(len(CLEAR_CASES)))
+def test_gpu_backward_empty_tiles(gpu_device, case):
+    """Few rois, of at most 12 voxels, for the tiles: the tiles without one get their zeros from blocks of
+    their own (bars as above)."""
+    from fda_helpers import TOL, assert_close, log
+
+    from ops3d_amd import _C
+
+    N, C, size, R, pooled, dt = CLEAR_CASES[case]
+    log(f"[case] roi_align3d backward empty tiles #{case}: N={N} C={C} size={size} R={R} {dt}")
+    r = np.random.default_rng(500 + case)
+    lo = r.uniform(0.0, 0.8, size=(R, 3)) * np.array(size[::-1]) - 1.0
+    rois = np.concatenate([r.integers(0, N, size=(R, 1)), lo, lo + r.uniform(1.0, 12.0, size=(R, 3))], 1)
+    rois = torch.from_numpy(rois.astype(np.float32)).to(dt)
+    g = torch.from_numpy(r.normal(size=(R, C) + pooled).astype(np.float32)).to(dt)
+    grad = torch.full((N, C) + size, 7.0, dtype=dt, device=gpu_device)
+    _C.roi_align_3d_backward(g.to(gpu_device), rois.to(gpu_device), grad, *pooled, 1.0, 2, 1)
+    torch.cuda.synchronize()
+    want = O.backward(g.double().numpy(), rois.double().numpy(), (N, C) + size, 1.0, 2, 1)
+    assert R == 0 or np.count_nonzero(want)
+    rtol, atol = TOL[dt]
+    assert_close("roi_align grad", grad, want, rtol, atol * (10 if dt == torch.float32 else 1))
+
+
+@pytest.mark.gpu
+def test_gpu_backward_crowded_tiles_first(gpu_device):
+    """More than 8192 blocks whose tiles hold several rois each: the tiles are taken by their number of
+    rois.  Channels do not meet, so the oracle takes five of the 5100."""
+    from fda_helpers import assert_close, log
+
+    from ops3d_amd import _C
+
+    N, C, size, R, pooled, pick = 1, 5100, (12, 24, 24), 12, (2, 3, 2), [0, 63, 64, 2000, 5099]
+    log(f"[case] roi_align3d backward crowded tiles first: C={C} size={size} R={R}")
+    g = torch.from_numpy(np.random.default_rng(7).normal(size=(R, C) + pooled).astype(np.float32))
+    rois = torch.from_numpy(_rois(R, N, size, seed=8, lo=-1.0))
+    grad = torch.full((N, C) + size, 7.0, device=gpu_device)
+    _C.roi_align_3d_backward(g.to(gpu_device), rois.to(gpu_device), grad, *pooled, 1.0, 2, 1)
+    torch.cuda.synchronize()
+    want = O.backward(g[:, pick].double().numpy(), rois.double().numpy(), (N, len(pick)) + size, 1.0, 2, 1)
+    assert_close("roi_align grad", grad[:, pick], want, 1e-5, 1e-5)
+    assert bool((grad != 7.0).all())
 
 
 @pytest.mark.gpu

@@ -363,6 +363,30 @@ def test_backward_accumulate_f32(gpu_device, dt):
                  __import__("fda_helpers").fp32_allowance(inp))
 
 
+@pytest.mark.parametrize("shapes,B,Q,G,D,dt", [
+    ([(12, 14, 30), (6, 7, 15), (2, 2, 4)], 1, 600, 8, 32, torch.bfloat16),     # a head per XCD
+    ([(11, 27, 45), (6, 14, 23), (3, 7, 12)], 2, 700, 6, 48, torch.float32),    # no XCD groups
+])
+def test_backward_accumulate_split_levels(gpu_device, shapes, B, Q, G, D, dt):
+    """The fp32 buffer over levels whose tiles are cut into different numbers of parts: the parts of a
+    tile are added to what the buffer holds, once per call."""
+    from ops3d_amd import _C
+
+    inp = random_inputs(shapes, B, Q, G, D, 4, dt, seed=Q, lo=-0.05, hi=1.05)
+    st, lsi = level_meta(inp["shapes"], gpu_device)
+    acc = torch.full(inp["value"].shape, 0.25, dtype=torch.float32, device=gpu_device)
+    args = [inp[k].to(gpu_device) for k in ("value", "sampling_loc_attn", "grad_output")]
+    for _ in range(2):
+        gs = _C.flash_deform_attn_backward_accumulate(args[0], st, lsi, args[1], args[2], acc, 64, 4)
+    torch.cuda.synchronize()
+    _, rgv, rgs = run_oracle(inp)
+    # two gradients of the fp32 bar (1e-6 each) and, with parts, sums in another order than one tile's:
+    # up to 4 Q = 2800 terms of about 0.1 in a voxel, sqrt(2800) * 0.1 * sqrt(2800) * 2^-24 / 2 = 8e-6
+    assert_close("accumulated grad_value", acc, 0.25 + 2 * rgv, 1e-5, 2e-5)
+    assert_close("grad_sla", gs, rgs, *TOL[dt], extra=None if dt != torch.float32 else
+                 __import__("fda_helpers").fp32_allowance(inp))
+
+
 @pytest.mark.parametrize("dt,G,D,lo,hi", [(torch.bfloat16, 8, 32, 0.0, 1.0), (torch.float32, 8, 32, -0.1, 1.1),
                                           (torch.float32, 3, 16, -0.1, 1.1), (torch.float16, 2, 64, 0.0, 1.0)])
 def test_scatter_baseline(gpu_device, dt, G, D, lo, hi):

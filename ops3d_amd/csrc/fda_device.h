@@ -56,7 +56,7 @@ struct Args {
   void *grad_loc_attn;        // [B,Q,G,P] T          (backward)
   // backward, tile formulation of grad_value
   uint32_t *keys;             // [N] bucketing key of each sample (tile_key; kKeyInvalid if outside)
-  float4 *stash;              // [N] (x, y, z, attn) of each sample: level pixel coordinates
+  float4 *stash;              // [N] x, y, z weights of each sample's upper corners, attention weight
   uint32_t *tile_counts;      // [B*G*T_h] entries per tile
   uint32_t *tile_start;       // [B*G*T_h] first entry of each tile (head base + exclusive scan)
   uint32_t *tile_cursor;      // [B*G*T_h] fill cursor of each tile

@@ -2,8 +2,8 @@
 
 ``nms_nd(dets, iou_threshold)`` takes dets [N, 7] (x1, y1, z1, x2, y2, z2, score) and returns
 ``(keep, dets)`` as the reference does: keep holds the int64 indices of the kept boxes in
-decreasing score order.  The work runs in libops3d_fda.so (csrc/nms3d.hip): the IoU bitmask
-and the greedy pass both on the GPU.
+decreasing score order.  The work runs in libops3d_fda.so (csrc/nms3d.hip), all on the GPU: from a
+list of the overlapping pairs, or from an IoU bitmask where the boxes overlap too much for it.
 """
 from __future__ import annotations
 

@@ -198,8 +198,8 @@ hipError_t launch(int dtype, int which, const Geometry &g, hipStream_t st) {
 }
 
 // Workspace of the backward (all offsets 256-byte aligned):
-//   keys, words    : N uint32 each, N = B*Q*G*L*K samples (home tile, tile-local word)
-//   stash          : N float4 (x, y, z, attn), level pixel coordinates
+//   keys           : N uint32, N = B*Q*G*L*K samples (tile_key: home tile, next-tile flags, level)
+//   stash          : N float4 (x, y, z weights of the upper corners, attention weight)
 //   entries        : 8N uint32 sample indices (a sample is listed in at most 8 tiles)
 //   counts, start, cursor : B*G*S + 1 uint32 each (a tile holds at least one voxel, so a head
 //                    has at most S tiles)
@@ -686,11 +686,14 @@ static int backward_impl(const void *value, const void *value_head_major, const 
     g3.a.tile_affinity = num_heads % 8 == 0;
     g3.a.chunk = tile_chunk(channels, elem_size(dtype), tile_lanes(geo.lpu, geo.cpl * elem_size(dtype)),
                             a.big_tiles != 0);
-    // Few entries per tile (at least ceil(S / tile voxels) tiles per head): a tile is a chain of
-    // loads of which each waits for the one before, so smaller chunks, which leave room for more
-    // blocks per CU.  200 queries of 3 levels, 37376 voxels, batch 2 (8 samples per tile): tile
-    // kernel 38.8 us, with chunks of 256 / 192 / 128 entries 33.8 / 34.0 / 35.2.
-    if ((uint64_t)ly.n < 16 * ly.tiles_least) g3.a.chunk = g3.a.chunk < 256 ? g3.a.chunk : 256;
+    // Few samples per tile (at least ceil(S / tile voxels) tiles per head): a tile is a chain of
+    // loads of which each waits for the one before, so chunks of at most 256 entries, which leave
+    // room for more blocks per CU.  Whole backward, us, the CU's share / 256, by samples per tile:
+    // 8 heads of 32 bf16 over 37376 voxels in 3 levels, batch 2: 8 61.7 / 56.9, 16 85.5 / 82.0,
+    // 33 99.9 / 95.7, 66 128 / 131, 131 181 / 194; of 16 fp32, batch 1: 8 48.9 / 43.7, 33 70.4 / 68.1,
+    // 66 85.6 / 87.6; of 32 bf16 over 147456 in 2: 1.4 76.1 / 68.1, 22 139.6 / 128.8, 44 171.5 / 162.5.
+    // (6 heads of 48 fp32 and 4 of 64 fp16: level.)
+    if ((uint64_t)ly.n < 32 * ly.tiles_least) g3.a.chunk = g3.a.chunk < 256 ? g3.a.chunk : 256;
     g3.lds = tile_kernel_lds_bytes(g3.a.chunk, channels * elem_size(dtype),
                                    tile_lanes(geo.lpu, geo.cpl * elem_size(dtype)), a.big_tiles != 0);
     g3.grid = (unsigned)device_cus();   // times the resident blocks per CU (launch_one)

@@ -375,7 +375,7 @@ TILE_CASES = [
     # N, C, (D, H, W), R, pooled, sampling_ratio, dtype
     (1, 63, (3, 5, 9), 10, (2, 2, 2), 2, torch.float32),          # partial tiles, 63 channels
     (2, 65, (4, 8, 4), 12, (3, 2, 4), 2, torch.bfloat16),         # whole tiles, a second channel group of 1
-    (1, 7, (1, 1, 1), 4, (2, 2, 2), 1, torch.float32),            # one voxel
+    (1, 7, (1, 1, 1), 4, (2, 2, 2), 1, torch.float32),            # one voxel, reached by no roi
     (1, 8, (6, 7, 8), 420, (2, 2, 2), 1, torch.float32),          # more rois in a tile than are listed at a time
     (1, 8, (8, 9, 10), 200, (6, 5, 6), 1, torch.bfloat16),        # rois of both kinds (bins below a voxel) in a tile
     (1, 250, (8, 6, 12), 9, (3, 3, 3), 0, torch.float16),         # runs of grad_output at odd alignments
@@ -385,9 +385,10 @@ TILE_CASES = [
     (1, 70, (9, 10, 11), 8, (3, 3, 3), 2, torch.float32),         # partial tiles on every axis
     (2, 5, (4, 6, 7), 259, (2, 2, 2), 1, torch.bfloat16),         # over four waves, over 64 rois to a wave
     (2, 70, (16, 40, 46), 9, (3, 2, 3), 2, torch.bfloat16),       # 1920 blocks of one wave, W not of 4
-    (1, 8, (1, 2, 32900), 12, (2, 2, 3), 2, torch.float32),       # 8225 blocks, 32 strips of 256 tiles
+    (1, 8, (1, 2, 32900), 12, (2, 2, 3), 2, torch.float32),       # 8225 blocks, reached by no roi
     (1, 70, (9, 10, 11), 17, (3, 3, 3), 2, torch.float32),        # rois over four waves, four or five each
     (1, 8, (10, 11, 12), 9, (7, 7, 7), 1, torch.float32),         # one wave each, bins below a voxel
+    (1, 7, (1, 1, 1), 40, (2, 2, 2), 1, torch.float32),           # one voxel that rois reach
 ]
 
 
@@ -419,6 +420,7 @@ CLEAR_CASES = [
     (1, 12, (3, 4, 1030), 2, (2, 2, 2), torch.float16),           # more than 256 tiles in x, one wave
     (2, 9, (5, 6, 1101), 20, (2, 2, 2), torch.bfloat16),          # more than 256 tiles in x, four waves
     (1, 66, (24, 40, 41), 16, (2, 2, 2), torch.bfloat16),         # a second channel group of 2, four waves
+    (1, 8, (1, 2, 32900), 12, (2, 2, 3), torch.float32),          # 8225 blocks, 33 strips of 256 tiles
     (2, 5, (6, 7, 9), 0, (2, 2, 2), torch.float32),               # no rois
 ]
 

@@ -682,9 +682,9 @@ __global__ __launch_bounds__(1024) void roi_tile_order_kernel(const uint8_t *cou
 // How a gather is launched, by its blocks (a wave per tile and 64 channels), the rois R and the tiles
 // (figures: at backward()).
 constexpr int kGSplitBlocks = 4096, kGSplitRois = 16;   // up to so many blocks, from so many rois: SPLIT
-constexpr int kGClearRois = 27;                  // R * 27 <= tiles: most tiles are empty, clear_tiles()
+constexpr int kGClearRois = 27;                  // R * 27 <= tiles: many tiles are empty, clear_tiles()
+constexpr int kGClearMiddle = 12288;             // up to so many blocks, not SPLIT: in the tiles' middle
 constexpr int kGUnordered = 8192, kGOrderRois = 12;     // more blocks, R * 12 > tiles: crowded tiles first
-constexpr int kGNotCleared = 0x7fffffff;
 constexpr int kGOrdered = 65535;                 // tiles that are ordered (16-bit numbers)
 constexpr int kGList = 192;                      // rois listed at a time
 
@@ -702,27 +702,36 @@ __device__ __forceinline__ RawOf<T> load_raw(__amdgpu_buffer_rsrc_t rs, uint32_t
 // row of tiles along x and kGClearChannels channels, 4 voxels per thread with the lanes along x.
 constexpr int kGClearWords = 8, kGClearChannels = 8;   // 256 tiles at a time
 template <typename T, int NT>
-__device__ __forceinline__ void clear_tiles(int blk, uint32_t *reached_l, const T *__restrict__ rois,
+__device__ __forceinline__ void clear_tiles(int blk, uint32_t *lds_l, const T *__restrict__ rois,
                                             const uint32_t *__restrict__ tr, T *__restrict__ grad, int C, int D, int H,
                                             int W, int R) {
   const int t = threadIdx.x, ntz = tiles_of(D), nty = tiles_of(H), ntx = tiles_of(W);
   const int parts = (C + kGClearChannels - 1) / kGClearChannels, c0 = blk % parts * kGClearChannels;
   const int ty = blk / parts % nty, tz = blk / parts / nty % ntz, n = blk / parts / nty / ntz;
   const int nc = min(kGClearChannels, C - c0);
+  uint32_t *const reached_l = lds_l, *const count_l = lds_l + kGClearWords, *const row_l = count_l + 1;
   for (int tx0 = 0; tx0 < ntx; tx0 += 32 * kGClearWords) {
     const int nt = min(32 * kGClearWords, ntx - tx0);
-    if (t < kGClearWords) reached_l[t] = 0;
+    if (t <= kGClearWords) lds_l[t] = 0;
     __syncthreads();
-    for (int i = t; i < R * 4; i += NT) {   // four threads per roi
-      const int r = i >> 2;
+    // the rois of this row of tiles, NT at a time, and then every pair of one of them and a tile
+    for (int r0 = 0; r0 < R; r0 += NT) {
+      const int r = min(r0 + t, R - 1);
       const uint32_t z = tr[(size_t)tz * R + r], y = tr[(size_t)(ntz + ty) * R + r];
-      if ((int)to_f(rois[(int64_t)r * 7]) != n || first_bin(z) > last_bin(z) || first_bin(y) > last_bin(y)) continue;
-      for (int k = i & 3; k < nt; k += 4) {
-        const uint32_t x = tr[(size_t)(ntz + nty + tx0 + k) * R + r];
+      if (r0 + t < R && (int)to_f(rois[(int64_t)r * 7]) == n && first_bin(z) <= last_bin(z) && first_bin(y) <= last_bin(y))
+        row_l[atomicAdd(count_l, 1u)] = (uint32_t)r;
+      __syncthreads();
+      const int pairs = (int)*count_l * nt;
+#pragma unroll 4
+      for (int i = t; i < pairs; i += NT) {
+        const int q = i / nt, k = i - q * nt;
+        const uint32_t x = tr[(size_t)(ntz + nty + tx0 + k) * R + row_l[q]];
         if (first_bin(x) <= last_bin(x)) atomicOr(&reached_l[k >> 5], 1u << (k & 31));
       }
+      __syncthreads();
+      if (t == 0) *count_l = 0;
+      __syncthreads();
     }
-    __syncthreads();
     for (int k0 = 0; k0 < nt; k0 += NT) {
       // threads in rows of the next power of two above the tiles
       const int m = min(NT, nt - k0), shift = m > 1 ? 32 - __clz(m - 1) : 0, kk = t & ((1 << shift) - 1), k = k0 + kk;
@@ -746,14 +755,14 @@ __device__ __forceinline__ void clear_tiles(int blk, uint32_t *reached_l, const 
 
 // SPLIT: a block of kGSplit waves per tile and channel group, each taking every kGSplit-th roi; their
 // sums are added in LDS, two planes at a time, wave w those of plane w (launched where a tile's chain
-// of rois is the time: few tiles, which run at once or nearly).  Blocks from clear_from on are
-// clear_tiles()'s, behind the tiles' since those end with the few crowded ones.
+// of rois is the time: few tiles, which run at once or nearly).  `clears` blocks from clear_at on are
+// clear_tiles()'s (multiples of 8: the tiles keep their XCDs).
 constexpr int kGSplit = 4;
 template <typename T, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, 4) void roi_align3d_backward_gather_kernel(
     const T *__restrict__ top_cl, const T *__restrict__ rois, T *__restrict__ grad, const float *__restrict__ wt,
     const uint32_t *__restrict__ tr, const unsigned short *__restrict__ order, int N, int C, int D, int H,
-    int W, int R, int PD, int PH, int PW, int blocks, int run, int clear_from) {
+    int W, int R, int PD, int PH, int PW, int blocks, int run, int clear_at, int clears) {
   constexpr int NW = SPLIT ? kGSplit : 1;
   static_assert(!SPLIT || kGSplit == kGT, "a wave per plane of the tile");
   // the rois' lists; with SPLIT then the waves' sums of two planes (32 KB: four blocks per CU)
@@ -770,9 +779,14 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, 4) void roi_align3d_back
   // the same rois' bins, and which run of a round of eight it takes moves on, so that no XCD gets
   // only the crowded middle of the volume.
   int bid = blockIdx.x, cg;
-  if (bid >= clear_from) {
-    clear_tiles<T, 64 * NW>(bid - clear_from, reinterpret_cast<uint32_t *>(lds_l), rois, tr, grad, C, D, H, W, R);
-    return;
+  if (bid >= clear_at) {
+    bid -= clears;
+    if (bid < clear_at) {
+      const int blk = bid + clears - clear_at;
+      if (blk < N * ntz * nty * ((C + kGClearChannels - 1) / kGClearChannels))
+        clear_tiles<T, 64 * NW>(blk, reinterpret_cast<uint32_t *>(lds_l), rois, tr, grad, C, D, H, W, R);
+      return;
+    }
   }
   if (order) {
     if (bid >= blocks) return;
@@ -1021,7 +1035,7 @@ __global__ __launch_bounds__(SPLIT ? 64 * kGSplit : 64, 4) void roi_align3d_back
     __builtin_amdgcn_wave_barrier();   // the list is read before the next rois are written to it
   }
   // nothing to store where the zeros come from clear_tiles(), no sums to add where there are none
-  const bool any = (SPLIT ? __syncthreads_or(reached) != 0 : reached) || clear_from == kGNotCleared;
+  const bool any = (SPLIT ? __syncthreads_or(reached) != 0 : reached) || clears == 0;
   if constexpr (SPLIT) {   // wave w: the sums of plane w, in acc[0]
     if (any) {
       float(*sums_l)[kSums][64] = reinterpret_cast<float(*)[kSums][64]>(lds_l);
@@ -1387,11 +1401,17 @@ inline size_t gather_tables_bytes(int R, int D, int H, int W, int PD, int PH, in
 //     10x23x65, 256, 213 of 4-16 (1224) 199 / 411; 30x60x60 f, 32, 60 (1800) 58 / 68; 24x48x48, 256,
 //     300 of 4-24 (3456) 260 / 322, 30 rois 82 / 77; 32x64x64, 192, 200 rois, 5^3 (6144) 132 / 130.
 //     Four blocks per CU: with 64 KB of sums, two, 213 rois took 267 and 21 rois 53.
-//   clear_tiles() / every wave stores: 2 x 32x64x64, 256, 64 rois of 4-16 (4096 tiles) 135 / 180; 110 of
-//     4-16 158 / 193; 150 of 4-32 212 / 215; f, 16 rois 127 / 211; 2 x 41x50x50, 256, 35 of 4-16, one
-//     sample, nearest (3718) 83 / 123, of 4-32 113 / 131; 24x48x48, 256, 9 rois (864) 50 / 51.  The
-//     stores of 4 voxels take 0.1 to 0.2 ms per 100 MB of gradient, a clear about 30 us, most of it
-//     beside the crowded tiles' chains.  As a pass of its own before the gather 64 rois took 141.
+//   clear_tiles() / every wave stores: 2 x 32x64x64, 256, 64 rois of 4-16 (4096 tiles) 128 / 179; 110 of
+//     4-16 168 / 205; 150 of 4-32 213 / 216; f, 16 rois 124 / 208; 2 x 41x50x50, 256, 35 of 4-16, one
+//     sample, nearest (3718) 75 / 116, of 4-32 103 / 125; 23x33x89, 250, 46 of 3-18, 3^3 (1242) 44 / 51,
+//     f 62 / 66; 24x48x48, 256, 9 rois (864) 46 / 47.  At 27 tiles per roi, rois of 4-30 reach nearly
+//     all tiles and lose up to 4 %, rois of 3-12 gain 5 to 30 %.  As a pass of its own before the
+//     gather 64 rois took 141.  The clear blocks stand behind the tiles', whose end is the chain of the
+//     last crowded ones, or, where one-wave tiles run in up to about three rounds, in their middle, or
+//     their own latency is the end (behind / middle / before them: 46 rois above (4968 blocks) 60 / 44
+//     / 49, f 71 / 62 / 66; 2 x 23x33x89 f, 80 of 3-18 (9936) 123 / 110 / 113; 2 x 40x50x50, 192, 28 of
+//     4-30 (10140) 84 / 78 / 87; 2 x 32x64x64 f, 256, 146 of 3-12, 5^3 (16384) 175 / 194 / 197;
+//     24x48x48, 256, 30 of 4-24 (SPLIT) 77 / 83 / 83).
 //   Crowded tiles first / in place: 2 x 32x64x64, 256, 512 rois 430 / 459, 400 rois 372 / 371, 300
 //     rois 321 / 288, 220 rois 292 / 248; 2 x 40x80x80, 512 rois (8000 tiles) 648 / 610, 300 rois
 //     521 / 425: the neighbours' stores then meet in no L2.
@@ -1425,7 +1445,7 @@ int backward(const void *grad_output, const void *rois, void *grad_input, float 
     const int64_t used = (int64_t)R * (ntz + nty + ntx) * 4, spare = (int64_t)R * (D + H + W) * 4 - used;
     unsigned short *order = nullptr;
     const bool split = blocks <= kGSplitBlocks && R >= kGSplitRois;
-    const int64_t clears = (int64_t)N * ntz * nty * ((C + kGClearChannels - 1) / kGClearChannels);
+    const int64_t clears = ((int64_t)N * ntz * nty * ((C + kGClearChannels - 1) / kGClearChannels) + 7) / 8 * 8;
     const bool cleared = (int64_t)R * kGClearRois <= tiles && grid + clears < (1 << 24);
     if (blocks > kGUnordered && (int64_t)R * kGOrderRois > tiles && tiles <= kGOrdered && tiles * 3 <= spare) {
       order = reinterpret_cast<unsigned short *>(reinterpret_cast<char *>(tr) + used);
@@ -1437,7 +1457,7 @@ int backward(const void *grad_output, const void *rois, void *grad_input, float 
     const auto gather = [&](auto kern, int threads) {
       hipLaunchKernelGGL(kern, dim3((unsigned)(grid + (cleared ? clears : 0))), dim3(threads), 0, st, top_cl,
                          static_cast<const T *>(rois), static_cast<T *>(grad_input), wt, tr, order, N, C, D, H, W, R, PD,
-                         PH, PW, (int)blocks, (int)run, cleared ? (int)grid : kGNotCleared);
+                         PH, PW, (int)blocks, (int)run, (int)(split || blocks > kGClearMiddle ? grid : grid / 16 * 8), cleared ? (int)clears : 0);
     };
     if (split) gather(roi_align3d_backward_gather_kernel<T, true>, 64 * kGSplit);
     else gather(roi_align3d_backward_gather_kernel<T, false>, 64);

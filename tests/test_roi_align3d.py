@@ -420,7 +420,7 @@ CLEAR_CASES = [
     (1, 12, (3, 4, 1030), 2, (2, 2, 2), torch.float16),           # more than 256 tiles in x, one wave
     (2, 9, (5, 6, 1101), 20, (2, 2, 2), torch.bfloat16),          # more than 256 tiles in x, four waves
     (1, 66, (24, 40, 41), 16, (2, 2, 2), torch.bfloat16),         # a second channel group of 2, four waves
-    (1, 8, (1, 2, 32900), 12, (2, 2, 3), torch.float32),          # 8225 blocks, 33 strips of 256 tiles
+    (1, 8, (1, 2, 49500), 12, (2, 2, 3), torch.float32),          # 12375 blocks, 49 strips of 256 tiles
     (2, 5, (6, 7, 9), 0, (2, 2, 2), torch.float32),               # no rois
 ]
 

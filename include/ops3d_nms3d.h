@@ -46,8 +46,8 @@ OPS3D_FDA_API int ops3d_nms3d(const float *boxes_sorted, const int64_t *order, i
  *              scores in index order) when ops3d_nms3d_pairs_ranks(n); order must then be NULL;
  *   order:     otherwise (scores not read) [n] int64, box indices by decreasing score;
  *   keep, num_keep: as above, but *num_keep = -1 when the boxes overlap too much for the list
- *              (more than about 32 pairs per box above the threshold): keep is then not written and
- *              the caller runs ops3d_nms3d_after_pairs.
+ *              (more than about 64 pairs per box above the threshold, or more than 32 where the boxes
+ *              make chains): keep is then not written and the caller runs ops3d_nms3d_after_pairs.
  * The workspace (ops3d_nms3d_pairs_workspace_bytes) must be 32-byte aligned.
  */
 OPS3D_FDA_API size_t ops3d_nms3d_pairs_workspace_bytes(int n);

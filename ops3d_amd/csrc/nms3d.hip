@@ -222,8 +222,10 @@ __global__ __launch_bounds__(kReduceThreads) void nms3d_reduce_kernel(const uint
 constexpr int kLists = 16;                 // pair lists (a counter each: fewer adds per address); one
                                            // wave of the resolve kernel serves each
 constexpr int kCounterStride = 32;         // counters 128 bytes apart
-constexpr int kPairsPerBox = 32;           // list capacity: above it the resolve kernel, one workgroup,
-                                           // can take longer than the mask's greedy pass
+constexpr int kPairsPerBox = 64;           // list capacity: two rounds over it cost less than half of
+                                           // the mask's greedy pass
+constexpr int kChainPairsPerBox = 32;      // above it chains cost the resolve kernel, one workgroup, as
+                                           // much as the mask path or more
 constexpr int kMaxPairBoxes = 1 << 18;     // three bitmaps of the boxes in 96 KB of LDS
 constexpr int kMaxRankBoxes = 8192;        // ranks by counting (n^2 comparisons), keys in 32 KB of LDS
 constexpr int kCells = 4096;               // 16^3
@@ -625,6 +627,11 @@ constexpr int kResolveThreads = 64 * kLists;
 // Costs in units of a pair read by a round (about 0.5 ns): a round besides its pairs, rounds per
 // inverse share of the boxes decided, the block pass, each of its blocks, each of its pairs.
 constexpr float kRoundCost = 2048.f, kRoundsPerShare = 8.f, kPassCost = 16384.f, kBlockCost = 3072.f, kSortCost = 2.5f;
+// Chains with many pairs cost more than the mask.  An eighth of the pairs tells them apart: of 1024
+// pairs, spread over the lists, those whose first box it does not block are about 16 / m in clusters of
+// m boxes that all overlap (and 17 % with independent scores at 40 pairs per box), but (7/8)^33 = 1 % where
+// every box follows 33 that overlap it.
+constexpr uint32_t kChainFirst = 48;
 constexpr int kMarkPairs = 1024;   // of a list: fewer are not worth a loop of their own
 __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *lists, int capacity,
                                                                         const uint32_t *counters, uint2 *by_block, int n,
@@ -634,6 +641,7 @@ __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *l
   __shared__ uint32_t left_l[2], open_l[2], part_l[kLists], over_l;
   __shared__ uint32_t mask_l[2][64][2];
   __shared__ uint64_t gone_l;
+  __shared__ uint32_t pairs_l;
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int words = (n + 31) / 32;
   uint32_t *kept = bits_l, *removed = bits_l + words, *blocked = bits_l + 2 * words;
@@ -643,10 +651,11 @@ __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *l
     blocked[w] = 0;
   }
   if (t < 2) left_l[t] = open_l[t] = 0;
-  if (t == 0) over_l = 0;
+  if (t == 0) over_l = pairs_l = 0;
   __syncthreads();
   const uint32_t total = counters[wv * kCounterStride];
   if (total > (uint32_t)capacity && lane == 0) over_l = 1;   // a list overflowed
+  if (lane == 0) atomicAdd(&pairs_l, min(total, (uint32_t)capacity));
   __syncthreads();
   if (over_l) {
     if (t == 0) *num_keep = -1;
@@ -656,6 +665,24 @@ __global__ __launch_bounds__(kResolveThreads) void nms3d_resolve_kernel(uint2 *l
   uint2 *list_out = lists + (int64_t)wv * capacity;
   const int nblk = (n + 63) / 64;
   int cnt = (int)total;
+  if (pairs_l > (uint32_t)n * kChainPairsPerBox) {   // many pairs: the mask if they are chains
+    for (int e = lane; e < cnt / 8; e += 64) {
+      const uint32_t b = list[8 * e + (5 * e & 7)].y;
+      if (!(blocked[b >> 5] >> (b & 31) & 1u)) atomicOr(&blocked[b >> 5], 1u << (b & 31));
+    }
+    __syncthreads();
+    const uint32_t a = cnt ? list[(uint64_t)lane * (uint32_t)cnt / 64].x : 0u;
+    const uint64_t m = __ballot(cnt && !(blocked[a >> 5] >> (a & 31) & 1u));
+    if (lane == 0) atomicAdd(&open_l[0], (uint32_t)__builtin_popcountll(m));
+    __syncthreads();
+    const uint32_t first = open_l[0];
+    __syncthreads();
+    if (first < kChainFirst) {
+      if (t == 0) *num_keep = -1;
+      return;
+    }
+    if (t == 0) open_l[0] = 0;   // settle() has a barrier before it adds to it
+  }
   // undecided boxes that no undecided box precedes are kept; the pairs left in all lists and the
   // boxes left undecided
   uint32_t more = 0, open_boxes = 0;
@@ -997,8 +1024,13 @@ int ops3d_nms3d_pairs_ranks(int n) { return n > 0 && n <= ops3d_nms::kMaxRankBox
 // rows whose boxes overlap the next 10, 4096 boxes 207 / 280, 16 384 boxes 672 / 957 (24 550); the next
 // 30, 4096 boxes 350 / 286, 16 384 boxes 985 / 979 (66 500), 65 536 boxes 4030 / 5330 (813 000); equal
 // scores in raster order, 20^3 boxes 344 / 491 (2970), 30^3 boxes 1080 / 1740 (6750).  The same grid
-// with random scores 149 / 550.  One workgroup spends 1.5 to 2.5 ns on a pair (a round or two, the sort
-// and the block pass), so at the lists' capacity of 32 pairs per box it is level with the mask path.
+// with random scores 149 / 550.  One workgroup spends 1.5 to 2.5 ns on a pair of a chain (a round or
+// two, the sort and the block pass), so at 32 pairs per box it is level with the mask path; rows that
+// overlap the next 40 are left to the mask: 4096 boxes 289 / 278 (the block pass 414), 16 384 1118 / 976,
+// 65 536 5680 / 5310.  Independent scores, or alike ones inside clusters, take a few rounds at any
+// length: clusters of 100 boxes that nearly all overlap (40 pairs per box), 4096 boxes 134 / 343, 8300
+// 326 / 620, 50 000 1222 / 4514 (lists of 32 per box, and so the mask: 344, 722, 4626), with scores
+// alike inside a cluster 151 / 304, 339 / 576, 1305 / 5107.
 int ops3d_nms3d_pairs(const float *boxes, int64_t box_stride, int64_t coord_stride, const float *scores,
                       int64_t score_stride, const int64_t *order, int n, float iou_threshold, void *workspace,
                       size_t workspace_bytes, int64_t *keep, int32_t *num_keep, void *stream) {

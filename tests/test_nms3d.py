@@ -252,7 +252,8 @@ def _clusters(n, m):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,m", [(64, 25), (64, 64), (128, 25), (128, 64), (300, 25), (1000, 25), (2000, 50)])
+@pytest.mark.parametrize("n,m", [(64, 25), (64, 64), (128, 25), (128, 64), (300, 25), (1000, 25), (2000, 50),
+                                 (1000, 100), (4096, 120), (9000, 100)])
 def test_gpu_pairs_crowded_blocks(gpu_device, n, m):
     """The pair path itself (no fallback to the mask behind it) holds the pairs of a few crowded blocks,
     down to a call of a single one: they are spread over all lists."""
@@ -299,6 +300,25 @@ def test_gpu_pairs_take_chains(gpu_device, kind, n, arg):
     got = _pairs_path(b, s, thr)
     assert got is not None
     assert got == _mask_path(b, s, thr)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,row,reach,gives_up", [(1000, 1000, 40, True), (4096, 4096, 60, True), (9001, 9001, 50, True),
+                                                  (2000, 160, 40, None), (9600, 120, 60, None)])
+def test_gpu_pairs_leave_long_lists_of_chains(gpu_device, n, row, reach, gives_up):
+    """Rows with more than 32 pairs per box: one chain is left to the mask path (a box is not blocked by
+    an eighth of the pairs with (7/8)^reach < 1 %), many short ones may be decided either way."""
+    from fda_helpers import log
+
+    from ops3d_amd import _C
+
+    log(f"[case] nms3d pair path, rows of {row} among {n} reaching {reach}")
+    boxes, scores = _row(n, reach, 0.3)
+    boxes[:, [1, 4]] += np.float32(5) * (np.arange(n) // row)[:, None].astype(np.float32)
+    b, s = torch.from_numpy(boxes).to(gpu_device), torch.from_numpy(scores).to(gpu_device)
+    got, want = _pairs_path(b, s, 0.3), _mask_path(b, s, 0.3)
+    assert got is None or (gives_up is None and got == want)
+    assert _C.nms_3d(b, s, 0.3).cpu().tolist() == want
 
 
 @pytest.mark.gpu
